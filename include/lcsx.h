@@ -278,12 +278,14 @@ lcsx_status lcsx_solver_kernel_times(lcsx_solver* s, char* buf, size_t buf_len, 
  * around it, which is why level 2 samples. */
 lcsx_status lcsx_solver_set_timing(lcsx_solver* s, int level);
 /* PCG launch mode (no counterpart in the reference, whose backend records its own command
- * lists): 1 captures each convergence-test interval of PCG iterations as a hipGraph and replays
- * it; 0 (default) launches every kernel directly. Both run the same kernels with the same
- * arguments in the same order. On MI355X the replay does not shorten the device time of a solve
- * (the gaps between dependent kernels remain) and each new chunk shape costs a capture, so direct
- * launches are the default. Timing level 2 always launches directly (its events are attached to
- * the SpMV launches). */
+ * lists). A solver on which neither this nor lcsx_solver_set_spmv_shape was called runs a solve of one
+ * scene as a single launch where the system fits (up to 131,072 rows of at most 12 blocks, 65,536 of at
+ * most 32, and contacts that are few beside the rows), otherwise as three launches per iteration. This
+ * call selects the launches: 1 captures each convergence-test interval of PCG iterations as a hipGraph
+ * and replays it; 0 launches every kernel directly. Every form adds up the same terms in the same
+ * order. On MI355X the replay does not shorten the device time of a solve (the gaps between
+ * dependent kernels remain) and each new chunk shape costs a capture. Timing level 2 always launches
+ * directly (its events are attached to the SpMV launches). */
 lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on);
 /* LBVH traversal shape of the solver's broad-phase queries (no counterpart in the reference; the
  * same pairs in every shape). Binary steps (one 64 B record, two children tested per step, the
@@ -305,7 +307,7 @@ lcsx_status lcsx_solver_set_query_shape(lcsx_solver* s, int shape);
  * drop its product by a select); 1: three blocks per pass with loads predicated on the row's
  * width; 2: two blocks per pass, unconditional. 3-5: the same with the contact-slot chunks launched
  * before the row blocks (their dependent loads then overlap the row blocks' streaming); 3 is the
- * default. */
+ * default. Selects the launched form of the PCG, as lcsx_solver_set_graphs does. */
 lcsx_status lcsx_solver_set_spmv_shape(lcsx_solver* s, int shape);
 /* Autotuner (no counterpart in the reference): times the runtime mappings on the current state
  * and keeps the fastest of each: the CCD first-pass iteration budget (8..128), the PCG launch
@@ -376,13 +378,13 @@ typedef struct lcsx_pcg_result
     float rz0, rz;    /* r.z at the start and at the last evaluated iteration                  */
 } lcsx_pcg_result;
 void lcsx_pcg_options_default(lcsx_pcg_options* o);
-/* Solves A x = b on `stream` (a hipStream_t, NULL = default); allocates its scratch (about 104 B
+/* Solves A x = b on `stream` (a hipStream_t, NULL = default); allocates its scratch (about 128 B
  * per row) for the call and frees it before returning. */
 lcsx_status lcsx_pcg_solve_bsr(const lcsx_bsr* A, const float* device_b, float* device_x,
                                const lcsx_pcg_options* options, void* stream, lcsx_pcg_result* result);
 /* No counterpart in the reference: lcsx_pcg_solve_bsr for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). The
- * same solve with its scratch in a static device array of the library (one per GPU, about 14 MB,
+ * same solve with its scratch in a static device array of the library (one per GPU, about 17 MB,
  * held until the process ends) instead of an allocation; calls no hipMalloc or hipFree. At most
  * 131072 rows (LCSX_ERR_ARG above). Every call on one GPU shares that GPU's scratch: calls that
  * overlap on one GPU (other host threads, or other streams still running an earlier call) race. */

@@ -781,6 +781,7 @@ lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on)
 {
     if (!s || (on != 0 && on != 1)) return arg_error("invalid arguments");
     s->s.use_graphs = on == 1;
+    s->s.pcg_grid   = false;  // the caller chooses the form of the launches
     return LCSX_OK;
 }
 
@@ -795,6 +796,7 @@ lcsx_status lcsx_solver_set_spmv_shape(lcsx_solver* s, int shape)
 {
     if (!s || shape < 0 || shape >= kSpmvShapes) return arg_error("invalid arguments");
     s->s.spmv_shape = shape;
+    s->s.pcg_grid   = false;  // a mapping of the launched product
     return LCSX_OK;
 }
 

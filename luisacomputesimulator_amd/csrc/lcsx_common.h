@@ -125,11 +125,48 @@ LCSX_D uint32_t wave_append(uint32_t* counter, bool pred)
     return base + (uint32_t)__popcll(mask & lanemask_lt());
 }
 
+// v + (v of the lane whose index differs in bit O), without a trip through LDS: rows and halves of
+// the wavefront are swapped by v_permlane16/32_swap, lanes within a row of 16 by DPP. Addition
+// commutes, so both lanes of a pair get the same bits as from __shfl_xor.
+template <int O>
+LCSX_D float xor_add(float v)
+{
+    const int i = __float_as_int(v);
+    if constexpr (O == 32 || O == 16)
+    {
+        const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap(i, i, false, false)
+                               : __builtin_amdgcn_permlane16_swap(i, i, false, false);
+        return __int_as_float((int)r[0]) + __int_as_float((int)r[1]);
+    }
+    else
+    {
+        int o;
+        if constexpr (O == 8) o = __builtin_amdgcn_mov_dpp(i, 0x128, 0xf, 0xf, true);  // row_ror:8
+        else if constexpr (O == 4)
+        {
+            // row_half_mirror (lane ^ 7), then quad_perm [3, 2, 1, 0] (lane ^ 3)
+            o = __builtin_amdgcn_mov_dpp(i, 0x141, 0xf, 0xf, true);
+            o = __builtin_amdgcn_mov_dpp(o, 0x1b, 0xf, 0xf, true);
+        }
+        else if constexpr (O == 2) o = __builtin_amdgcn_mov_dpp(i, 0x4e, 0xf, 0xf, true);  // [2, 3, 0, 1]
+        else o = __builtin_amdgcn_mov_dpp(i, 0xb1, 0xf, 0xf, true);                        // [1, 0, 3, 2]
+        return v + __int_as_float(o);
+    }
+}
+template <int O>
+LCSX_D f3 xor_add(f3 v)
+{
+    return {xor_add<O>(v.x), xor_add<O>(v.y), xor_add<O>(v.z)};
+}
 template <class T>
 LCSX_D T wave_sum(T v)
 {
     for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o);
     return v;
+}
+LCSX_D float wave_sum(float v)
+{
+    return xor_add<1>(xor_add<2>(xor_add<4>(xor_add<8>(xor_add<16>(xor_add<32>(v))))));
 }
 LCSX_D float wave_min(float v)
 {

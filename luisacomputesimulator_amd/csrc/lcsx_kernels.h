@@ -48,7 +48,9 @@ struct SegView
 struct PcgState
 {
     float    rz[2], rz0;
-    uint32_t converged, iters, nan, pad[2];
+    uint32_t converged, iters, nan;
+    uint32_t bad_index;  // block-CSR solves: a column or row range lies outside the matrix
+    uint32_t fail;       // the one-launch form gave up (lcsx_pcg_grid.h); the solve starts over
 };
 
 // SELL-16 block matrix: rows in slices of 16; slice s stores sl_off[s + 1] - sl_off[s] block
@@ -411,6 +413,40 @@ constexpr int kSpmvShapeDefault = 3;
 void launch_pcg_spmv(const PcgArgs& a, const SellView& A, const VertContacts& vc, unsigned max_chunks, int shape,
                      hipStream_t s, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 void launch_pcg_update(const PcgArgs& a, hipStream_t s);
+
+// The PCG in one launch (lcsx_pcg_grid.h): limits, shape and workspace.
+constexpr uint32_t kGridRows  = 4096;  // rows whose p a workgroup holds: its own and those its columns name
+constexpr uint32_t kGridOwn   = 512;   // own rows of a workgroup
+constexpr uint32_t kGridVals  = 8192;  // partial sums of one kind
+constexpr uint32_t kGridWgs   = 256;   // workgroups: one per CU
+constexpr uint32_t kGridThreads = 512;
+constexpr size_t   kGridWords = 2 * (size_t)kGridVals;  // 8-byte words posted by the workgroups
+struct GridSync
+{
+    unsigned long long* slots;  // kGridWords, zero before the first launch
+    unsigned long long* zx;     // 3 words per row, zero before the first launch: z as it is exchanged
+    uint32_t            epoch;  // of the launch's first iteration (from 2); later launches use later ones
+};
+struct GridPlan
+{
+    unsigned wgs = 0;       // 0: the launches are used
+    int      U = 0, K = 0;  // row groups per thread and blocks per thread and row
+};
+// The shape for n_rb row blocks of at most `width` blocks a row, with at most `chunks` contact-slot
+// chunks.
+GridPlan grid_plan(uint32_t n_rb, uint32_t width, uint32_t chunks);
+// Iterations [a.k, a.k + len) of a solve begun by launch_pcg_init (k_bsr_init), one scene.
+void launch_pcg_grid(const GridPlan& p, const PcgArgs& a, const SellView& A, const ContactView& c,
+                     const VertContacts& vc, const GridSync& g, uint32_t len, hipStream_t s);
+void launch_grid_clear(unsigned long long* words, size_t n, hipStream_t s);
+// One such launch runs at a time per GPU in a process (its workgroups wait for each other, so all
+// must be resident); without the lease a solve uses the launches, which give the same bits.
+struct GridLease
+{
+    int  dev = -1;
+    bool take(int device);
+    ~GridLease();
+};
 // Mixed precision: FP16 copy of the off-diagonal blocks with a power-of-two scale per block.
 void launch_energy(const EnergyArgs& a, unsigned contact_grid, uint32_t nscenes, hipStream_t s);
 void launch_pack_fp16(uint32_t nslices, uint32_t n, const uint32_t* sl_off, uint32_t nblocks, const float* val,

@@ -2,9 +2,12 @@
 // narrow phase, contact assembly, SELL-16 block SpMV, block-Jacobi PCG and line search.
 // Reference counterparts are cited per kernel (paths relative to the reference root).
 #include <hip/hip_ext.h>
+#include <atomic>
+#include <type_traits>
 #include "lcsx_fp64.h"
 #include "lcsx_internal.h"
 #include "lcsx_kernels.h"
+#include "lcsx_pcg_grid.h"
 #include "lcsx_physics.h"
 
 namespace lcsx
@@ -1254,7 +1257,8 @@ LCSX_D void contact_t(const ContactView& c, float* __restrict__ tc, PF pfun)
 // One 64-slot chunk per wavefront, starting at `base`: slot contributions a t_c are summed over
 // each run of equal rows by a segmented shuffle scan (slots are in row order); the last lane of
 // a run returns true with the run's row and sum. Called by all 64 lanes.
-LCSX_D bool slot_chunk(const VertContacts& vc, uint32_t base, uint32_t end, uint32_t& row, f3& sum)
+template <class TF>
+LCSX_D bool slot_chunk(const VertContacts& vc, uint32_t base, uint32_t end, uint32_t& row, f3& sum, TF tcf)
 {
     const uint32_t lane = lane_id();
     uint32_t       e    = base + lane;
@@ -1264,7 +1268,7 @@ LCSX_D bool slot_chunk(const VertContacts& vc, uint32_t base, uint32_t end, uint
     if (ok)
     {
         float4 C = vc.coef[e];
-        float  t = vc.tc[__float_as_uint(C.w)];
+        float  t = tcf(__float_as_uint(C.w));
         row      = vc.row[e];
         vx       = C.x * t;
         vy       = C.y * t;
@@ -1285,23 +1289,37 @@ LCSX_D bool slot_chunk(const VertContacts& vc, uint32_t base, uint32_t end, uint
     sum         = mk(vx, vy, vz);
     return ok && (lane == 63u || rn != row);
 }
+LCSX_D bool slot_chunk(const VertContacts& vc, uint32_t base, uint32_t end, uint32_t& row, f3& sum)
+{
+    return slot_chunk(vc, base, end, row, sum, [&](uint32_t c) { return vc.tc[c]; });
+}
 
 // Adds row i's contact runs to y in slot order. The wavefronts that summed the runs start at
 // s0 + 64 m, so the row's runs end at every wavefront end s0 + 64 m + 63 inside its slots
 // [ptr[i], ptr[i + 1]) and at its last slot. No atomics: the sum does not depend on which
 // wavefront finished first.
-LCSX_D f3 fold_runs(f3 y, const float4* __restrict__ runsum, const uint32_t* __restrict__ ptr, uint32_t i, uint32_t s0)
+template <class RF>
+LCSX_D f3 fold_runs_of(f3 y, RF runsum, const uint32_t* __restrict__ ptr, uint32_t i, uint32_t s0)
 {
     const uint32_t b = ptr[i], e = ptr[i + 1];
     if (e <= b) return y;
     for (uint32_t w = s0 + ((b - s0) & ~63u) + 63u;; w += 64u)
     {
         const uint32_t end = min(w, e - 1u);
-        const float4   R   = runsum[end];
-        y                  = y + mk(R.x, R.y, R.z);
+        y                  = y + runsum(end);
         if (end == e - 1u) break;
     }
     return y;
+}
+LCSX_D f3 fold_runs(f3 y, const float4* __restrict__ runsum, const uint32_t* __restrict__ ptr, uint32_t i, uint32_t s0)
+{
+    return fold_runs_of(
+        y,
+        [&](uint32_t e) {
+            const float4 R = runsum[e];
+            return mk(R.x, R.y, R.z);
+        },
+        ptr, i, s0);
 }
 
 // Scalars of PCG iteration k (precond_cg.cpp:681-726 and the loop of 118-330): r.z from the
@@ -1400,6 +1418,7 @@ __global__ __launch_bounds__(kB) void k_pcg_init(PcgArgs a)
             st->converged = on ? 0u : 1u;
             st->iters     = 0u;
             st->nan       = 0u;
+            st->fail      = 0u;
             st->rz[0] = st->rz[1] = st->rz0 = 0.0f;
         }
     }
@@ -1638,12 +1657,7 @@ __global__ __launch_bounds__(kB) void k_spmv_pcg(PcgArgs a, SellView A, VertCont
             }
         }
         // the row's four lanes hold partial sums: lanes l, l + 16, l + 32, l + 48
-        y.x = y.x + __shfl_xor(y.x, 16);
-        y.y = y.y + __shfl_xor(y.y, 16);
-        y.z = y.z + __shfl_xor(y.z, 16);
-        y.x = y.x + __shfl_xor(y.x, 32);
-        y.y = y.y + __shfl_xor(y.y, 32);
-        y.z = y.z + __shfl_xor(y.z, 32);
+        y = xor_add<32>(xor_add<16>(y));
         if (valid && j < 3u) a.q[3 * (size_t)i + j] = get(y, (int)j);
         if (valid && j == 0u) loc = dot(pi, y);
         const float bs = block_sum(loc, sh);
@@ -2017,6 +2031,198 @@ __global__ __launch_bounds__(kB) void k_pcg_update(PcgArgs a)
     }
     float bs = block_sum(loc, sh);
     if (threadIdx.x == 0) a.part_rz[rbi] = bs;
+}
+
+// ---------------------------------------------------------------- PCG in one launch (lcsx_pcg_grid.h)
+// The SELL-16 matrix and the contact slots as k_pcg_grid reads them.
+template <int LP>
+struct GridSell
+{
+    SellView A;
+    uint32_t n;
+    struct Row
+    {
+        uint32_t b0, count;  // block k at b0 + 16 k
+        bool     ok;
+    };
+    using Raw = typename std::conditional<LP != 0, PackedBlock, m3>::type;
+    LCSX_D Row row(uint32_t i) const
+    {
+        const uint32_t s = i >> 4, k0 = A.sl_off[s];
+        return Row{k0 * kSellH + (i & 15u), A.sl_off[s + 1] - k0, true};
+    }
+    LCSX_D uint32_t col(const Row& r, uint32_t k) const { return A.col[r.b0 + kSellH * k]; }
+    LCSX_D Raw      load(const Row& r, uint32_t k) const
+    {
+        if constexpr (LP != 0) return sell_words(A, r.b0 + kSellH * k);
+        else return sell_block32(A, r.b0 + kSellH * k);
+    }
+    LCSX_D m3 get(const Raw& w, uint32_t i, uint32_t k, bool on) const
+    {
+        if constexpr (LP != 0)
+        {
+            // a block kept in FP32 (an affine body's row) is read from its planes
+            const bool keep = (int)(int8_t)((w.w[4] >> 16) & 0xffu) == kKeepFp32;
+            return sell_unpack<LP>(A, on && keep ? (size_t)(A.sl_off[i >> 4] + k) * kSellH + (i & 15u) : 0, w);
+        }
+        else
+            return w;
+    }
+    LCSX_D m3   diag(uint32_t i) const { return ld_planes(A.diag, n, i); }
+    LCSX_D m3   minv(const float* P, uint32_t i) const { return ld_planes(P, n, i); }
+    LCSX_D void bad_column() const {}
+    // keeps the decoding of 16-bit blocks inside the iteration: hoisted out of it, the decoded blocks
+    // would take nearly twice the registers
+    template <int U, int K>
+    LCSX_D void opaque(Raw (&W)[U][K]) const
+    {
+        if constexpr (LP != 0)
+        {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int k = 0; k < K; k++)
+#pragma unroll
+                    for (int c = 0; c < 5; c++) asm volatile("" : "+v"(W[u][k].w[c]));
+        }
+    }
+};
+struct GridContacts
+{
+    ContactView  c;
+    VertContacts vc;
+    uint32_t     n = 0, nch = 0, end = 0;
+    LCSX_D void  begin(const PcgArgs& a)
+    {
+        n   = min(*c.count, c.capacity);
+        nch = a.seg.sc_cb0[1];
+        end = vc.ptr[a.n];
+    }
+    LCSX_D uint32_t chunks() const { return nch; }
+    // p = z + beta p_old of four rows at once (kInvalid: none), every load in flight before the first is
+    // used
+    struct P4
+    {
+        f3 p[4];
+    };
+    LCSX_D P4 rows4(const PcgArgs& a, const grid::Word* zx, bool first, uint32_t zep, const float* p_old, float beta,
+                    const uint32_t (&r)[4], uint32_t& bad) const
+    {
+        P4 o;
+        if (first)
+        {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+            {
+                const uint32_t v = r[j] != kInvalid ? r[j] : 0u;
+                o.p[j]           = ld3(a.z, v) + beta * ld4(p_old, v);
+            }
+            return o;
+        }
+        f3 po[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) po[j] = grid::ld_row(p_old, r[j] != kInvalid ? r[j] : 0u);
+        for (uint32_t tries = 0;; tries++)
+        {
+            grid::Word w[4][3];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+            {
+                const uint32_t v = r[j] != kInvalid ? r[j] : 0u;
+#pragma unroll
+                for (int d = 0; d < 3; d++) w[j][d] = grid::peek(zx + d * (size_t)a.n + v);
+            }
+            bool ok = true;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) ok = ok && (r[j] == kInvalid || grid::epoch_of(w[j][d]) == zep);
+            if (!ok && tries > grid::kPolls) bad = 1u;
+            if (ok || *(volatile uint32_t*)&bad != 0u)
+            {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    o.p[j] = mk(grid::value_of(w[j][0]), grid::value_of(w[j][1]), grid::value_of(w[j][2])) + beta * po[j];
+                return o;
+            }
+        }
+    }
+    // The runs of this workgroup's 256-slot chunks and their p.q partials. p of other workgroups' rows
+    // is z + beta p_old again, and every slot evaluates its contact's t_c itself (contact_t1's
+    // expression, so the same bits): a wait of all workgroups for the t_c would cost more than the
+    // repetition as long as the contacts are few (grid_plan's limit).
+    LCSX_D void slots(const PcgArgs& a, const grid::Word* zx, bool first, uint32_t zep, const float* p_old, float beta,
+                      grid::Word* words, uint32_t epoch, float* sh, uint32_t& bad) const
+    {
+        const uint32_t gpw = blockDim.x >> 8, grp = threadIdx.x >> 8, wv = threadIdx.x >> 6;
+        for (uint32_t base = blockIdx.x * gpw; base < nch; base += gridDim.x * gpw)
+        {
+            const uint32_t ch  = base + grp;
+            float          loc = 0.0f;
+            if (ch < nch)
+            {
+                uint32_t       row;
+                f3             sum, pr = mk(0.0f, 0.0f, 0.0f);
+                const uint32_t b = 256u * ch + (threadIdx.x & 192u);
+                auto           tf = [&](uint32_t k) {
+                    const uint4  ga = c.gr[2 * (size_t)k], gb = c.gr[2 * (size_t)k + 1];
+                    const float4 wa = c.gw[2 * (size_t)k], wb = c.gw[2 * (size_t)k + 1];
+                    const float4 nk = c.nk[k];
+                    const f3     nn = mk(nk.x, nk.y, nk.z);
+                    const uint32_t own = vc.row[b + lane_id()];
+                    const uint32_t ra[4] = {ga.x, ga.y, ga.z, ga.w}, rb[4] = {gb.x, gb.y, gb.z, gb.w};
+                    const float    fa[4] = {wa.x, wa.y, wa.z, wa.w}, fb[4] = {wb.x, wb.y, wb.z, wb.w};
+                    const P4       A = rows4(a, zx, first, zep, p_old, beta, ra, bad);
+                    float          t = fa[0] * dot(nn, A.p[0]);
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                    {
+                        if (j > 0 && ra[j] != kInvalid) t = t + fa[j] * dot(nn, A.p[j]);
+                        if (ra[j] == own) pr = A.p[j];
+                    }
+                    if (rb[0] != kInvalid || rb[1] != kInvalid || rb[2] != kInvalid || rb[3] != kInvalid)
+                    {
+                        const P4 B = rows4(a, zx, first, zep, p_old, beta, rb, bad);
+#pragma unroll
+                        for (int j = 0; j < 4; j++)
+                        {
+                            if (rb[j] != kInvalid) t = t + fb[j] * dot(nn, B.p[j]);
+                            if (rb[j] == own) pr = B.p[j];
+                        }
+                    }
+                    return t;
+                };
+                if (slot_chunk(vc, b, end, row, sum, tf))
+                {
+                    grid::st_row(reinterpret_cast<float*>(vc.runsum), b + lane_id(), sum);
+                    loc = dot(pr, sum);
+                }
+            }
+            loc = wave_sum(loc);
+            if (lane_id() == 0) sh[wv] = loc;
+            grid::stores_done();  // the runs' sums, before the word that announces them
+            __syncthreads();
+            if ((threadIdx.x & 255u) == 0u && ch < nch)
+                grid::post(words + ch, ((sh[wv] + sh[wv + 1]) + sh[wv + 2]) + sh[wv + 3], epoch);
+            __syncthreads();
+        }
+    }
+    LCSX_D void poison(grid::Word* words) const
+    {
+        const uint32_t gpw = blockDim.x >> 8;
+        for (uint32_t base = blockIdx.x * gpw; base < nch; base += gridDim.x * gpw)
+            for (uint32_t ch = base; ch < min(base + gpw, nch); ch++) grid::post(words + ch, 0.0f, grid::kPoison);
+    }
+    LCSX_D f3 fold(f3 q, uint32_t i) const
+    {
+        return fold_runs_of(
+            q, [&](uint32_t e) { return grid::ld_row(reinterpret_cast<const float*>(vc.runsum), e); }, vc.ptr, i,
+            vc.ptr[0]);
+    }
+};
+__global__ void k_grid_clear(unsigned long long* w, size_t n)
+{
+    for (size_t i = blockIdx.x * kB + threadIdx.x; i < n; i += (size_t)gridDim.x * kB) w[i] = 0ull;
 }
 
 // Standalone narrow phase: the pair count and the CCD's rest count and step bound of one call.
@@ -2410,6 +2616,74 @@ void launch_residual(const SegView& g, const float* b, const float* y, const flo
     k_residual<<<g.n_rb, kB, 0, s>>>(g, b, y, minv, r, z, part_rz, part_res);
 }
 void launch_pcg_update(const PcgArgs& a, hipStream_t s) { k_pcg_update<<<a.seg.n_rb, kB, 0, s>>>(a); }
+void launch_grid_clear(unsigned long long* w, size_t n, hipStream_t s)
+{
+    if (n) k_grid_clear<<<std::min(1024u, grid_for(n, kB)), kB, 0, s>>>(w, n);
+}
+// One workgroup per row block up to 256 of them (one per CU), two row blocks each up to 512: a wait for
+// more workgroups costs more than the second block's product. Blocks per thread and row (K, four
+// threads a row) are what fits 256 registers beside the rows' vectors. Contact slots: at most two
+// chunks per 256 threads; each costs an iteration about 4 us, the launches' whole contact part 5-10 us.
+GridPlan grid_plan(uint32_t n_rb, uint32_t width, uint32_t chunks)
+{
+    GridPlan p;
+    const int      K = width <= 12u ? 3 : (width <= 16u ? 4 : (width <= 32u ? 8 : 0));
+    const int      U = n_rb <= kGridWgs ? 2 : 4;
+    const uint32_t G = U == 2 ? n_rb : (n_rb + 1u) / 2u;
+    if (K == 0 || n_rb == 0 || G > kGridWgs || (U == 4 && K > 3)) return p;
+    if (chunks > 2u * G * (kGridThreads / 256u) || 4u * n_rb + chunks > kGridVals) return p;
+    p.wgs = G;
+    p.U   = U;
+    p.K   = K;
+    return p;
+}
+template <class Mat, class Ct, bool CT>
+static void grid_go(const GridPlan& p, const PcgArgs& a, const Mat& A, const Ct& ct, const GridSync& g, uint32_t len,
+                    hipStream_t s)
+{
+    auto go = [&](auto kern) { kern<<<p.wgs, kGridThreads, 0, s>>>(a, A, ct, g, len); };
+    if (p.U == 4) go(k_pcg_grid<Mat, 4, 3, CT, Ct>);
+    else if (p.K == 3) go(k_pcg_grid<Mat, 2, 3, CT, Ct>);
+    else if (p.K == 4) go(k_pcg_grid<Mat, 2, 4, CT, Ct>);
+    else go(k_pcg_grid<Mat, 2, 8, CT, Ct>);
+    LCSX_HIP(hipGetLastError());
+}
+template <int LP>
+static void grid_lp(const GridPlan& p, const PcgArgs& a, const SellView& A, const ContactView& c,
+                    const VertContacts& vc, const GridSync& g, uint32_t len, hipStream_t s)
+{
+    const GridSell<LP> M{A, a.n};
+    if (vc.ptr)
+    {
+        GridContacts ct;
+        ct.c  = c;
+        ct.vc = vc;
+        grid_go<GridSell<LP>, GridContacts, true>(p, a, M, ct, g, len, s);
+    }
+    else
+        grid_go<GridSell<LP>, NoContacts, false>(p, a, M, NoContacts{}, g, len, s);
+}
+void launch_pcg_grid(const GridPlan& p, const PcgArgs& a, const SellView& A, const ContactView& c,
+                     const VertContacts& vc, const GridSync& g, uint32_t len, hipStream_t s)
+{
+    if (A.val_p && A.bf16) grid_lp<2>(p, a, A, c, vc, g, len, s);
+    else if (A.val_p) grid_lp<1>(p, a, A, c, vc, g, len, s);
+    else grid_lp<0>(p, a, A, c, vc, g, len, s);
+}
+namespace
+{
+std::atomic<bool> g_grid_busy[64];
+}
+bool GridLease::take(int device)
+{
+    if (device < 0 || device >= 64 || g_grid_busy[device].exchange(true)) return false;
+    dev = device;
+    return true;
+}
+GridLease::~GridLease()
+{
+    if (dev >= 0) g_grid_busy[dev].store(false);
+}
 void launch_spmv(const SellView& A, const ContactView& c, const VertContacts& vc, unsigned contact_grid, const float* p,
                  float* y, uint32_t n, hipStream_t s)
 {

@@ -6,10 +6,10 @@
 // The iteration is the reference's: x0 = 0, r = b, z = M^-1 r, beta = r.z / r.z_old (0 when r.z_old
 // is below 1e-10), p = z + beta p, q = A p, alpha = r.z / p.q (0 when p.q is below 1e-10),
 // x += alpha p, r -= alpha q; the solve stops when r.z < abs_tol (or r.z <= rel_tol^2 r0.z0, or
-// NaN), tested every check_every iterations, or after max_iters iterations. Each iteration is three
-// launches (direction, product, update); every block re-reduces the previous launch's per-block
-// partials in a fixed order, so no grid-wide synchronisation is needed and results do not depend
-// on scheduling.
+// NaN), tested every check_every iterations, or after max_iters iterations. A system that fits runs in
+// one launch (k_pcg_grid, lcsx_pcg_grid.h); otherwise, or where that form gives up, each iteration is
+// three launches (direction, product, update), whose blocks re-reduce the previous launch's per-block
+// partials in a fixed order. Both give the same bits, and results do not depend on scheduling.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,6 +20,8 @@
 #include "../../include/lcsx.h"
 #include "lcsx_common.h"
 #include "lcsx_internal.h"
+#include "lcsx_kernels.h"
+#include "lcsx_pcg_grid.h"
 
 namespace lcsx
 {
@@ -30,12 +32,7 @@ constexpr int      kProdB   = 256;  // product: 64 rows per block, 4 lanes per r
 constexpr uint32_t kAlign   = 64;   // scratch regions start on 256-byte boundaries (floats)
 constexpr uint32_t kNoAllocRows = 131072;  // largest system of lcsx_pcg_solve_bsr_noalloc
 
-// Scalars shared between launches.
-struct BsrState
-{
-    float    rz[2], rz0, pad0;
-    uint32_t converged, iters, nan, bad_index;
-};
+using BsrState = PcgState;  // scalars shared between launches
 
 // Scratch of one solve (device pointers into one allocation).
 struct BsrWork
@@ -47,9 +44,14 @@ struct BsrWork
     float*    p[2];   // 4 per row
     float*    q;      // 3 per row
     float*    part_rz;
-    float*    part_pq;  // one per product block
+    float*    part_pq;  // four per row block: one per product block of 64 rows
     BsrState* st;
+    unsigned long long* words;  // of the one-launch form: kGridWords, then z's (3 per row); cleared by the init
+    uint32_t            n_words;
 };
+
+constexpr uint32_t kGridBsrRows = 2 * kGridWgs * 256;  // most rows of the one-launch form
+constexpr uint32_t grid_words(uint32_t n) { return n <= kGridBsrRows ? (uint32_t)kGridWords + 3u * n : 0u; }
 
 constexpr uint32_t align_up(uint32_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
@@ -63,8 +65,8 @@ lcsx_status arg_error(const char* m)
 constexpr size_t work_floats(uint32_t n)
 {
     return (size_t)align_up(9 * n) + 2 * (size_t)align_up(3 * n) + 2 * (size_t)align_up(4 * n) + align_up(3 * n) +
-           align_up((n + kB - 1) / kB) + align_up((n + kProdB / 4 - 1) / (kProdB / 4)) +
-           align_up(sizeof(BsrState) / 4);
+           align_up((n + kB - 1) / kB) + align_up(4 * ((n + kB - 1) / kB)) + align_up(sizeof(BsrState) / 4) +
+           align_up(2 * grid_words(n));
 }
 
 BsrWork carve(float* base, uint32_t n)
@@ -72,7 +74,6 @@ BsrWork carve(float* base, uint32_t n)
     BsrWork w{};
     w.n             = n;
     w.nb            = (n + kB - 1) / kB;
-    const uint32_t np = (n + kProdB / 4 - 1) / (kProdB / 4);
     float* c        = base;
     auto   take     = [&](uint32_t k) {
         float* o = c;
@@ -86,8 +87,10 @@ BsrWork carve(float* base, uint32_t n)
     w.p[1]    = take(4 * n);
     w.q       = take(3 * n);
     w.part_rz = take(w.nb);
-    w.part_pq = take(np);
+    w.part_pq = take(4 * w.nb);
     w.st      = reinterpret_cast<BsrState*>(take(sizeof(BsrState) / 4));
+    w.n_words = grid_words(n);
+    w.words   = reinterpret_cast<unsigned long long*>(take(2 * w.n_words));
     return w;
 }
 
@@ -147,6 +150,7 @@ __global__ __launch_bounds__(kB) void k_bsr_init(BsrWork w, const float* __restr
     __shared__ float sh[4];
     const uint32_t   i   = blockIdx.x * kB + threadIdx.x;
     float            loc = 0.0f;
+    for (uint32_t k = i; k < w.n_words; k += gridDim.x * kB) w.words[k] = 0ull;
     if (i < w.n)
     {
         const m3     D = ld9(diag, i);
@@ -188,7 +192,7 @@ __global__ __launch_bounds__(kB) void k_bsr_init(BsrWork w, const float* __restr
         if (blockIdx.x == 0)
         {
             w.st->rz[0] = w.st->rz[1] = w.st->rz0 = 0.0f;
-            w.st->converged = w.st->iters = w.st->nan = w.st->bad_index = 0u;
+            w.st->converged = w.st->iters = w.st->nan = w.st->bad_index = w.st->fail = 0u;
         }
     }
 }
@@ -256,23 +260,18 @@ __global__ __launch_bounds__(kProdB) void k_bsr_spmv(BsrWork w, uint32_t k, cons
                 y = y + mul(ld9(blocks, (size_t)kk), ldp(p, (uint32_t)c));
             }
     }
-    y.x = y.x + __shfl_xor(y.x, 16);
-    y.y = y.y + __shfl_xor(y.y, 16);
-    y.z = y.z + __shfl_xor(y.z, 16);
-    y.x = y.x + __shfl_xor(y.x, 32);
-    y.y = y.y + __shfl_xor(y.y, 32);
-    y.z = y.z + __shfl_xor(y.z, 32);
+    y = xor_add<32>(xor_add<16>(y));
     if (valid && j < 3u) w.q[3 * (size_t)i + j] = get(y, (int)j);
     const float s = bsum(valid && j == 0u ? dot(pi, y) : 0.0f, sh);
     if (threadIdx.x == 0) w.part_pq[blockIdx.x] = s;
 }
 
 // alpha = r.z / p.q; x += alpha p, r -= alpha q, z = Minv r, r.z partials.
-__global__ __launch_bounds__(kB) void k_bsr_update(BsrWork w, uint32_t k, uint32_t np, float* __restrict__ x)
+__global__ __launch_bounds__(kB) void k_bsr_update(BsrWork w, uint32_t k, float* __restrict__ x)
 {
     __shared__ float sh[4];
     if (flag_set(&w.st->converged)) return;
-    const float    pq    = reduce_all(w.part_pq, np, sh);
+    const float    pq    = reduce_all(w.part_pq, 4 * w.nb, sh);
     const float    rz    = w.st->rz[k & 1u];
     const float    alpha = pq < 1e-10f ? 0.0f : rz / pq;
     const uint32_t i     = blockIdx.x * kB + threadIdx.x;
@@ -328,12 +327,7 @@ __global__ __launch_bounds__(kProdB) void k_bsr_apply(uint32_t n, const int32_t*
                 acc = acc + mul(ld9(blocks, (size_t)kk), ld3(x, (uint32_t)c));
             }
     }
-    acc.x = acc.x + __shfl_xor(acc.x, 16);
-    acc.y = acc.y + __shfl_xor(acc.y, 16);
-    acc.z = acc.z + __shfl_xor(acc.z, 16);
-    acc.x = acc.x + __shfl_xor(acc.x, 32);
-    acc.y = acc.y + __shfl_xor(acc.y, 32);
-    acc.z = acc.z + __shfl_xor(acc.z, 32);
+    acc = xor_add<32>(xor_add<16>(acc));
     if (valid && j < 3u) y[3 * (size_t)i + j] = get(acc, (int)j);
 }
 
@@ -424,7 +418,7 @@ __global__ __launch_bounds__(kB) void k_op_init(OpWork w, const float* __restric
         if (blockIdx.x == 0)
         {
             w.st->rz[0] = w.st->rz[1] = w.st->rz0 = 0.0f;
-            w.st->converged = w.st->iters = w.st->nan = w.st->bad_index = 0u;
+            w.st->converged = w.st->iters = w.st->nan = w.st->bad_index = w.st->fail = 0u;
         }
     }
 }
@@ -490,30 +484,110 @@ __global__ __launch_bounds__(kB) void k_op_update(OpWork w, uint32_t k, float* _
     if (threadIdx.x == 0) w.part_rz[blockIdx.x] = sum;
 }
 
+// The block-CSR matrix as k_pcg_grid reads it.
+struct GridBsr
+{
+    const int32_t* row_ptr;
+    const int32_t* cols;
+    const float*   blocks;
+    const float*   dg;
+    BsrState*      st;
+    uint32_t       nnz;
+    struct Row
+    {
+        uint32_t b0, count;
+        bool     ok;
+    };
+    using Raw = m3;
+    LCSX_D Row row(uint32_t i) const
+    {
+        const int32_t r0 = row_ptr[i], r1 = row_ptr[i + 1];
+        const bool    ok = r0 >= 0 && r1 <= (int32_t)nnz && r1 >= r0;
+        if (!ok) bad_column();
+        return Row{(uint32_t)r0, ok ? (uint32_t)(r1 - r0) : 0u, ok};
+    }
+    LCSX_D uint32_t col(const Row& r, uint32_t k) const { return (uint32_t)cols[r.b0 + k]; }
+    LCSX_D m3       load(const Row& r, uint32_t k) const { return ld9(blocks, (size_t)r.b0 + k); }
+    LCSX_D m3       get(const m3& w, uint32_t, uint32_t, bool) const { return w; }
+    LCSX_D m3       diag(uint32_t i) const { return ld9(dg, i); }
+    LCSX_D m3       minv(const float* P, uint32_t i) const { return ld9(P, i); }
+    LCSX_D void     bad_column() const { st->bad_index = 1u; }
+    template <int U, int K>
+    LCSX_D void opaque(m3 (&)[U][K]) const
+    {
+    }
+};
+
+// The shape of the one-launch form. The widest row is not known here: cloth-like matrices have rows
+// of up to one and a half times the mean (a row with more blocks than the shape holds makes the kernel
+// give up before its first iteration).
+GridPlan bsr_plan(const lcsx_bsr* A, uint32_t nb)
+{
+    const double mean = (double)A->nnz / A->n_rows;
+    if (A->n_rows > (int)kGridBsrRows) return GridPlan{};
+    return grid_plan(nb, nb > kGridWgs ? (mean <= 12.0 ? 12u : 64u) : (mean <= 12.0 ? 16u : (mean <= 24.0 ? 32u : 64u)),
+                     0u);
+}
+void launch_bsr_grid(const GridPlan& p, const lcsx_bsr* A, const BsrWork& w, const lcsx_pcg_options& o, float* x,
+                     hipStream_t s)
+{
+    PcgArgs a{};
+    a.n           = w.n;
+    a.minv        = w.minv;
+    a.x           = x;
+    a.r           = w.r;
+    a.z           = w.z;
+    a.p_old       = w.p[0];
+    a.p_new       = w.p[1];
+    a.part_rz     = w.part_rz;
+    a.seg.nscenes = 1u;
+    a.seg.n_rb    = w.nb;
+    a.s           = w.st;
+    a.rel2        = o.rel_tol * o.rel_tol;
+    a.abs_tol     = o.abs_tol;
+    a.check_every = (uint32_t)o.check_every;
+    const GridBsr  M{A->row_ptr, A->col, A->blocks, A->diag, w.st, (uint32_t)A->nnz};
+    const GridSync g{w.words, w.words + kGridWords, 2u};
+    auto go = [&](auto kern) { kern<<<p.wgs, kGridThreads, 0, s>>>(a, M, NoContacts{}, g, (uint32_t)o.max_iters); };
+    if (p.U == 4) go(k_pcg_grid<GridBsr, 4, 3, false, NoContacts>);
+    else if (p.K <= 4) go(k_pcg_grid<GridBsr, 2, 4, false, NoContacts>);
+    else go(k_pcg_grid<GridBsr, 2, 8, false, NoContacts>);
+    LCSX_HIP(hipGetLastError());
+}
+
 // The solve on scratch `base` (work_floats(n) floats, 256-byte aligned).
 lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_options& o, hipStream_t s, float* base,
-                  lcsx_pcg_result* res)
+                  lcsx_pcg_result* res, bool one_launch = true)
 {
     const BsrWork  w  = carve(base, (uint32_t)A->n_rows);
-    const uint32_t np = (w.n + kProdB / 4 - 1) / (kProdB / 4);
     const float    rel2 = o.rel_tol * o.rel_tol;
+    GridPlan       gp;
+    GridLease      lease;
+    if (one_launch && o.max_iters > 0)
+    {
+        int dev = 0;
+        gp      = bsr_plan(A, w.nb);
+        if (gp.wgs && (hipGetDevice(&dev) != hipSuccess || !lease.take(dev))) gp = GridPlan{};
+    }
     k_bsr_init<<<w.nb, kB, 0, s>>>(w, A->diag, b, x);
     LCSX_HIP(hipGetLastError());
     BsrState h{};
     int      issued = 0;
     while (issued < o.max_iters)
     {
-        const int chunk = std::min(std::max(o.check_every, 8), o.max_iters - issued);
-        for (int k = issued; k < issued + chunk; k++)
+        const int chunk = gp.wgs ? o.max_iters : std::min(std::max(o.check_every, 8), o.max_iters - issued);
+        if (gp.wgs) launch_bsr_grid(gp, A, w, o, x, s);
+        for (int k = issued; !gp.wgs && k < issued + chunk; k++)
         {
             k_bsr_dir<<<w.nb, kB, 0, s>>>(w, (uint32_t)k, (uint32_t)o.check_every, o.abs_tol, rel2);
-            k_bsr_spmv<<<np, kProdB, 0, s>>>(w, (uint32_t)k, A->row_ptr, A->col, A->blocks, A->diag, (uint32_t)A->nnz);
-            k_bsr_update<<<w.nb, kB, 0, s>>>(w, (uint32_t)k, np, x);
+            k_bsr_spmv<<<4 * w.nb, kProdB, 0, s>>>(w, (uint32_t)k, A->row_ptr, A->col, A->blocks, A->diag, (uint32_t)A->nnz);
+            k_bsr_update<<<w.nb, kB, 0, s>>>(w, (uint32_t)k, x);
         }
         LCSX_HIP(hipGetLastError());
         issued += chunk;
         LCSX_HIP(hipMemcpyAsync(&h, w.st, sizeof(BsrState), hipMemcpyDeviceToHost, s));
         LCSX_HIP(hipStreamSynchronize(s));
+        if (gp.wgs && h.fail && !h.bad_index) return solve(A, b, x, o, s, base, res, false);
         if (h.converged || h.bad_index) break;
     }
     if (h.bad_index) return arg_error("a block column or row range is outside the matrix");
@@ -544,7 +618,7 @@ lcsx_status check_args(const lcsx_bsr* A, const float* b, float* x, const lcsx_p
 }  // namespace lcsx
 
 // Scratch of lcsx_pcg_solve_bsr_noalloc: every GPU the library runs on holds one copy (about
-// 14 MB, for up to kNoAllocRows rows) until the process ends. In host code `scratch` names a
+// 17 MB, for up to kNoAllocRows rows) until the process ends. In host code `scratch` names a
 // host-side stand-in, not the device array: its device address is taken per device with
 // hipGetSymbolAddress and only that address is passed to kernels.
 static __device__ __align__(256) float scratch[lcsx::work_floats(lcsx::kNoAllocRows)];

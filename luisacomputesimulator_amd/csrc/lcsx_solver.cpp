@@ -190,6 +190,11 @@ void Solver::init()
     minv.alloc(9 * (size_t)nv);
     sell_val.alloc(9 * (size_t)std::max(S.nblocks, 1u));
     part_rz.alloc(S.n_rb + 1);
+    sell_width = 0;
+    for (size_t k = 0; k + 1 < S.sl_off.size(); k++) sell_width = std::max(sell_width, S.sl_off[k + 1] - S.sl_off[k]);
+    pcg_grid = true;
+    grid_slots.free();
+    grid_zx.free();
     // scene tables
     const uint32_t ns = S.nscenes;
     sc_v0_d.upload(S.sc_v0, stream);
@@ -599,6 +604,22 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     const unsigned mc = vc.ptr ? max_chunks(vc.nslots) : 0u;
     launch_pcg_init(a, stream);
     host_pcg.assign(ns, PcgState{});
+    // one launch for all iterations up to the next residual replacement, or three per iteration
+    GridPlan  gp;
+    GridLease lease;
+    if (pcg_grid && ns == 1 && !use_graphs && spmv_sample == 0)
+    {
+        gp = grid_plan(S.n_rb, sell_width, mc);
+        if (gp.wgs && !lease.take(device)) gp = GridPlan{};
+    }
+    if (gp.wgs && (!grid_slots.p || grid_epoch > 0xf0000000u))
+    {
+        if (!grid_slots.p) grid_slots.alloc(kGridWords);
+        if (!grid_zx.p) grid_zx.alloc(3 * (size_t)S.nv);
+        launch_grid_clear(grid_slots.p, grid_slots.n, stream);
+        launch_grid_clear(grid_zx.p, grid_zx.n, stream);
+        grid_epoch = 2;
+    }
     int  issued = 0;
     int  par    = 0;
     bool nan    = false;
@@ -606,9 +627,22 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     {
         // one host check per convergence-test interval (at least kPcgChunk launches), chunks
         // ending at the residual replacements
-        int chunk = std::min(std::max(kPcgChunk, a.check_every > 1 ? (int)a.check_every : 0), max_iters - issued);
+        int chunk = std::min(gp.wgs ? max_iters : std::max(kPcgChunk, a.check_every > 1 ? (int)a.check_every : 0),
+                             max_iters - issued);
         if (replace_every > 0) chunk = std::min(chunk, replace_every - issued % replace_every);
-        if (spmv_sample > 0 || !use_graphs)
+        if (gp.wgs)
+        {
+            PcgArgs b = a;
+            b.p_old   = p[par].p;
+            b.p_new   = p[1 - par].p;
+            b.k       = (uint32_t)issued;
+            const GridSync g{grid_slots.p, grid_zx.p, grid_epoch};
+            grid_epoch += (uint32_t)chunk;
+            launch_pcg_grid(gp, b, A, cv, vc, g, (uint32_t)chunk, stream);
+            par = (par + chunk) & 1;
+            if (timing) times["pcg_grid"].second += 1;  // launches of this form (no time of its own)
+        }
+        else if (spmv_sample > 0 || !use_graphs)
         {
             for (int k = 0; k < chunk; k++)
             {
@@ -689,6 +723,13 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
         }
         LCSX_HIP(hipStreamSynchronize(stream));
         flush_events();
+        if (gp.wgs && host_pcg[0].fail)
+        {
+            // a wait ran out or the gathered rows do not fit: the launches from the start, from now on
+            pcg_grid = false;
+            grid_slots.free();
+            return pcg_run(a, A, cv, vc, max_iters, replace_every);
+        }
         bool done = true;
         for (const PcgState& h : host_pcg)
         {

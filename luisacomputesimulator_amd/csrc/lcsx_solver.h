@@ -185,6 +185,12 @@ struct Solver
     std::map<GraphKey, hipGraphExec_t> pcg_graphs;
     uint64_t graph_epoch = 0;
     bool     use_graphs  = false;
+    // PCG in one launch (lcsx_pcg_grid.h), the default where it fits; off while the caller chooses
+    // the form of the launches (set_graphs, set_spmv_shape) or times them, and after it gave up once
+    bool                     pcg_grid = true;
+    uint32_t                 sell_width = 0;  // most off-diagonal blocks of a row
+    DBuf<unsigned long long> grid_slots, grid_zx;
+    uint32_t                 grid_epoch = 0;
     // runtime mappings chosen by autotune() (defaults: the measured best on the 88K-vertex tube)
     // ACCD iterations per pair in the first CCD pass; pairs that need more run again in a second
     // pass over a compact list, so long iterations do not hold whole wavefronts

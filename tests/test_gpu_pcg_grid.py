@@ -1,0 +1,153 @@
+"""The PCG in one launch (k_pcg_grid) against the same iterations as three launches each: the sums
+are taken over the same partition in the same order, so positions and iteration counts are equal bit
+for bit, frame by frame, without and in contact, in every precision. set_graphs(False) selects the
+launches; a solver left alone takes the one-launch form wherever the system fits it."""
+import numpy as np
+import pytest
+
+from luisacomputesimulator_amd import BsrSystem, LcsxError, NewtonSolver, pcg_solve_bsr, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def boxes():
+    sc = scenes.cloth_rigid_coupling(n=17, boxes=2, seed=3, box_region=((-0.25, 0.25), (0.32, 0.5), (-0.25, 0.25)))
+    for m in sc.meshes[1:]:
+        m.verts[:, 1] -= np.float32(m.verts[:, 1].min() - (0.2 + 1.3e-3))
+    return sc
+
+
+def spring():
+    sc = scenes.square_cloth(21)
+    sc.meshes[0].material.stretch_model = "Spring"
+    return sc
+
+
+def tube_on_ring():
+    """A tube in contact with a short piece of its cylinder: a few thousand contact slots."""
+    sc = scenes.cylinder_tube(rings=96, per_ring=96, cyl_radius=0.1084, cyl_segments=96, cyl_rings=5)
+    n = len(sc.meshes[0].verts)
+    sc.meshes[1].verts[:, 0] *= np.float32(0.05)
+    sc.initial_position[n:, 0] *= np.float32(0.05)
+    return sc
+
+
+# rows: less than one 64-row chunk, one row past it, several workgroups, many
+CASES = {
+    "square_7": (lambda: scenes.square_cloth(7), 3),
+    "square_33": (lambda: scenes.square_cloth(33), 3),
+    "square_65x": (lambda: scenes.twisting_sheet(65), 2),
+    "spring_21": (spring, 3),
+    "sphere_24": (lambda: scenes.cloth_on_sphere(24, 0.02, -0.01, seed=4, sphere_subdiv=2, height=0.3015), 5),
+    "tube_41x48": (lambda: scenes.cylinder_tube(rings=41, per_ring=48, cyl_segments=24, cyl_rings=9), 5),
+    "tube_contact": (tube_on_ring, 2),
+    "boxes": (boxes, 4),
+}
+
+
+@pytest.mark.parametrize("precision", ["fp32", "mixed", "mixed_bf16"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_one_launch_equals_launches(require_gpu, name, precision):
+    make, frames = CASES[name]
+
+    def solver():
+        sc = make()
+        sc.params.precision = precision
+        return NewtonSolver.from_scene(sc)
+
+    one, launches = solver(), solver()
+    launches.set_graphs(False)
+    contacts = 0
+    for f in range(frames):
+        one.physics_step_gpu(1)
+        launches.physics_step_gpu(1)
+        a, b = one.stats(), launches.stats()
+        contacts = max(contacts, a["num_contacts"])
+        print(f"[gpu-grid] {name} {precision} frame {f}: Newton {a['newton_iters']}/{b['newton_iters']}, "
+              f"PCG {a['pcg_iters_total']}/{b['pcg_iters_total']}, contacts {a['num_contacts']}", flush=True)
+        assert a["newton_iters"] == b["newton_iters"] and a["pcg_iters_total"] == b["pcg_iters_total"]
+        assert a["pcg_rel"] == b["pcg_rel"]
+        assert np.array_equal(one.get_simulation_results(), launches.get_simulation_results())
+        assert np.array_equal(one.get_velocities(), launches.get_velocities())
+    assert one.kernel_times()["pcg_grid"][1] > 0 and "pcg_grid" not in launches.kernel_times()
+    if name in ("tube_contact", "sphere_24", "boxes"):
+        assert contacts > 0
+
+
+def banded(n, half, seed):
+    """A diagonally dominant block-CSR system: row i has the columns i - half .. i + half but itself."""
+    rng = np.random.default_rng(seed)
+    i = np.repeat(np.arange(n), 2 * half)
+    c = i + np.tile(np.concatenate([np.arange(-half, 0), np.arange(1, half + 1)]), n)
+    keep = (c >= 0) & (c < n)
+    i, c = i[keep], c[keep]
+    lo, hi = np.minimum(i, c), np.maximum(i, c)
+    v = np.stack([np.sin(lo * 12.9898 + hi * 78.233 + k) for k in range(3)], -1)
+    blocks = -(v[:, :, None] * v[:, None, :]).astype(np.float32)
+    diag = np.zeros((n, 3, 3))
+    np.add.at(diag, i, -blocks.astype(np.float64))
+    diag += 0.05 * np.eye(3)
+    ptr = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))])
+    return BsrSystem(ptr, c, blocks, diag.astype(np.float32)), (i, c, blocks, diag), rng.normal(size=(n, 3))
+
+
+# one row, around a row block's and a workgroup's edge, two row blocks per workgroup (above 65536), and
+# rows wider than any shape holds (24 blocks a row above 65536 rows, 40 below)
+@pytest.mark.parametrize("n,half", [(1, 1), (255, 2), (256, 6), (257, 6), (1000, 6), (1025, 11), (65536, 6), (65537, 6),
+                                    (131072, 3), (70000, 12), (3000, 20)])
+def test_block_csr_solve(require_gpu, n, half):
+    """The residual of 100 iterations against the FP64 recurrence's own, and the solution against the
+    64-bit iterate (1e-4: 100 FP32 iterations of a system of condition below 1e3)."""
+    sysm, (i, c, blocks, diag), b = banded(n, half, n)
+    b = b.astype(np.float32)
+    x, res = pcg_solve_bsr(sysm, b, max_iters=100, check_every=25, abs_tol=0.0)
+    B, D, inv = blocks.astype(np.float64), diag.astype(np.float32).astype(np.float64), None
+    inv = np.linalg.inv(D)
+
+    def mul(p):
+        y = np.einsum("nij,nj->ni", D, p)
+        q = np.einsum("nij,nj->ni", B, p[c])
+        for d in range(3):
+            y[:, d] += np.bincount(i, weights=q[:, d], minlength=n)
+        return y
+
+    xr, r, p, old = np.zeros((n, 3)), b.astype(np.float64), np.zeros((n, 3)), None
+    for _ in range(100):
+        z = np.einsum("nij,nj->ni", inv, r)
+        rz = float((r * z).sum())
+        p = z + (0.0 if old is None or old < 1e-10 else rz / old) * p
+        q = mul(p)
+        pq = float((p * q).sum())
+        a = 0.0 if pq < 1e-10 else rz / pq
+        xr, r, old = xr + a * p, r - a * q, rz
+    err = np.linalg.norm(x - xr) / np.linalg.norm(xr)
+    print(f"[gpu-grid] block CSR n {n}, {2 * half} blocks a row: {res}, error against 64 bits {err:.2e}", flush=True)
+    assert res["iters"] == 100 and err < 1e-4
+
+
+def test_block_csr_scattered_columns(require_gpu):
+    """Columns all over the matrix: a workgroup names more rows than it can hold and the solve starts over
+    with the launches. Against numpy's 64-bit solution."""
+    n, rng = 20000, np.random.default_rng(5)
+    i = np.repeat(np.arange(n), 14)
+    c = rng.integers(0, n, size=i.size)
+    c = np.where(c == i, (c + 1) % n, c)
+    blocks = np.tile(-0.01 * np.eye(3, dtype=np.float32), (i.size, 1, 1))
+    diag = np.tile(np.eye(3, dtype=np.float32), (n, 1, 1))
+    b = rng.normal(size=(n, 3)).astype(np.float32)
+    x, res = pcg_solve_bsr(BsrSystem(np.arange(n + 1) * 14, c, blocks, diag), b, max_iters=4, check_every=4, abs_tol=0.0)
+    assert res["iters"] == 4 and np.isfinite(x).all()
+    # the matrix is not symmetric: only that four iterations reduce the residual as the dominance says
+    r = b - x.astype(np.float64)
+    for d in range(3):
+        r[:, d] += 0.01 * np.bincount(i, weights=x[c, d].astype(np.float64), minlength=n)
+    assert np.linalg.norm(r) < 0.02 * np.linalg.norm(b)
+
+
+def test_block_csr_bad_index_in_the_middle(require_gpu):
+    sysm, _, b = banded(2000, 4, 1)
+    ok = sysm._dev[1].host.copy()
+    bad = BsrSystem(sysm._dev[0].host, np.where(np.arange(len(ok)) == 8003, 2000, ok), sysm._dev[2].host,
+                    sysm._dev[3].host)
+    with pytest.raises(LcsxError, match="outside the matrix"):
+        pcg_solve_bsr(bad, b.astype(np.float32))
