@@ -86,30 +86,25 @@ struct Lbvh
     DBuf<uint32_t>    keys[2], vals[2], hist;
     DBuf<float4>      center;
     DBuf<uint64_t>    morton_sorted;
-    DBuf<uint32_t>    parent, object_idx, counters, gbox;
+    DBuf<uint32_t>    parent, object_idx, gbox;
     DBuf<uint2>       children;
     DBuf<NodeBox>     nodes;
     // per inner node: both child boxes with the child codes in the .w lanes (inner child: its
     // node id; leaf child: 0x80000000 | element id), so a traversal step is one 64 B load
     DBuf<float4>      packed;
-    // level-ordered refit: node depths (pointer jumping: anc / height / counters as buffers), inner
-    // nodes sorted by depth, level offsets
-    DBuf<uint32_t>        height, order, level_hist, level_ptr, level_cursor, anc[2], scan_tmp;
-    std::vector<uint32_t> level_ptr_h;
-    uint32_t              levels = 0;          // deepest level
-    bool                  use_levels = false;  // false: one-pass ticket refit (very tall trees)
-    const uint32_t*       depth = nullptr;     // per inner node (height or counters)
+    DBuf<uint32_t>        scan_tmp;
     // treelet refit: every inner node whose subtree has at most kTreeletLeaves leaves belongs to
     // the treelet of its highest such ancestor; a treelet's inner nodes are a contiguous index
-    // range (Karras layout), refit by one workgroup level by level. The inner nodes above the
-    // treelets ("top"), sorted by depth, are refit by one workgroup afterwards.
-    DBuf<uint32_t>        tsize, tfirst, tleaf, troots, tcount, top_flag, top_pos, top_order, top_level_ptr;
+    // range (Karras layout), refit by one workgroup. The inner nodes above the treelets ("top"),
+    // sorted by depth, are refit by one workgroup afterwards. tcount: treelets, top nodes.
+    DBuf<uint32_t>        tsize, tfirst, tleaf, troots, tcount, top_list, top_depth, top_order, top_level_ptr;
     // per top node (in top_order): its two children's node ids, bit 31 set on a top child, and
     // the top children's indices in top_order (top_idx: node id -> index, top nodes only)
     DBuf<uint4>           top_child;
     DBuf<uint32_t>        top_idx;
-    uint32_t              ntop = 0;   // inner nodes above the treelets
-    std::vector<uint32_t> top_lvp_h;  // top_level_ptr on the host (levels + 2 offsets) when ntop > kTopLds
+    bool                  counted = false;  // ntop and ntreelets were read back (large trees, batches)
+    uint32_t              ntop = 0;         // inner nodes above the treelets
+    std::vector<uint32_t> top_lvp_h;        // top_level_ptr on the host when ntop > kTopLds
     uint32_t              ntreelets = 0;
     // packed keys: largest element id under each child (false) or largest sorted leaf index
     // (true, for sorted self-queries)
@@ -118,7 +113,7 @@ struct Lbvh
     // traversal stack entries past a query's LDS part (grown by lbvh_query as needed)
     mutable DBuf<uint32_t> spill;
     // per inner node: the 4-wide record (the slots of both children's packed records; a leaf
-    // child is one slot and an empty one), written by the level-ordered refit (wide_ready)
+    // child is one slot and an empty one), written by the refit (wide_ready)
     DBuf<float4>      packed4;
     bool              wide_ready = false;
 
@@ -128,6 +123,7 @@ struct Lbvh
     // verts_per_seg: vertices of each segment; the global box of segment g covers its first
     // min(n_g, 256 ceil(verts_g / 256)) leaves (lbvh.cpp:958, 968)
     void construct(const float* x, const uint32_t* verts_per_seg, hipStream_t s);
+    void finish(hipStream_t s);  // construct, from the sorted leaves on
     void refit(const float* x0, const float* x1, const float* pad, hipStream_t s);
     uint32_t n_inner() const { return ni; }
     uint32_t n_nodes() const { return n + ni; }

@@ -3,8 +3,9 @@
 //
 // Semantics follow reference Solver/CollisionDetector/lbvh.cpp (file:line per kernel below);
 // the data path is MI355X-first: the sort runs on the device (the reference sorts on the host
-// and copies keys twice per tree and frame), refit uses one atomic ticket per inner node
-// instead of a float-flag spin protocol, and pair lists are appended with one atomic per wave.
+// and copies keys twice per tree and frame), the refit climbs subtrees of up to 1024 leaves in LDS
+// instead of the whole tree with a float-flag spin protocol, and pair lists are appended with one
+// atomic per staged batch.
 #include "lcsx_internal.h"
 #include "lcsx_physics.h"
 
@@ -16,6 +17,8 @@ namespace
 constexpr int kBlock     = 256;
 constexpr int kSortItems = 16;  // keys per thread per sort pass
 constexpr int kSortTile  = kBlock * kSortItems;
+constexpr uint32_t kTreeletLeaves = 1024;    // most leaves of a treelet
+constexpr uint32_t kUncounted     = 200000;  // largest single tree whose top is not counted on the host
 
 LCSX_HD uint32_t expand_bits(uint32_t b)
 {
@@ -145,6 +148,172 @@ __global__ __launch_bounds__(kBlock) void k_morton(uint32_t n, const float4* __r
     f3     c   = mk(c4.x, c4.y, c4.z) - lo;
     keys[l]    = morton32(mk(c.x * inv.x, c.y * inv.y, c.z * inv.z));
     vals[l]    = l;
+}
+
+// Everything up to the sorted leaves in one workgroup, for one tree of at most kSmallLeaves leaves:
+// the centres, the global box over the first `cover` leaves, the Morton keys, four radix passes in LDS
+// and the leaf records, the values of k_leaf_centers, k_morton, the sort and k_leaves. The launches
+// this replaces (24, of 2-13 us each with as much again in gaps) are what a small tree's construction
+// consists of: 23 us for 3,136 edges. Twice as many leaves per thread as the 8 here spill registers and
+// take 175 us for 14,000 leaves, no less than the launches.
+// A wavefront owns a contiguous stretch of `per` times 64 leaves, so ranking its batches of 64 in
+// order against its own running digit counts keeps the sort stable without a barrier per batch.
+constexpr uint32_t kSmallLeaves = 8192;
+template <int kPer>
+__global__ __launch_bounds__(1024) void k_build_small(uint32_t n, uint32_t ni, int arity, const uint32_t* __restrict__ prims,
+                                                       const float* __restrict__ x, uint32_t cover,
+                                                       uint32_t* __restrict__ gbox, uint64_t* __restrict__ morton_sorted,
+                                                       uint32_t* __restrict__ sorted, uint2* __restrict__ children,
+                                                       uint32_t* __restrict__ object_idx, uint32_t* __restrict__ parent,
+                                                       uint32_t* __restrict__ tcount)
+{
+    constexpr uint32_t kN = 1024u * kPer;
+    __shared__ uint32_t skey[kN];
+    __shared__ uint16_t sval[kN];
+    __shared__ uint32_t cnt[16][256];
+    __shared__ uint32_t wsum[16];
+    __shared__ float    sb[16][6];
+    const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
+    const uint32_t per = (n + 1023u) / 1024u, base = w * 64u * per;  // this wavefront's leaves
+    uint32_t       key[kPer];
+    uint16_t       val[kPer];
+    float          v[6] = {3.0e38f, 3.0e38f, 3.0e38f, -3.0e38f, -3.0e38f, -3.0e38f};
+    if (t < 2u) tcount[t] = 0u;
+    for (uint32_t i = 0; i < per; i++)
+    {
+        const uint32_t l = base + 64u * i + lane;
+        if (l >= min(n, cover)) continue;
+        f3 p0 = ld3(x, prims[(uint32_t)arity * l]), p1 = ld3(x, prims[(uint32_t)arity * l + 1]);
+        f3 blo = vmin(p0, p1), bhi = vmax(p0, p1);
+        if (arity == 3)
+        {
+            f3 p2 = ld3(x, prims[3 * l + 2]);
+            blo   = vmin(p0, vmin(p1, p2));
+            bhi   = vmax(p0, vmax(p1, p2));
+        }
+        v[0] = fminf(v[0], blo.x);
+        v[1] = fminf(v[1], blo.y);
+        v[2] = fminf(v[2], blo.z);
+        v[3] = fmaxf(v[3], bhi.x);
+        v[4] = fmaxf(v[4], bhi.y);
+        v[5] = fmaxf(v[5], bhi.z);
+    }
+    for (int k = 0; k < 3; k++) v[k] = wave_min(v[k]);
+    for (int k = 3; k < 6; k++) v[k] = wave_max(v[k]);
+    if (lane == 0)
+        for (int k = 0; k < 6; k++) sb[w][k] = v[k];
+    __syncthreads();
+    for (int ww = 0; ww < 16; ww++)
+        for (int k = 0; k < 6; k++) v[k] = k < 3 ? smin(v[k], sb[ww][k]) : smax(v[k], sb[ww][k]);
+    if (t < 6u)
+    {
+        float r = sb[0][t];
+        for (int ww = 1; ww < 16; ww++) r = t < 3u ? smin(r, sb[ww][t]) : smax(r, sb[ww][t]);
+        gbox[t] = f2ord(r);
+    }
+    const f3 lo = mk(v[0], v[1], v[2]), ext = vmax(mk(v[3], v[4], v[5]) - lo, mk(1e-6f, 1e-6f, 1e-6f));
+    const f3 inv = mk(1.0f / ext.x, 1.0f / ext.y, 1.0f / ext.z);
+#pragma unroll
+    for (int i = 0; i < kPer; i++)
+    {
+        const uint32_t l = base + 64u * (uint32_t)i + lane;
+        key[i]           = 0u;
+        val[i]           = (uint16_t)l;
+        if ((uint32_t)i < per && l < n)
+        {
+            f3 p0 = ld3(x, prims[(uint32_t)arity * l]), p1 = ld3(x, prims[(uint32_t)arity * l + 1]), cen = 0.5f * (p0 + p1);
+            if (arity == 3) cen = 0.333333f * ((p0 + p1) + ld3(x, prims[3 * l + 2]));
+            const f3 c = cen - lo;
+            key[i]     = morton32(mk(c.x * inv.x, c.y * inv.y, c.z * inv.z));
+        }
+    }
+    for (int shift = 0; shift < 32; shift += 8)
+    {
+        for (uint32_t d = lane; d < 256u; d += 64u) cnt[w][d] = 0u;
+        uint32_t off[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; i++)
+        {
+            off[i] = 0u;
+            if ((uint32_t)i >= per) continue;  // the same for the whole workgroup
+            const bool     valid = base + 64u * (uint32_t)i + lane < n;
+            const uint32_t d     = (key[i] >> shift) & 255u;
+            uint64_t       peers = __ballot(valid);
+            for (int b = 0; b < 8; b++)
+            {
+                const bool     bit = (d >> b) & 1u;
+                const uint64_t bal = __ballot(bit);
+                peers &= bit ? bal : ~bal;
+            }
+            const uint32_t rank = (uint32_t)__popcll(peers & lanemask_lt());
+            if (valid)
+            {
+                const uint32_t c = cnt[w][d];
+                off[i]           = c + rank;
+                __builtin_amdgcn_wave_barrier();
+                if (rank == 0u) cnt[w][d] = c + (uint32_t)__popcll(peers);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        // exclusive scan of the counts, digit by digit and wavefront by wavefront: four per thread
+        const uint32_t d = t >> 2, q = (t & 3u) * 4u;
+        uint32_t       c4[4], s = 0u;
+        for (int k = 0; k < 4; k++)
+        {
+            c4[k] = cnt[q + k][d];
+            s += c4[k];
+        }
+        uint32_t inc = s;
+        for (int o = 1; o < 64; o <<= 1)
+        {
+            const uint32_t u = __shfl_up(inc, o);
+            if ((int)lane >= o) inc += u;
+        }
+        if (lane == 63u) wsum[w] = inc;
+        __syncthreads();
+        uint32_t run = inc - s;
+        for (uint32_t ww = 0; ww < w; ww++) run += wsum[ww];
+        for (int k = 0; k < 4; k++)
+        {
+            cnt[q + k][d] = run;
+            run += c4[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kPer; i++)
+            if ((uint32_t)i < per && base + 64u * (uint32_t)i + lane < n)
+            {
+                const uint32_t pos = cnt[w][(key[i] >> shift) & 255u] + off[i];
+                skey[pos]          = key[i];
+                sval[pos]          = val[i];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kPer; i++)
+        {
+            const uint32_t l = base + 64u * (uint32_t)i + lane;
+            if ((uint32_t)i < per && l < n)
+            {
+                key[i] = skey[l];
+                val[i] = sval[l];
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; i++)
+    {
+        const uint32_t l = base + 64u * (uint32_t)i + lane;
+        if ((uint32_t)i < per && l < n)
+        {
+            const uint32_t o   = val[i];
+            sorted[l]          = o;
+            morton_sorted[l]   = ((uint64_t)key[i] << 32) | (uint64_t)o;
+            children[ni + l]   = make_uint2(o, o);
+            object_idx[ni + l] = o;
+            if (n == 1u) parent[ni + l] = kInvalid;
+        }
+    }
 }
 
 // ---------------------------------------------------------------- stable LSD radix sort
@@ -312,131 +481,67 @@ __global__ __launch_bounds__(kBlock) void k_karras(uint32_t ni_, const uint64_t*
     tleaf[gid]  = (uint32_t)(L + a);  // its first leaf in sorted order
 }
 
-// Treelet roots: inner nodes of at most kTreeletLeaves leaves whose parent has more (or is none).
+// Treelet roots: inner nodes of at most `limit` leaves whose parent has more (or is none), and the
+// inner nodes above them ("top"), both listed in any order, one atomic per wavefront. count[0]:
+// treelet roots, count[1]: top nodes (zero before the launch).
 __global__ __launch_bounds__(kBlock) void k_treelet_mark(uint32_t ni, const uint32_t* __restrict__ parent,
                                                           const uint32_t* __restrict__ tsize, uint32_t limit,
-                                                          uint32_t* count, uint32_t* __restrict__ troots)
+                                                          uint32_t* count, uint32_t* __restrict__ troots,
+                                                          uint32_t* __restrict__ top)
 {
-    // count[0]: treelet roots (listed in troots); count[1]: the inner nodes above the treelets
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= ni) return;
-    if (tsize[i] > limit)
+    const uint32_t i      = blockIdx.x * kBlock + threadIdx.x;
+    bool           is_top = false, is_root = false;
+    if (i < ni)
     {
-        atomicAdd(count + 1, 1u);
-        return;
+        is_top = tsize[i] > limit;
+        if (!is_top)
+        {
+            const uint32_t p = parent[i];
+            is_root          = p == kInvalid || tsize[p] > limit;
+        }
     }
-    const uint32_t p = parent[i];
-    if (p != kInvalid && tsize[p] <= limit) return;
-    troots[atomicAdd(count, 1u)] = i;
+    const uint32_t a = wave_append(count, is_root), b = wave_append(count + 1, is_top);
+    if (is_root) troots[a] = i;
+    if (is_top) top[b] = i;
 }
 
-// Inner nodes above the treelets, in the depth order of `order`: flags, then a scatter by the
-// exclusive scan of the flags, and per level the first position.
-__global__ __launch_bounds__(kBlock) void k_top_flags(uint32_t ni, const uint32_t* __restrict__ order,
-                                                       const uint32_t* __restrict__ tsize, uint32_t limit,
-                                                       uint32_t* __restrict__ flag)
+// The top nodes sorted by depth (their ancestors are top nodes; order within a level is free) with
+// the levels' offsets and every top node's place (top_idx), one workgroup. A depth is below 64: a
+// node's common prefix of the distinct 64-bit keys is longer than its parent's.
+constexpr uint32_t kMaxLevels = 64;
+__global__ __launch_bounds__(1024) void k_top_sort(const uint32_t* __restrict__ count, const uint32_t* __restrict__ parent,
+                                                    const uint32_t* __restrict__ top, uint32_t* __restrict__ depth,
+                                                    uint32_t* __restrict__ top_order, uint32_t* __restrict__ top_idx,
+                                                    uint32_t* __restrict__ level_ptr)
 {
-    uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k < ni) flag[k] = tsize[order[k]] > limit ? 1u : 0u;
-}
-__global__ __launch_bounds__(kBlock) void k_top_scatter(uint32_t ni, const uint32_t* __restrict__ order,
-                                                         const uint32_t* __restrict__ flag, const uint32_t* __restrict__ pos,
-                                                         uint32_t* __restrict__ top_order)
-{
-    uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k < ni && flag[k]) top_order[pos[k]] = order[k];
-}
-__global__ __launch_bounds__(kBlock) void k_top_levels(uint32_t nl, const uint32_t* __restrict__ level_ptr,
-                                                        const uint32_t* __restrict__ pos, uint32_t* __restrict__ top_level_ptr)
-{
-    uint32_t h = blockIdx.x * kBlock + threadIdx.x;
-    if (h < nl) top_level_ptr[h] = pos[level_ptr[h]];
-}
-
-// update_*_leave_aabb (lbvh.cpp:636-683) + refit (lbvh.cpp:702-754) in one pass, for trees taller
-// than the level-ordered refit handles: the second child to arrive at an inner node (atomic
-// ticket) computes its box; fences publish boxes across XCD L2s.
-__global__ __launch_bounds__(kBlock) void k_refit(uint32_t n, uint32_t ni, int arity, const uint32_t* __restrict__ prims,
-                                                   const uint32_t* __restrict__ sorted_to_orig,
-                                                   const float* __restrict__ x0, const float* __restrict__ x1,
-                                                   const float* __restrict__ pad, const uint32_t* __restrict__ parent,
-                                                   const uint2* __restrict__ children, NodeBox* nodes,
-                                                   float4* __restrict__ packed, uint32_t* counters, int sorted_keys)
-{
-    uint32_t l = blockIdx.x * kBlock + threadIdx.x;
-    if (l >= n) return;
-    uint32_t o = sorted_to_orig[l];
-    f3       lo, hi;
-    float    th;
-    if (arity == 3)
+    __shared__ uint32_t cnt[kMaxLevels], at[kMaxLevels];
+    const uint32_t      T = count[1];
+    if (threadIdx.x < kMaxLevels) cnt[threadIdx.x] = 0u;
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < T; k += 1024u)
     {
-        uint32_t a = prims[3 * o], b = prims[3 * o + 1], c = prims[3 * o + 2];
-        f3       s0 = ld3(x0, a), s1 = ld3(x0, b), s2 = ld3(x0, c);
-        f3       e0 = ld3(x1, a), e1 = ld3(x1, b), e2 = ld3(x1, c);
-        lo = vmin(vmin(s0, vmin(s1, s2)), vmin(e0, vmin(e1, e2)));
-        hi = vmax(vmax(s0, vmax(s1, s2)), vmax(e0, vmax(e1, e2)));
-        th = pad[a];
+        uint32_t d = 0u;
+        for (uint32_t q = parent[top[k]]; q != kInvalid && d < kMaxLevels - 1u; q = parent[q]) d++;
+        depth[k] = d;
+        atomicAdd(&cnt[d], 1u);
     }
-    else
+    __syncthreads();
+    if (threadIdx.x == 0)
     {
-        uint32_t a = prims[2 * o], b = prims[2 * o + 1];
-        f3       s0 = ld3(x0, a), s1 = ld3(x0, b), e0 = ld3(x1, a), e1 = ld3(x1, b);
-        lo = vmin(vmin(s0, s1), vmin(e0, e1));
-        hi = vmax(vmax(s0, s1), vmax(e0, e1));
-        th = pad[a];
+        uint32_t run = 0u;
+        for (uint32_t h = 0; h < kMaxLevels; h++)
+        {
+            level_ptr[h] = at[h] = run;
+            run += cnt[h];
+        }
+        level_ptr[kMaxLevels] = run;
     }
-    lo              = lo - mk(th, th, th);
-    hi              = hi + mk(th, th, th);
-    uint32_t cur    = ni + l;
-    NodeBox  box    = {make_float4(lo.x, lo.y, lo.z, 0.0f), make_float4(hi.x, hi.y, hi.z, 0.0f)};
-    nodes[cur]      = box;
-    // a tree of n leaves has depth < n; the bound only guards against a corrupted parent array
-    for (uint32_t depth = 0; depth < n; depth++)
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < T; k += 1024u)
     {
-        uint32_t p = parent[cur];
-        if (p == kInvalid || p >= ni) break;
-        __threadfence();
-        if (atomicAdd(&counters[p], 1u) == 0u) break;
-        __threadfence();
-        uint2   c = children[p];
-        NodeBox A = nodes[c.x], B = nodes[c.y];
-        NodeBox U;
-        U.lo     = make_float4(smin(A.lo.x, B.lo.x), smin(A.lo.y, B.lo.y), smin(A.lo.z, B.lo.z), 0.0f);
-        U.hi     = make_float4(smax(A.hi.x, B.hi.x), smax(A.hi.y, B.hi.y), smax(A.hi.z, B.hi.z), 0.0f);
-        nodes[p] = U;
-        // child codes (leaves keep (element, element) in children[]) and the largest element id
-        // under each child (an inner child's record was published before its ticket)
-        uint32_t ca, cb, ma, mb;
-        if (c.x >= ni)
-        {
-            ma = children[c.x].x;
-            ca = 0x80000000u | ma;
-            if (sorted_keys) ma = c.x - ni;
-        }
-        else
-        {
-            ca = c.x;
-            const float4* C = packed + 4 * (size_t)c.x;
-            ma              = max(__float_as_uint(C[1].w), __float_as_uint(C[3].w));
-        }
-        if (c.y >= ni)
-        {
-            mb = children[c.y].x;
-            cb = 0x80000000u | mb;
-            if (sorted_keys) mb = c.y - ni;
-        }
-        else
-        {
-            cb = c.y;
-            const float4* C = packed + 4 * (size_t)c.y;
-            mb              = max(__float_as_uint(C[1].w), __float_as_uint(C[3].w));
-        }
-        float4* P = packed + 4 * (size_t)p;
-        P[0] = make_float4(A.lo.x, A.lo.y, A.lo.z, __uint_as_float(ca));
-        P[1] = make_float4(A.hi.x, A.hi.y, A.hi.z, __uint_as_float(ma));
-        P[2] = make_float4(B.lo.x, B.lo.y, B.lo.z, __uint_as_float(cb));
-        P[3] = make_float4(B.hi.x, B.hi.y, B.hi.z, __uint_as_float(mb));
-        cur  = p;
+        const uint32_t pos = atomicAdd(&at[depth[k]], 1u), p = top[k];
+        top_order[pos] = p;
+        top_idx[p]     = pos;
     }
 }
 
@@ -446,97 +551,26 @@ __global__ void k_fill_u32(uint32_t* a, uint32_t n, uint32_t v)
     if (i < n) a[i] = v;
 }
 
-// ---------------------------------------------------------------- level-ordered refit
-// Cross-workgroup hand-off inside one kernel needs device-scope fences, which on a multi-XCD
-// part write back and invalidate L2. The refit therefore runs one launch per node depth, deepest
-// first: an inner node's children are one level deeper, so kernel boundaries order the levels.
-// Depths come from pointer jumping over the parent links (kDepthRounds launches, no atomics): after
-// round r each node holds its distance to its 2^r-th ancestor; depths of kMaxLevels or more land in
-// the overflow bin and keep the ticket refit. The top levels run in one workgroup.
-constexpr uint32_t kMaxLevels   = 256;
-constexpr int      kDepthRounds = 8;  // 2^8 = kMaxLevels
+// ---------------------------------------------------------------- refit
+// Cross-workgroup hand-off inside one kernel needs device-scope fences, which on a multi-XCD part
+// write back and invalidate L2. The refit therefore runs in steps ordered by kernel boundaries: the
+// leaf boxes, the treelets (one workgroup each, climbing in LDS) and the nodes above them.
 
-__global__ __launch_bounds__(kBlock) void k_depth_init(uint32_t ni, const uint32_t* __restrict__ parent,
-                                                        uint32_t* __restrict__ anc, uint32_t* __restrict__ dep)
-{
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= ni) return;
-    uint32_t p = parent[i];
-    anc[i]     = p;
-    dep[i]     = p == kInvalid ? 0u : 1u;
-}
-
-__global__ __launch_bounds__(kBlock) void k_depth_jump(uint32_t ni, const uint32_t* __restrict__ anc_in,
-                                                        const uint32_t* __restrict__ dep_in, uint32_t* __restrict__ anc_out,
-                                                        uint32_t* __restrict__ dep_out)
-{
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= ni) return;
-    uint32_t a = anc_in[i], d = dep_in[i];
-    if (a == kInvalid)
-    {
-        anc_out[i] = a;
-        dep_out[i] = d;
-        return;
-    }
-    anc_out[i] = anc_in[a];
-    dep_out[i] = min(d + dep_in[a], kMaxLevels);
-}
-
-// hist[h] for h < kMaxLevels; taller nodes are counted in hist[kMaxLevels]. Per-block LDS
-// histograms, one global atomic per non-empty bin and block.
-__global__ __launch_bounds__(kBlock) void k_level_hist(uint32_t ni, const uint32_t* __restrict__ height, uint32_t* hist)
-{
-    __shared__ uint32_t cnt[kMaxLevels + 1];
-    for (uint32_t b = threadIdx.x; b <= kMaxLevels; b += kBlock) cnt[b] = 0u;
-    __syncthreads();
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < ni) atomicAdd(&cnt[min(height[i], kMaxLevels)], 1u);
-    __syncthreads();
-    for (uint32_t b = threadIdx.x; b <= kMaxLevels; b += kBlock)
-        if (cnt[b]) atomicAdd(&hist[b], cnt[b]);
-}
-
-// order[level_ptr[h] ..] = inner nodes of height h (any order within a level)
-// top_idx of every top node; then, per top node, its children and which of them are top nodes
-__global__ __launch_bounds__(kBlock) void k_top_index(uint32_t ni, const uint32_t* __restrict__ top_order,
-                                                       const uint32_t* __restrict__ top_count, uint32_t* __restrict__ top_idx)
-{
-    uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k < ni && k < *top_count) top_idx[top_order[k]] = k;
-}
+// per top node: its children, and which of them are top nodes at which place
 __global__ __launch_bounds__(kBlock) void k_top_children(uint32_t ni, const uint32_t* __restrict__ top_order,
                                                           const uint32_t* __restrict__ top_count,
                                                           const uint2* __restrict__ children,
                                                           const uint32_t* __restrict__ tsize, uint32_t limit,
                                                           const uint32_t* __restrict__ top_idx, uint4* __restrict__ top_child)
 {
-    uint32_t k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= ni || k >= *top_count) return;
-    const uint2 c  = children[top_order[k]];
-    const bool  ta = c.x < ni && tsize[c.x] > limit, tb = c.y < ni && tsize[c.y] > limit;
-    top_child[k]   = make_uint4(c.x | (ta ? 0x80000000u : 0u), c.y | (tb ? 0x80000000u : 0u), ta ? top_idx[c.x] : 0u,
-                                tb ? top_idx[c.y] : 0u);
-}
-__global__ __launch_bounds__(kBlock) void k_level_scatter(uint32_t ni, const uint32_t* __restrict__ height,
-                                                           const uint32_t* __restrict__ level_ptr, uint32_t* cursor,
-                                                           uint32_t* __restrict__ order)
-{
-    __shared__ uint32_t cnt[kMaxLevels], base[kMaxLevels];
-    for (uint32_t b = threadIdx.x; b < kMaxLevels; b += kBlock) cnt[b] = 0u;
-    __syncthreads();
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    uint32_t h = 0, r = 0;
-    if (i < ni)
+    const uint32_t T = *top_count;
+    for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < T; k += gridDim.x * kBlock)
     {
-        h = height[i];
-        r = atomicAdd(&cnt[h], 1u);
+        const uint2 c  = children[top_order[k]];
+        const bool  ta = c.x < ni && tsize[c.x] > limit, tb = c.y < ni && tsize[c.y] > limit;
+        top_child[k]   = make_uint4(c.x | (ta ? 0x80000000u : 0u), c.y | (tb ? 0x80000000u : 0u), ta ? top_idx[c.x] : 0u,
+                                    tb ? top_idx[c.y] : 0u);
     }
-    __syncthreads();
-    for (uint32_t b = threadIdx.x; b < kMaxLevels; b += kBlock)
-        if (cnt[b]) base[b] = atomicAdd(&cursor[b], cnt[b]);
-    __syncthreads();
-    if (i < ni) order[level_ptr[h] + base[h] + r] = i;
 }
 
 // update_*_leave_aabb, lbvh.cpp:636-683: leaf box = AABB(x0 and x1 of the element) +- pad[v0]
@@ -812,129 +846,118 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
     }
 }
 
-// One treelet per workgroup: its inner nodes (a contiguous index range of at most
-// kTreeletLeaves - 1 nodes) level by level from its deepest, a barrier between levels; the
-// children of a node are one level deeper in the same treelet, or leaves of its leaf range. The
-// leaf boxes, leaf codes and the nodes' children are read once into LDS, and every box, key and
-// record a level needs comes from LDS, so a level costs a barrier, not a round trip to L2. The
-// results (node boxes, the binary and the four-wide records) are the ones inner_box writes.
-constexpr uint32_t kTreeletLeaves = 1024;
-constexpr int      kTreeletBlock  = 1024;
-__global__ __launch_bounds__(kTreeletBlock) void k_refit_treelets(const uint32_t* __restrict__ troots,
+// One treelet per workgroup: its inner nodes, a contiguous index range of at most kTreeletLeaves - 1
+// nodes, whose children lie in the treelet or are leaves of its leaf range. One thread per leaf
+// climbs: of a node's two children the one that arrives last (a ticket in LDS) forms its box and
+// goes on, so there is no barrier between levels, and everything the climb reads was put into LDS
+// before it. The node boxes and records are written after the climb, all nodes at once. The results
+// are the ones inner_box writes. (Level by level with the records written inside a level, every
+// level's barrier waited for stores: 57 us on average on the cloth tube's 385 and 688 treelets, now 29.)
+constexpr int kTreeletBlock = 1024;
+__global__ __launch_bounds__(kTreeletBlock) void k_refit_treelets(const uint32_t* __restrict__ count,
+                                                                   const uint32_t* __restrict__ troots,
                                                                    const uint32_t* __restrict__ tsize,
                                                                    const uint32_t* __restrict__ tfirst,
                                                                    const uint32_t* __restrict__ tleaf,
-                                                                   const uint32_t* __restrict__ depth, uint32_t ni,
+                                                                   const uint32_t* __restrict__ parent, uint32_t ni,
                                                                    const uint2* __restrict__ children, NodeBox* nodes,
                                                                    float4* packed, float4* packed4, int sorted_keys)
 {
-    constexpr int      kPer = (int)kTreeletLeaves / kTreeletBlock;
-    constexpr uint32_t kN   = kTreeletLeaves;
+    static_assert(kTreeletLeaves == kTreeletBlock, "one thread per leaf and per inner node");
+    constexpr uint32_t kN = kTreeletLeaves;
     __shared__ float    lb[6][kN], ib[6][kN];  // leaf and inner boxes (lo.xyz, hi.xyz)
-    __shared__ uint32_t lcode[kN], lkey[kN], ikey[kN], ich[2][kN];
-    __shared__ uint32_t hmax;
-    const uint32_t r = troots[blockIdx.x], first = tfirst[r], cnt = tsize[r] - 1u, leaf0 = tleaf[r], d0 = depth[r];
-    const uint32_t nl = cnt + 1u;
-    if (threadIdx.x == 0) hmax = 0u;
-    for (uint32_t l = threadIdx.x; l < nl; l += kTreeletBlock)
+    __shared__ uint32_t lcode[kN], lkey[kN], ikey[kN], ich[2][kN], ticket[kN];
+    __shared__ uint16_t up[kN];  // a node's parent in the treelet
+    const uint32_t      k = threadIdx.x, T = count[0];
+    for (uint32_t b = blockIdx.x; b < T; b += gridDim.x)
     {
-        const NodeBox B = nodes[ni + leaf0 + l];
-        lb[0][l] = B.lo.x;
-        lb[1][l] = B.lo.y;
-        lb[2][l] = B.lo.z;
-        lb[3][l] = B.hi.x;
-        lb[4][l] = B.hi.y;
-        lb[5][l] = B.hi.z;
-        const uint32_t el = children[ni + leaf0 + l].x;  // a leaf keeps (element, element)
-        lcode[l]          = 0x80000000u | el;
-        lkey[l]           = sorted_keys ? leaf0 + l : el;
-    }
-    uint32_t lv[kPer], mx = 0u;
-#pragma unroll
-    for (int j = 0; j < kPer; j++)
-    {
-        const uint32_t k = threadIdx.x + (uint32_t)j * kTreeletBlock;
-        lv[j]            = kInvalid;
+        const uint32_t r = troots[b], first = tfirst[r], cnt = tsize[r] - 1u, leaf0 = tleaf[r], nl = cnt + 1u;
+        uint32_t       node = kN;  // the leaf's parent in the treelet
+        if (k < nl)
+        {
+            const NodeBox  B  = nodes[ni + leaf0 + k];
+            const uint32_t el = children[ni + leaf0 + k].x;  // a leaf keeps (element, element)
+            node              = parent[ni + leaf0 + k] - first;
+            lb[0][k]          = B.lo.x;
+            lb[1][k]          = B.lo.y;
+            lb[2][k]          = B.lo.z;
+            lb[3][k]          = B.hi.x;
+            lb[4][k]          = B.hi.y;
+            lb[5][k]          = B.hi.z;
+            lcode[k]          = 0x80000000u | el;
+            lkey[k]           = sorted_keys ? leaf0 + k : el;
+        }
         if (k < cnt)
         {
-            const uint2    c = children[first + k];
-            const uint32_t d = depth[first + k];
-            ich[0][k]        = c.x;
-            ich[1][k]        = c.y;
-            lv[j]            = d >= d0 ? d - d0 : kInvalid;
-            if (lv[j] != kInvalid) mx = max(mx, lv[j]);
-        }
-    }
-    atomicMax(&hmax, mx);
-    __syncthreads();
-    // a child's box, code and key from LDS (c: node id, a leaf of the range or an inner node)
-    auto child = [&](uint32_t c, float* bx, uint32_t& code, uint32_t& key) {
-        if (c >= ni)
-        {
-            const uint32_t l = c - ni - leaf0;
-#pragma unroll
-            for (int t = 0; t < 6; t++) bx[t] = lb[t][l];
-            code = lcode[l];
-            key  = lkey[l];
-        }
-        else
-        {
-            const uint32_t l = c - first;
-#pragma unroll
-            for (int t = 0; t < 6; t++) bx[t] = ib[t][l];
-            code = c;
-            key  = ikey[l];
-        }
-    };
-    auto slot = [&](float4* Q, const float* bx, uint32_t code, uint32_t key) {
-        Q[0] = make_float4(bx[0], bx[1], bx[2], __uint_as_float(code));
-        Q[1] = make_float4(bx[3], bx[4], bx[5], __uint_as_float(key));
-    };
-    for (int h = (int)min(hmax, kMaxLevels); h >= 0; h--)
-    {
-#pragma unroll
-        for (int j = 0; j < kPer; j++)
-        {
-            if (lv[j] != (uint32_t)h) continue;
-            const uint32_t k = threadIdx.x + (uint32_t)j * kTreeletBlock, p = first + k;
-            float          A[6], B[6];
-            uint32_t       ca, cb, ma, mb;
-            child(ich[0][k], A, ca, ma);
-            child(ich[1][k], B, cb, mb);
-            const float U[6] = {smin(A[0], B[0]), smin(A[1], B[1]), smin(A[2], B[2]),
-                                smax(A[3], B[3]), smax(A[4], B[4]), smax(A[5], B[5])};
-#pragma unroll
-            for (int t = 0; t < 6; t++) ib[t][k] = U[t];
-            ikey[k]  = max(ma, mb);
-            nodes[p] = NodeBox{make_float4(U[0], U[1], U[2], 0.0f), make_float4(U[3], U[4], U[5], 0.0f)};
-            float4* P = packed + 4 * (size_t)p;
-            slot(P, A, ca, ma);
-            slot(P + 2, B, cb, mb);
-            // the four-wide record: the slots of both children's records (a leaf child: itself
-            // and an empty slot)
-            float4* Q = packed4 + 8 * (size_t)p;
-            for (int side = 0; side < 2; side++)
-            {
-                const uint32_t c  = ich[side][k];
-                float4*        QS = Q + 4 * side;
-                if (c >= ni)
-                {
-                    slot(QS, side == 0 ? A : B, side == 0 ? ca : cb, side == 0 ? ma : mb);
-                    empty_slot(QS + 2);
-                }
-                else
-                {
-                    const uint32_t l = c - first;
-                    float          G[6];
-                    uint32_t       cg, kg;
-                    child(ich[0][l], G, cg, kg);
-                    slot(QS, G, cg, kg);
-                    child(ich[1][l], G, cg, kg);
-                    slot(QS + 2, G, cg, kg);
-                }
-            }
+            const uint2 c = children[first + k];
+            ich[0][k]     = c.x;
+            ich[1][k]     = c.y;
+            up[k]         = (uint16_t)(first + k == r ? kN : parent[first + k] - first);
+            ticket[k]     = 0u;
         }
         __syncthreads();
+        // a child's box and key from LDS (c: node id, a leaf of the range or an inner node)
+        auto child = [&](uint32_t c, float* bx, uint32_t& key) {
+            const bool     leaf = c >= ni;
+            const uint32_t l    = leaf ? c - ni - leaf0 : c - first;
+#pragma unroll
+            for (int t = 0; t < 6; t++) bx[t] = leaf ? lb[t][l] : ib[t][l];
+            key = leaf ? lkey[l] : ikey[l];
+        };
+        // a treelet of cnt nodes is climbed in at most cnt steps
+        for (uint32_t step = 0; node < kN && step < cnt; step++)
+        {
+            if (atomicAdd(&ticket[node], 1u) == 0u) break;  // the sibling comes later
+            __threadfence_block();
+            float    A[6], B[6];
+            uint32_t ma, mb;
+            child(ich[0][node], A, ma);
+            child(ich[1][node], B, mb);
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+            {
+                ib[t][node]     = smin(A[t], B[t]);
+                ib[t + 3][node] = smax(A[t + 3], B[t + 3]);
+            }
+            ikey[node] = max(ma, mb);
+            __threadfence_block();
+            node = up[node];
+        }
+        __syncthreads();
+        // the records: lane by lane along memory (eight lanes per four-wide record, four per binary
+        // one, two per box), so a wavefront's store is one contiguous kilobyte; a thread per node
+        // wrote 14 times 64 separate lines
+        auto part = [&](uint32_t c, bool hi) {
+            const bool     leaf = c >= ni;
+            const uint32_t l    = leaf ? c - ni - leaf0 : c - first, t = hi ? 3u : 0u;
+            if (leaf) return make_float4(lb[t][l], lb[t + 1][l], lb[t + 2][l], __uint_as_float(hi ? lkey[l] : lcode[l]));
+            return make_float4(ib[t][l], ib[t + 1][l], ib[t + 2][l], __uint_as_float(hi ? ikey[l] : c));
+        };
+        float4* const Q = packed4 + 8 * (size_t)first;
+        for (uint32_t i = k; i < 8u * cnt; i += kN)
+        {
+            const uint32_t c = ich[(i >> 2) & 1u][i >> 3], sub = (i >> 1) & 1u;
+            const bool     hi = (i & 1u) != 0u;
+            float4         v;
+            if (c < ni) v = part(ich[sub][c - first], hi);
+            else if (sub == 0u) v = part(c, hi);
+            else
+            {
+                // a leaf child: itself and an empty slot
+                const float inf = __int_as_float(hi ? 0xff800000 : 0x7f800000);
+                v               = make_float4(inf, inf, inf, __uint_as_float(hi ? 0u : 0x80000000u));
+            }
+            Q[i] = v;
+        }
+        float4* const P = packed + 4 * (size_t)first;
+        for (uint32_t i = k; i < 4u * cnt; i += kN) P[i] = part(ich[(i >> 1) & 1u][i >> 2], (i & 1u) != 0u);
+        float4* const N = &nodes[first].lo;
+        for (uint32_t i = k; i < 2u * cnt; i += kN)
+        {
+            const uint32_t t = 3u * (i & 1u);
+            N[i]             = make_float4(ib[t][i >> 1], ib[t + 1][i >> 1], ib[t + 2][i >> 1], 0.0f);
+        }
+        __syncthreads();  // the next treelet's LDS
     }
 }
 
@@ -1439,7 +1462,7 @@ void Lbvh::init(int arity_, const uint32_t* device_prims, uint32_t n_leaves, con
     }
     uint32_t nb = (n + kSortTile - 1) / kSortTile;
     hist.alloc(256 * (size_t)nb + 1);
-    scan_tmp.alloc(scan_tmp_words(std::max(256 * nb, ni + 1)));
+    scan_tmp.alloc(scan_tmp_words(256 * nb));
     center.alloc(n);
     morton_sorted.alloc(n);
     parent.alloc(n_nodes());
@@ -1448,25 +1471,17 @@ void Lbvh::init(int arity_, const uint32_t* device_prims, uint32_t n_leaves, con
     nodes.alloc(n_nodes());
     packed.alloc(4 * (size_t)(ni ? ni : 1));
     packed4.alloc(8 * (size_t)(ni ? ni : 1));
-    counters.alloc(ni ? ni : 1);
-    height.alloc(ni ? ni : 1);
     tsize.alloc(ni ? ni : 1);
     tfirst.alloc(ni ? ni : 1);
     tleaf.alloc(ni ? ni : 1);
     troots.alloc(ni ? ni : 1);
     tcount.alloc(2);
-    top_flag.alloc(ni ? ni : 1);
-    top_pos.alloc((size_t)ni + 1);
+    top_list.alloc(ni ? ni : 1);
+    top_depth.alloc(ni ? ni : 1);
     top_order.alloc(ni ? ni : 1);
-    top_level_ptr.alloc(kMaxLevels + 2);
+    top_level_ptr.alloc(kMaxLevels + 1);
     top_idx.alloc(ni ? ni : 1);
     top_child.alloc(ni ? ni : 1);
-    anc[0].alloc(ni ? ni : 1);
-    anc[1].alloc(ni ? ni : 1);
-    order.alloc(ni ? ni : 1);
-    level_hist.alloc(kMaxLevels + 1);
-    level_ptr.alloc(kMaxLevels + 2);
-    level_cursor.alloc(kMaxLevels + 1);
     gbox.alloc(6 * (size_t)nseg);
     sorted_to_orig = vals[0].p;
     LCSX_HIP(hipStreamSynchronize(s0));
@@ -1487,6 +1502,18 @@ void Lbvh::construct(const float* x, const uint32_t* verts_per_seg, hipStream_t 
         tab[4 * g + 3] = cover_h[g];
     }
     seg_tab.upload(tab, s);
+    if (nseg == 1 && n <= kSmallLeaves)
+    {
+        sorted_to_orig = vals[0].p;
+        auto go        = [&](auto kern) {
+            kern<<<1, 1024, 0, s>>>(n, ni, arity, prims, x, cover_h[0], gbox.p, morton_sorted.p, sorted_to_orig, children.p,
+                                    object_idx.p, parent.p, tcount.p);
+        };
+        if (n <= 4096u) go(k_build_small<4>);
+        else go(k_build_small<8>);
+        finish(s);
+        return;
+    }
     k_init_gbox<<<grid_for(6 * nseg, kBlock), kBlock, 0, s>>>(gbox.p, nseg);
     k_leaf_centers<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, arity, prims, x, seg_of_leaf.p, seg_tab.p, center.p, gbox.p);
     k_morton<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, center.p, seg_of_leaf.p, gbox.p, keys[0].p, vals[0].p);
@@ -1516,93 +1543,77 @@ void Lbvh::construct(const float* x, const uint32_t* verts_per_seg, hipStream_t 
     sorted_to_orig = vals[cur].p;
     k_leaves<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, ni, keys[cur].p, vals[cur].p, seg_of_leaf.p, seg_tab.p,
                                                     morton_sorted.p, children.p, object_idx.p, parent.p);
-    if (ni) k_karras<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, morton_sorted.p, inner_seg.p, seg_tab.p, parent.p,
-                                                            children.p, object_idx.p, tsize.p, tfirst.p, tleaf.p);
-    LCSX_HIP(hipGetLastError());
-    use_levels = false;
-    if (ni == 0) return;
-    // node depths and the depth-sorted order of inner nodes (one host read of the histogram)
-    k_depth_init<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, parent.p, anc[0].p, height.p);
-    uint32_t* dep[2] = {height.p, counters.p};
-    for (int r = 0; r < kDepthRounds; r++)
-        k_depth_jump<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, anc[r & 1].p, dep[r & 1], anc[1 - (r & 1)].p,
-                                                             dep[1 - (r & 1)]);
-    depth = dep[kDepthRounds & 1];
-    k_fill_u32<<<grid_for(kMaxLevels + 1, kBlock), kBlock, 0, s>>>(level_hist.p, kMaxLevels + 1, 0u);
-    k_level_hist<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, depth, level_hist.p);
     k_fill_u32<<<1, kBlock, 0, s>>>(tcount.p, 2u, 0u);
-    k_treelet_mark<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, parent.p, tsize.p, kTreeletLeaves, tcount.p, troots.p);
-    std::vector<uint32_t> hist(kMaxLevels + 1);
-    uint32_t              nt[2] = {0u, 0u};
-    LCSX_HIP(hipMemcpyAsync(hist.data(), level_hist.p, hist.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    LCSX_HIP(hipMemcpyAsync(nt, tcount.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    LCSX_HIP(hipStreamSynchronize(s));
-    if (hist[kMaxLevels] != 0) return;  // deeper than kMaxLevels: keep the ticket refit
-    ntreelets = nt[0];
-    ntop      = nt[1];
-    level_ptr_h.assign(kMaxLevels + 2, 0u);
-    levels = 0;
-    for (uint32_t h = 0; h <= kMaxLevels; h++)
+    finish(s);
+}
+
+// From the sorted leaves (and tcount zeroed): the inner nodes, and the split into treelets and the
+// nodes above them. One tree of up to kUncounted leaves stays off the host: its treelets and top nodes
+// are counted on the device (about 2.5 and 1.5 per 1024 leaves on the cloth meshes, far from kTopLds).
+// Larger trees and batches read the two counts back, since a top beyond kTopLds is refit with one
+// launch per level.
+void Lbvh::finish(hipStream_t s)
+{
+    if (ni == 0)
     {
-        level_ptr_h[h + 1] = level_ptr_h[h] + hist[h];
-        if (hist[h]) levels = h;
+        LCSX_HIP(hipGetLastError());
+        return;
     }
-    LCSX_HIP(hipMemcpyAsync(level_ptr.p, level_ptr_h.data(), level_ptr_h.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    k_fill_u32<<<grid_for(kMaxLevels + 1, kBlock), kBlock, 0, s>>>(level_cursor.p, kMaxLevels + 1, 0u);
-    k_level_scatter<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, depth, level_ptr.p, level_cursor.p, order.p);
-    // the inner nodes above the treelets, in depth order, with their level offsets
-    k_top_flags<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, order.p, tsize.p, kTreeletLeaves, top_flag.p);
-    launch_scan_excl_u32(top_flag.p, top_pos.p, ni, scan_tmp.p, s);
-    k_top_scatter<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, order.p, top_flag.p, top_pos.p, top_order.p);
-    k_top_levels<<<grid_for(levels + 2, kBlock), kBlock, 0, s>>>(levels + 2, level_ptr.p, top_pos.p, top_level_ptr.p);
-    k_top_index<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, top_order.p, top_level_ptr.p + levels + 1, top_idx.p);
-    k_top_children<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, top_order.p, top_level_ptr.p + levels + 1, children.p,
-                                                            tsize.p, kTreeletLeaves, top_idx.p, top_child.p);
-    // a forest whose top exceeds k_refit_top's LDS table is refit one launch per level, from
-    // the level offsets read back here
-    top_lvp_h.clear();
-    if (ntop > kTopLds)
+    k_karras<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, morton_sorted.p, inner_seg.p, seg_tab.p, parent.p, children.p,
+                                                     object_idx.p, tsize.p, tfirst.p, tleaf.p);
+    k_treelet_mark<<<grid_for(ni, kBlock), kBlock, 0, s>>>(ni, parent.p, tsize.p, kTreeletLeaves, tcount.p, troots.p,
+                                                           top_list.p);
+    counted = !(nseg == 1 && n <= kUncounted);
+    ntop = ntreelets = 0;
+    if (counted)
     {
-        top_lvp_h.assign(levels + 2, 0u);
-        LCSX_HIP(hipMemcpyAsync(top_lvp_h.data(), top_level_ptr.p, (levels + 2) * sizeof(uint32_t),
-                                hipMemcpyDeviceToHost, s));
+        uint32_t nt[2] = {0u, 0u};
+        LCSX_HIP(hipMemcpyAsync(nt, tcount.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         LCSX_HIP(hipStreamSynchronize(s));
+        ntreelets = nt[0];
+        ntop      = nt[1];
+    }
+    top_lvp_h.clear();
+    if (n > kTreeletLeaves && (!counted || ntop))
+    {
+        k_top_sort<<<1, 1024, 0, s>>>(tcount.p, parent.p, top_list.p, top_depth.p, top_order.p, top_idx.p, top_level_ptr.p);
+        k_top_children<<<counted ? grid_for(ntop, kBlock) : 16u, kBlock, 0, s>>>(
+            ni, top_order.p, tcount.p + 1, children.p, tsize.p, kTreeletLeaves, top_idx.p, top_child.p);
+        if (ntop > kTopLds)
+        {
+            top_lvp_h.assign(kMaxLevels + 1, 0u);
+            LCSX_HIP(hipMemcpyAsync(top_lvp_h.data(), top_level_ptr.p, (kMaxLevels + 1) * sizeof(uint32_t),
+                                    hipMemcpyDeviceToHost, s));
+            LCSX_HIP(hipStreamSynchronize(s));
+        }
     }
     LCSX_HIP(hipGetLastError());
-    use_levels = true;
 }
 
 void Lbvh::refit(const float* x0, const float* x1, const float* pad, hipStream_t s)
 {
     if (n == 0) return;
-    if (use_levels || ni == 0)
-    {
-        k_refit_leaves<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, ni, arity, prims, sorted_to_orig, x0, x1, pad, nodes.p);
-        if (ni == 0) return;
-        if (ntreelets)
-            k_refit_treelets<<<ntreelets, kTreeletBlock, 0, s>>>(troots.p, tsize.p, tfirst.p, tleaf.p, depth, ni,
-                                                                 children.p, nodes.p, packed.p, packed4.p, sorted_keys);
-        // the nodes above the treelets (none when the root is a treelet's root)
-        if (ntop <= kTopLds || top_lvp_h.size() != levels + 2u)
-            k_refit_top<<<1, 1024, 0, s>>>(top_order.p, top_level_ptr.p, levels, ni, top_child.p, children.p, nodes.p,
-                                           packed.p, packed4.p, sorted_keys);
-        else
-            for (int h = (int)levels; h >= 0; h--)
-            {
-                const uint32_t b = top_lvp_h[h], e = top_lvp_h[h + 1];
-                if (e > b)
-                    k_refit_range<<<grid_for(e - b, kBlock), kBlock, 0, s>>>(top_order.p + b, e - b, ni, children.p,
-                                                                             nodes.p, packed.p, packed4.p, sorted_keys);
-            }
-        LCSX_HIP(hipGetLastError());
-        wide_ready = true;
-        return;
-    }
-    wide_ready = false;  // the ticket refit writes the binary records only
-    k_fill_u32<<<grid_for((uint32_t)counters.n, kBlock), kBlock, 0, s>>>(counters.p, (uint32_t)counters.n, 0u);
-    k_refit<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, ni, arity, prims, sorted_to_orig, x0, x1, pad, parent.p, children.p,
-                                                   nodes.p, packed.p, counters.p, sorted_keys);
+    k_refit_leaves<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, ni, arity, prims, sorted_to_orig, x0, x1, pad, nodes.p);
+    if (ni == 0) return;
+    // uncounted: about one workgroup per treelet, each taking every grid-th one
+    const uint32_t tgrid = counted ? ntreelets : n / 384u + 1u;
+    if (tgrid)
+        k_refit_treelets<<<tgrid, kTreeletBlock, 0, s>>>(tcount.p, troots.p, tsize.p, tfirst.p, tleaf.p, parent.p, ni,
+                                                         children.p, nodes.p, packed.p, packed4.p, sorted_keys);
+    // the nodes above the treelets (none up to kTreeletLeaves leaves)
+    if (n > kTreeletLeaves && (!counted || (ntop && ntop <= kTopLds)))
+        k_refit_top<<<1, 1024, 0, s>>>(top_order.p, top_level_ptr.p, kMaxLevels - 1u, ni, top_child.p, children.p, nodes.p,
+                                       packed.p, packed4.p, sorted_keys);
+    else if (ntop > kTopLds)
+        for (int h = (int)kMaxLevels - 1; h >= 0; h--)
+        {
+            const uint32_t b = top_lvp_h[h], e = top_lvp_h[h + 1];
+            if (e > b)
+                k_refit_range<<<grid_for(e - b, kBlock), kBlock, 0, s>>>(top_order.p + b, e - b, ni, children.p, nodes.p,
+                                                                         packed.p, packed4.p, sorted_keys);
+        }
     LCSX_HIP(hipGetLastError());
+    wide_ready = true;
 }
 
 uint32_t sort_hist_words(uint32_t n) { return 256u * ((n + kSortTile - 1) / kSortTile) + 1u; }
