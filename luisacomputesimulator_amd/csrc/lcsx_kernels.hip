@@ -1107,6 +1107,77 @@ __global__ __launch_bounds__(1024) void k_scan_apply(const uint32_t* in, uint32_
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = part[gridDim.x];
 }
 
+// The three steps for up to kScanPasses tiles in one workgroup: pass i covers values 4096 i .. of which
+// thread t holds four; every value is loaded before the first wait.
+constexpr uint32_t kScanPasses = 9;
+template <int kP>
+__global__ __launch_bounds__(1024) void k_scan_one(const uint32_t* in, uint32_t n, uint32_t* out)
+{
+    __shared__ uint32_t tot[kP * 16 + 1];
+    const uint32_t      t = threadIdx.x, w = t >> 6, lane = t & 63u;
+    uint32_t            x[kP][4], inc[kP];
+#pragma unroll
+    for (int i = 0; i < kP; i++)
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; k++)
+        {
+            const uint32_t at = (uint32_t)i * kScanTile + 4u * t + k;
+            x[i][k]           = at < n ? in[at] : 0u;
+        }
+#pragma unroll
+    for (int i = 0; i < kP; i++)
+    {
+        inc[i] = ((x[i][0] + x[i][1]) + x[i][2]) + x[i][3];
+        for (int o = 1; o < 64; o <<= 1)
+        {
+            const uint32_t u = __shfl_up(inc[i], o);
+            if ((int)lane >= o) inc[i] += u;
+        }
+        if (lane == 63u) tot[16 * i + w] = inc[i];
+    }
+    __syncthreads();
+    if (t < 64u)
+    {
+        // exclusive scan of the wavefronts' totals, kP / 4 consecutive ones per lane
+        constexpr int kPer = (kP * 16 + 63) / 64;
+        uint32_t      v[kPer], s = 0u;
+        for (int k = 0; k < kPer; k++)
+        {
+            const uint32_t at = kPer * t + (uint32_t)k;
+            v[k]              = at < kP * 16u ? tot[at] : 0u;
+            s += v[k];
+        }
+        uint32_t run = s;
+        for (int o = 1; o < 64; o <<= 1)
+        {
+            const uint32_t u = __shfl_up(run, o);
+            if ((int)lane >= o) run += u;
+        }
+        if (t == 63u) tot[kP * 16] = run;
+        run -= s;
+        for (int k = 0; k < kPer; k++)
+        {
+            const uint32_t at = kPer * t + (uint32_t)k;
+            if (at < kP * 16u) tot[at] = run;
+            run += v[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kP; i++)
+    {
+        uint32_t run = tot[16 * i + w] + inc[i] - (((x[i][0] + x[i][1]) + x[i][2]) + x[i][3]);
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; k++)
+        {
+            const uint32_t at = (uint32_t)i * kScanTile + 4u * t + k;
+            if (at < n) out[at] = run;
+            run += x[i][k];
+        }
+    }
+    if (t == 0) out[n] = tot[kP * 16];
+}
+
 __global__ __launch_bounds__(kB) void k_vc_fill(ContactView c, const uint32_t* __restrict__ ptr, uint32_t* __restrict__ cursor,
                                                  uint32_t* __restrict__ list, uint32_t* __restrict__ row)
 {
@@ -2464,9 +2535,15 @@ void launch_scan_excl_u32(const uint32_t* in, uint32_t* out, uint32_t n, uint32_
         k_fill_u32<<<1, kB, 0, s>>>(out, 1, 0u);
         return;
     }
-    k_scan_tiles<<<m, 1024, 0, s>>>(in, n, tmp);
-    k_scan_parts<<<1, 1024, 0, s>>>(tmp, m);
-    k_scan_apply<<<m, 1024, 0, s>>>(in, n, tmp, out);
+    if (m == 1) k_scan_one<1><<<1, 1024, 0, s>>>(in, n, out);
+    else if (m <= 4) k_scan_one<4><<<1, 1024, 0, s>>>(in, n, out);
+    else if (m <= kScanPasses) k_scan_one<kScanPasses><<<1, 1024, 0, s>>>(in, n, out);
+    else
+    {
+        k_scan_tiles<<<m, 1024, 0, s>>>(in, n, tmp);
+        k_scan_parts<<<1, 1024, 0, s>>>(tmp, m);
+        k_scan_apply<<<m, 1024, 0, s>>>(in, n, tmp, out);
+    }
 }
 void launch_fill_u32(uint32_t* a, uint32_t n, uint32_t v, hipStream_t s)
 {

@@ -15,8 +15,7 @@ namespace lcsx
 namespace
 {
 constexpr int kBlock     = 256;
-constexpr int kSortItems = 16;  // keys per thread per sort pass
-constexpr int kSortTile  = kBlock * kSortItems;
+constexpr int kSortItems = 16;  // most keys per thread and sort pass
 constexpr uint32_t kTreeletLeaves = 1024;    // most leaves of a treelet
 constexpr uint32_t kUncounted     = 200000;  // largest single tree whose top is not counted on the host
 
@@ -317,15 +316,22 @@ __global__ __launch_bounds__(1024) void k_build_small(uint32_t n, uint32_t ni, i
 }
 
 // ---------------------------------------------------------------- stable LSD radix sort
+// Keys per thread of a pass over n keys: a tile's rounds are serial, so few keys want small tiles
+// (187,088 leaves: 17 us a scatter with 16 keys per thread in 46 workgroups, 10 us with 8 in 92), as
+// long as one workgroup can still scan the tiles' counts.
+int sort_items(uint32_t n) { return n <= 65536u ? 4 : (n <= 294912u ? 8 : kSortItems); }
+
 // Histogram of the digit (dig >> shift) & 255 per tile.
+template <int kItems>
 __global__ __launch_bounds__(kBlock) void k_radix_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
                                                         uint32_t* __restrict__ hist, uint32_t nblocks)
 {
     __shared__ uint32_t h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    uint32_t base = blockIdx.x * kSortTile;
-    for (int i = 0; i < kSortItems; i++)
+    uint32_t base = blockIdx.x * (kBlock * kItems);
+#pragma unroll
+    for (int i = 0; i < kItems; i++)
     {
         uint32_t idx = base + i * kBlock + threadIdx.x;
         if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
@@ -336,6 +342,7 @@ __global__ __launch_bounds__(kBlock) void k_radix_hist(const uint32_t* __restric
 
 // Stable scatter by the digit of dig (kin, or the segment keys hin): kin, vin and, when present,
 // hin move together.
+template <int kItems>
 __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                            uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                            const uint32_t* __restrict__ hin, uint32_t* __restrict__ hout,
@@ -347,15 +354,23 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t* __rest
     __shared__ uint32_t s_cnt[4][256];
     const uint32_t      t = threadIdx.x, w = t >> 6, lane = t & 63;
     s_base[t]              = hist[t * nblocks + blockIdx.x];
-    const uint32_t base    = blockIdx.x * kSortTile;
-    for (int i = 0; i < kSortItems; i++)
+    const uint32_t base    = blockIdx.x * (kBlock * kItems);
+    uint32_t       key[kItems], dg[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; i++)
+    {
+        const uint32_t idx = base + i * kBlock + t;
+        key[i]             = idx < n ? kin[idx] : 0u;
+        dg[i]              = idx < n ? dig[idx] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < kItems; i++)
     {
         for (int k = 0; k < 4; k++) s_cnt[w][lane + 64 * k] = 0;
         __syncthreads();
         uint32_t idx   = base + i * kBlock + t;
         bool     valid = idx < n;
-        uint32_t key   = valid ? kin[idx] : 0u;
-        uint32_t d     = ((valid ? dig[idx] : 0u) >> shift) & 255u;
+        uint32_t d     = (dg[i] >> shift) & 255u;
         uint64_t peers = __ballot(valid);
         for (int b = 0; b < 8; b++)
         {
@@ -370,7 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t* __rest
         {
             uint32_t off = s_base[d] + rank;
             for (uint32_t ww = 0; ww < w; ww++) off += s_cnt[ww][d];
-            kout[off] = key;
+            kout[off] = key[i];
             vout[off] = vin[idx];
             if (hin) hout[off] = hin[idx];
         }
@@ -378,6 +393,22 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t* __rest
         s_base[t] += s_cnt[0][t] + s_cnt[1][t] + s_cnt[2][t] + s_cnt[3][t];
         __syncthreads();
     }
+}
+
+// One pass: the tiles' digit counts, their scan, the scatter.
+void sort_pass(uint32_t n, int shift, const uint32_t* dig, const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
+               uint32_t* vout, const uint32_t* hin, uint32_t* hout, uint32_t* hist, uint32_t* tmp, hipStream_t s)
+{
+    const int      items = sort_items(n);
+    const uint32_t nb    = (n + kBlock * items - 1) / (kBlock * items);
+    auto           go    = [&](auto hk, auto sk) {
+        hk<<<nb, kBlock, 0, s>>>(dig, n, shift, hist, nb);
+        launch_scan_excl_u32(hist, hist, 256 * nb, tmp, s);
+        sk<<<nb, kBlock, 0, s>>>(kin, vin, kout, vout, hin, hout, dig, n, shift, hist, nb);
+    };
+    if (items == 4) go(k_radix_hist<4>, k_radix_scatter<4>);
+    else if (items == 8) go(k_radix_hist<8>, k_radix_scatter<8>);
+    else go(k_radix_hist<kSortItems>, k_radix_scatter<kSortItems>);
 }
 
 // fn_apply_sorted, lbvh.cpp:525-539 (+ the 64-bit keys the build reads: Morton key and the leaf's
@@ -1460,9 +1491,8 @@ void Lbvh::init(int arity_, const uint32_t* device_prims, uint32_t n_leaves, con
         khi[0].alloc(n);
         khi[1].alloc(n);
     }
-    uint32_t nb = (n + kSortTile - 1) / kSortTile;
-    hist.alloc(256 * (size_t)nb + 1);
-    scan_tmp.alloc(scan_tmp_words(256 * nb));
+    hist.alloc(sort_hist_words(n));
+    scan_tmp.alloc(scan_tmp_words(sort_hist_words(n)));
     center.alloc(n);
     morton_sorted.alloc(n);
     parent.alloc(n_nodes());
@@ -1517,15 +1547,12 @@ void Lbvh::construct(const float* x, const uint32_t* verts_per_seg, hipStream_t 
     k_init_gbox<<<grid_for(6 * nseg, kBlock), kBlock, 0, s>>>(gbox.p, nseg);
     k_leaf_centers<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, arity, prims, x, seg_of_leaf.p, seg_tab.p, center.p, gbox.p);
     k_morton<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, center.p, seg_of_leaf.p, gbox.p, keys[0].p, vals[0].p);
-    uint32_t nb  = (n + kSortTile - 1) / kSortTile;
-    int      cur = 0;
+    int cur = 0;
     // four passes over the Morton key, then (several segments) passes over the segment id
     for (int shift = 0; shift < 32; shift += 8)
     {
-        k_radix_hist<<<nb, kBlock, 0, s>>>(keys[cur].p, n, shift, hist.p, nb);
-        launch_scan_excl_u32(hist.p, hist.p, 256 * nb, scan_tmp.p, s);
-        k_radix_scatter<<<nb, kBlock, 0, s>>>(keys[cur].p, vals[cur].p, keys[1 - cur].p, vals[1 - cur].p, nullptr,
-                                               nullptr, keys[cur].p, n, shift, hist.p, nb);
+        sort_pass(n, shift, keys[cur].p, keys[cur].p, vals[cur].p, keys[1 - cur].p, vals[1 - cur].p, nullptr, nullptr,
+                  hist.p, scan_tmp.p, s);
         cur = 1 - cur;
     }
     if (nseg > 1)
@@ -1533,10 +1560,8 @@ void Lbvh::construct(const float* x, const uint32_t* verts_per_seg, hipStream_t 
         k_seg_keys<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, vals[cur].p, seg_of_leaf.p, khi[cur].p);
         for (int shift = 0; shift < 32 && ((nseg - 1) >> shift) != 0u; shift += 8)
         {
-            k_radix_hist<<<nb, kBlock, 0, s>>>(khi[cur].p, n, shift, hist.p, nb);
-            launch_scan_excl_u32(hist.p, hist.p, 256 * nb, scan_tmp.p, s);
-            k_radix_scatter<<<nb, kBlock, 0, s>>>(keys[cur].p, vals[cur].p, keys[1 - cur].p, vals[1 - cur].p,
-                                                   khi[cur].p, khi[1 - cur].p, khi[cur].p, n, shift, hist.p, nb);
+            sort_pass(n, shift, khi[cur].p, keys[cur].p, vals[cur].p, keys[1 - cur].p, vals[1 - cur].p, khi[cur].p,
+                      khi[1 - cur].p, hist.p, scan_tmp.p, s);
             cur = 1 - cur;
         }
     }
@@ -1616,13 +1641,16 @@ void Lbvh::refit(const float* x0, const float* x1, const float* pad, hipStream_t
     wide_ready = true;
 }
 
-uint32_t sort_hist_words(uint32_t n) { return 256u * ((n + kSortTile - 1) / kSortTile) + 1u; }
+uint32_t sort_hist_words(uint32_t n)
+{
+    const uint32_t tile = (uint32_t)(kBlock * sort_items(n));
+    return 256u * ((n + tile - 1u) / tile) + 1u;
+}
 
 int launch_sort_key_pairs(uint32_t* lo[2], uint32_t* hi[2], uint32_t* val[2], uint32_t n, int lo_bits, int hi_bits,
                           uint32_t* hist, uint32_t* tmp, hipStream_t s)
 {
-    const uint32_t nb  = (n + kSortTile - 1) / kSortTile;
-    int            cur = 0;
+    int cur = 0;
     if (n == 0) return cur;
     // the low key's digits, then the high key's (stable passes: the result is ordered by (hi, lo))
     for (int pass = 0; pass < 2; pass++)
@@ -1631,10 +1659,7 @@ int launch_sort_key_pairs(uint32_t* lo[2], uint32_t* hi[2], uint32_t* val[2], ui
         for (int shift = 0; shift < bits; shift += 8)
         {
             const uint32_t* dig = pass == 0 ? lo[cur] : hi[cur];
-            k_radix_hist<<<nb, kBlock, 0, s>>>(dig, n, shift, hist, nb);
-            launch_scan_excl_u32(hist, hist, 256 * nb, tmp, s);
-            k_radix_scatter<<<nb, kBlock, 0, s>>>(lo[cur], val[cur], lo[1 - cur], val[1 - cur], hi[cur], hi[1 - cur], dig,
-                                                   n, shift, hist, nb);
+            sort_pass(n, shift, dig, lo[cur], val[cur], lo[1 - cur], val[1 - cur], hi[cur], hi[1 - cur], hist, tmp, s);
             cur = 1 - cur;
         }
     }
