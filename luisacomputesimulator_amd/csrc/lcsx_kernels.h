@@ -83,7 +83,8 @@ struct ContactView
     const uint32_t* count;
     uint32_t        capacity;
     // generalized DOFs, two entries per contact: up to 8 rows (~0u: unused) and their weights (a
-    // soft vertex with its weight, a rigid side as its body's 4 rows with weights sum w (1, X))
+    // soft vertex with its weight, a rigid side as its body's 4 rows with weights sum w (1, X));
+    // null without bodies: the contact's own vertices and weights
     const uint4*    gr;
     const float4*   gw;
 };

@@ -111,7 +111,21 @@ LCSX_D float reduce_prefetched(const float* __restrict__ part, const PrePartials
 #pragma unroll
     for (int u = 0; u < kPre; u++)
         if (threadIdx.x + (uint32_t)u * kB < p.n) v = v + p.v[u];
-    for (uint32_t i = threadIdx.x + kPre * kB; i < p.n; i += kB) v = v + part[i < p.n0 ? p.b0 + i : p.b1 + (i - p.n0)];
+    // the rest in batches, every load of a batch in flight (a long list of contact chunks)
+    constexpr uint32_t kIn = 12u;
+    for (uint32_t i = threadIdx.x + kPre * kB; i < p.n; i += kIn * kB)
+    {
+        float w[kIn];
+#pragma unroll
+        for (uint32_t u = 0; u < kIn; u++)
+        {
+            const uint32_t q = i + u * kB;
+            w[u]             = q < p.n ? part[q < p.n0 ? p.b0 + q : p.b1 + (q - p.n0)] : 0.0f;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kIn; u++)
+            if (i + u * kB < p.n) v = v + w[u];
+    }
     v = block_sum(v, sh);
     if (threadIdx.x == 0) bc = v;
     __syncthreads();
@@ -595,10 +609,25 @@ __global__ __launch_bounds__(kB) void k_rigid_positions(uint32_t n, const uint8_
 // ---------------------------------------------------------------- narrow phase
 // Contact record (the reference's CollisionPairTemplate, collision_data.h:48-127):
 // idx (type bit 31 in idx.z for VF, idx.w for EE), (n, k2), weights, (k1, area*kappa, bary0, bary1).
+// Appends the block's emitted contacts with one atomic on the shared counter (one per wavefront was
+// what the DCD waited for in contact: 474 us for 0.7M contacts, now 173). Called by all threads of
+// the block; `turn` alternates from call to call, so one call's LDS words outlive the next one's start.
 LCSX_D void push_contact(const ContactBuf& cb, bool emit, uint4 idx, f3 n, float k1, float k2, float ak, float b0,
-                         float b1, float4 w)
+                         float b1, float4 w, uint32_t turn)
 {
-    uint32_t slot = wave_append(cb.count, emit);
+    __shared__ uint32_t cnt[2][4], base[2];
+    const uint32_t      wv   = threadIdx.x >> 6, o = turn & 1u;
+    const uint64_t      mask = __ballot(emit);
+    if (lane_id() == 0) cnt[o][wv] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        const uint32_t tot = cnt[o][0] + cnt[o][1] + cnt[o][2] + cnt[o][3];
+        base[o]            = tot ? count_reserve(cb.count, tot) : 0u;
+    }
+    __syncthreads();
+    uint32_t slot = base[o] + (uint32_t)__popcll(mask & lanemask_lt());
+    for (uint32_t k = 0; k < wv; k++) slot += cnt[o][k];
     if (emit && slot < cb.capacity)
     {
         cb.idx[slot] = idx;
@@ -615,12 +644,15 @@ template <bool FP64>
 __global__ __launch_bounds__(kB) void k_dcd_vf(DcdArgs a)
 {
     uint32_t n = min(*a.pair_count, a.pair_capacity);
-    for (uint32_t p = blockIdx.x * kB + threadIdx.x; p < n; p += gridDim.x * kB)
+    uint32_t turn = 0u;
+    for (uint32_t first = blockIdx.x * kB; first < n; first += gridDim.x * kB, turn++)
     {
+        const bool     in = first + threadIdx.x < n;
+        const uint32_t p  = in ? first + threadIdx.x : n - 1u;
         uint32_t vid = a.pairs[2 * (size_t)p], fid = a.pairs[2 * (size_t)p + 1];
         uint32_t f0 = a.faces[3 * fid], f1 = a.faces[3 * fid + 1], f2 = a.faces[3 * fid + 2];
         // shared vertex, or both sides on one rigid body (narrow_phase.cpp:806-807)
-        bool     skip = (vid == f0 || vid == f1 || vid == f2) ||
+        bool     skip = !in || (vid == f0 || vid == f1 || vid == f2) ||
                     (a.vert_body && a.vert_body[vid] != kInvalid && a.vert_body[vid] == a.vert_body[f0]);
         bool     emit = false;
         uint4    idx  = make_uint4(vid, f0, f1 | 0x80000000u, f2);
@@ -669,7 +701,8 @@ __global__ __launch_bounds__(kB) void k_dcd_vf(DcdArgs a)
                 emit     = true;
             }
         }
-        push_contact(a.out, emit, idx, nrm, k1, k2, ak, b.x, b.y, make_float4(1.0f, -b.x, -b.y, (b.x + b.y) - 1.0f));
+        push_contact(a.out, emit, idx, nrm, k1, k2, ak, b.x, b.y, make_float4(1.0f, -b.x, -b.y, (b.x + b.y) - 1.0f),
+                     turn);
     }
 }
 
@@ -678,12 +711,15 @@ template <bool FP64>
 __global__ __launch_bounds__(kB) void k_dcd_ee(DcdArgs a)
 {
     uint32_t n = min(*a.pair_count, a.pair_capacity);
-    for (uint32_t p = blockIdx.x * kB + threadIdx.x; p < n; p += gridDim.x * kB)
+    uint32_t turn = 0u;
+    for (uint32_t first = blockIdx.x * kB; first < n; first += gridDim.x * kB, turn++)
     {
+        const bool     in = first + threadIdx.x < n;
+        const uint32_t p  = in ? first + threadIdx.x : n - 1u;
         uint32_t l = a.pairs[2 * (size_t)p], r = a.pairs[2 * (size_t)p + 1];
         uint32_t a0 = a.edges[2 * l], a1 = a.edges[2 * l + 1], b0 = a.edges[2 * r], b1 = a.edges[2 * r + 1];
         // shared vertex, or both edges on one rigid body (narrow_phase.cpp:972-974)
-        bool     skip = (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) ||
+        bool     skip = !in || (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) ||
                     (a.vert_body && a.vert_body[a0] != kInvalid && a.vert_body[a0] == a.vert_body[b0]);
         bool     emit = false;
         uint4    idx  = make_uint4(a0, a1, b0, b1 | 0x80000000u);
@@ -732,7 +768,7 @@ __global__ __launch_bounds__(kB) void k_dcd_ee(DcdArgs a)
             }
         }
         push_contact(a.out, emit, idx, nrm, k1, k2, ak, c.v[0], c.v[2],
-                     make_float4(c.v[0], 1.0f - c.v[0], -c.v[2], c.v[2] - 1.0f));
+                     make_float4(c.v[0], 1.0f - c.v[0], -c.v[2], c.v[2] - 1.0f), turn);
     }
 }
 
@@ -912,17 +948,35 @@ __global__ __launch_bounds__(kB) void k_contact_lift(ContactView c, const uint32
     }
 }
 
+// Entries [4 half, 4 half + 4) of contact k's generalized DOFs. Without bodies (gr null) they are the
+// contact's own four vertices and weights.
+LCSX_D void gdofs4(const ContactView& c, uint32_t k, uint32_t half, uint32_t r[4], float w[4])
+{
+    uint4  a = make_uint4(kInvalid, kInvalid, kInvalid, kInvalid);
+    float4 u = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (c.gr)
+    {
+        a = c.gr[2 * (size_t)k + half];
+        u = c.gw[2 * (size_t)k + half];
+    }
+    else if (half == 0u)
+    {
+        a = c.idx[k];
+        u = c.w[k];
+        a = make_uint4(a.x & 0x7fffffffu, a.y & 0x7fffffffu, a.z & 0x7fffffffu, a.w & 0x7fffffffu);
+    }
+    r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+    w[0] = u.x; w[1] = u.y; w[2] = u.z; w[3] = u.w;
+}
 LCSX_D void gdofs(const ContactView& c, uint32_t k, uint32_t r[8], float w[8])
 {
-    uint4  a = c.gr[2 * (size_t)k], b = c.gr[2 * (size_t)k + 1];
-    float4 u = c.gw[2 * (size_t)k], v = c.gw[2 * (size_t)k + 1];
-    r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w; r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
-    w[0] = u.x; w[1] = u.y; w[2] = u.z; w[3] = u.w; w[4] = v.x; w[5] = v.y; w[6] = v.z; w[7] = v.w;
+    gdofs4(c, k, 0u, r, w);
+    gdofs4(c, k, 1u, r + 4, w + 4);
 }
 LCSX_D float gweight(const ContactView& c, uint32_t k, uint32_t j)
 {
-    float4 u = c.gw[2 * (size_t)k + (j >> 2)];
-    uint32_t l = j & 3u;
+    const float4   u = c.gr ? c.gw[2 * (size_t)k + (j >> 2)] : c.w[k];
+    const uint32_t l = j & 3u;
     return l == 0 ? u.x : (l == 1 ? u.y : (l == 2 ? u.z : u.w));
 }
 
@@ -1198,38 +1252,55 @@ __global__ __launch_bounds__(kB) void k_vc_fill(ContactView c, const uint32_t* _
     }
 }
 
-// Each row's slots in a fixed order: by the contact's vertex ids (with the type bit), then the
-// entry. The narrow phase appends contacts with atomics, so contact ids differ from run to run;
+// Each row's slots in a fixed order: by the contact's vertex ids (with the type bit; a contact names
+// a row once). The narrow phase appends contacts with atomics, so contact ids differ from run to run;
 // ordering the slots by content makes every per-row sum (contact gradient and Hessian, the SpMV's
 // contact runs) add its terms in the same order in every run, so a state and its contact set give
-// the same rounding. A slot's place is its rank among its row's slots (one thread per slot, m
-// compares for a row of m slots, so a collider vertex with hundreds of slots costs no more than a
-// few hundred loads per thread); the keys are unique within a row.
-LCSX_D bool slot_less(uint4 ia, uint32_t a, uint4 ib, uint32_t b)
-{
-    if (ia.x != ib.x) return ia.x < ib.x;
-    if (ia.y != ib.y) return ia.y < ib.y;
-    if (ia.z != ib.z) return ia.z < ib.z;
-    if (ia.w != ib.w) return ia.w < ib.w;
-    return (a & 7u) < (b & 7u);
-}
+// the same rounding. A slot's place is its rank among its row's slots, whose keys are unique. One
+// thread per slot walks a short row by itself; the slots of a longer one (a collider vertex has
+// hundreds) are compared by their wavefront together, 64 of the row's keys at a time from registers
+// (2.8M slots: 678 us when every thread walked its row, now 316).
 __global__ __launch_bounds__(kB) void k_vc_rank(ContactView c, const uint32_t* __restrict__ ptr,
                                                  const uint32_t* __restrict__ row, const uint32_t* __restrict__ total,
                                                  const uint32_t* __restrict__ list, uint32_t* __restrict__ out)
 {
-    const uint32_t n = *total;
-    for (uint32_t e = blockIdx.x * kB + threadIdx.x; e < n; e += gridDim.x * kB)
+    constexpr uint32_t kShort = 32u;
+    const uint32_t     n = *total, lane = lane_id();
+    for (uint32_t e0 = blockIdx.x * kB + (threadIdx.x & ~63u); e0 < n; e0 += gridDim.x * kB)
     {
-        const uint32_t v = row[e], b = ptr[v], m = ptr[v + 1] - b;
-        const uint32_t x = list[e];
+        const bool     on = e0 + lane < n;
+        const uint32_t e  = on ? e0 + lane : n - 1u;
+        const uint32_t v = row[e], b = ptr[v], m = ptr[v + 1] - b, x = list[e];
         const uint4    kx = c.idx[x >> 3];
-        uint32_t       rank = 0;
-        for (uint32_t t = 0; t < m; t++)
+        const uint64_t hx = ((uint64_t)kx.x << 32) | kx.y, lx = ((uint64_t)kx.z << 32) | kx.w;
+        auto less = [&](uint64_t hy, uint64_t ly) { return (hy < hx) | ((hy == hx) & (ly < lx)); };
+        uint32_t rank = 0u;
+        if (on && m <= kShort)
+            for (uint32_t t = 0; t < m; t++)
+            {
+                const uint4 ky = c.idx[list[b + t] >> 3];
+                rank += less(((uint64_t)ky.x << 32) | ky.y, ((uint64_t)ky.z << 32) | ky.w) ? 1u : 0u;
+            }
+        for (uint64_t todo = __ballot(on && m > kShort); todo != 0ull;)
         {
-            const uint32_t y = list[b + t];
-            rank += slot_less(c.idx[y >> 3], y, kx, x) ? 1u : 0u;
+            const int      lead = __ffsll((unsigned long long)todo) - 1;
+            const uint32_t rb = (uint32_t)__builtin_amdgcn_readlane((int)b, lead);
+            const uint32_t rm = (uint32_t)__builtin_amdgcn_readlane((int)m, lead);
+            const bool     mine = on && b == rb;  // rows with slots start at different places
+            for (uint32_t u0 = 0; u0 < rm; u0 += 64u)
+            {
+                const uint4 ky = u0 + lane < rm ? c.idx[list[rb + u0 + lane] >> 3] : make_uint4(0u, 0u, 0u, 0u);
+                const uint32_t cnt = min(64u, rm - u0);
+                for (uint32_t s = 0; s < cnt; s++)
+                {
+                    auto rl = [&](uint32_t q) { return (uint32_t)__builtin_amdgcn_readlane((int)q, (int)s); };
+                    const uint64_t hy = ((uint64_t)rl(ky.x) << 32) | rl(ky.y), ly = ((uint64_t)rl(ky.z) << 32) | rl(ky.w);
+                    rank += (mine & less(hy, ly)) ? 1u : 0u;
+                }
+            }
+            todo &= ~__ballot(mine);
         }
-        out[b + rank] = x;
+        if (on) out[b + rank] = x;
     }
 }
 
@@ -1238,30 +1309,41 @@ __global__ __launch_bounds__(kB) void k_vc_rank(ContactView c, const uint32_t* _
 __global__ __launch_bounds__(kB) void k_contact_assemble(ContactView c, VertContacts vc, float* __restrict__ cgB,
                                                           float* __restrict__ diag, uint32_t nv)
 {
-    uint32_t i = blockIdx.x * kB + threadIdx.x;
-    if (i >= nv) return;
-    uint32_t e0 = vc.ptr[i], e1 = vc.ptr[i + 1];
-    if (e0 == e1) return;
-    f3    g = mk(0.0f, 0.0f, 0.0f);
-    float D[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++) D[k] = 0.0f;
-    for (uint32_t e = e0; e < e1; e++)
+    // One wavefront per row: 64 slots' twelve terms (gradient 3, block 9) at a time into LDS, lane by
+    // lane one slot, then added in slot order, twelve lanes one entry each. (A thread per row was a chain
+    // of as many round trips as the row has slots: 543 us with 2.8M slots, now 91.)
+    __shared__ float term[kB / 64][12][64 + 1];
+    const uint32_t   lane = lane_id(), w = threadIdx.x >> 6, waves = gridDim.x * (kB / 64u);
+    for (uint32_t i = blockIdx.x * (kB / 64u) + w; i < nv; i += waves)
     {
-        uint32_t ent = vc.list[e], k = ent >> 3, j = ent & 7u;
-        float4   nk = c.nk[k], ax = c.aux[k];
-        float    wj     = gweight(c, k, j);
-        float    nv3[3] = {nk.x, nk.y, nk.z};
-        g               = g + (ax.x * wj) * mk(nk.x, nk.y, nk.z);
-        float s         = (nk.w * wj) * wj;
+        const uint32_t e0 = vc.ptr[i], e1 = vc.ptr[i + 1];
+        if (e0 == e1) continue;
+        float sum = 0.0f;
+        for (uint32_t e = e0; e < e1; e += 64u)
+        {
+            const uint32_t cnt = min(64u, e1 - e);
+            if (lane < cnt)
+            {
+                const uint32_t ent = vc.list[e + lane], k = ent >> 3;
+                const float4   nk  = c.nk[k];
+                const float    ax = c.aux[k].x, wj = gweight(c, k, ent & 7u), gs = ax * wj, s = (nk.w * wj) * wj;
+                const float    n3[3] = {nk.x, nk.y, nk.z};
 #pragma unroll
-        for (int r = 0; r < 3; r++)
+                for (int r = 0; r < 3; r++)
+                {
+                    term[w][r][lane] = gs * n3[r];
 #pragma unroll
-            for (int cc = 0; cc < 3; cc++) D[3 * r + cc] = D[3 * r + cc] + s * (nv3[r] * nv3[cc]);
+                    for (int cc = 0; cc < 3; cc++) term[w][3 + 3 * r + cc][lane] = s * (n3[r] * n3[cc]);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (lane < 12u)
+                for (uint32_t q = 0; q < cnt; q++) sum = sum + term[w][lane][q];
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (lane < 3u) cgB[3 * (size_t)i + lane] = cgB[3 * (size_t)i + lane] + sum;
+        else if (lane < 12u) diag[(lane - 3u) * (size_t)nv + i] = diag[(lane - 3u) * (size_t)nv + i] + sum;
     }
-    st3(cgB, i, ld3(cgB, i) + g);
-#pragma unroll
-    for (int k = 0; k < 9; k++) diag[k * (size_t)nv + i] = diag[k * (size_t)nv + i] + D[k];
 }
 
 // Per-slot coefficient a = k2 w_j n (the contact's id in .w), in list order. With the contact
@@ -1307,16 +1389,27 @@ __global__ __launch_bounds__(1024) void k_chunk_table(SegView g, const uint32_t*
     uint32_t run = part[t] - sum;
     for (uint32_t sc = b; sc < e; sc++)
     {
-        uint32_t c0 = run, k = nch(sc), s0 = ptr[g.sc_v0[sc]];
-        sc_cb0[sc]  = c0;
-        for (uint32_t c = 0; c < k; c++)
-        {
-            cb_scene[c0 + c] = sc;
-            cb_slot0[c0 + c] = s0 + 256u * c;
-        }
-        run += k;
+        sc_cb0[sc] = run;
+        run += nch(sc);
     }
-    if (t == 1023u) sc_cb0[S] = part[1023];
+    const uint32_t total = part[1023];
+    if (t == 1023u) sc_cb0[S] = total;
+    __threadfence_block();
+    __syncthreads();
+    // the chunks, all threads over all scenes' (a scene's chunks by one thread: 430 us for one scene
+    // with 11,000)
+    for (uint32_t c = t; c < total; c += 1024u)
+    {
+        uint32_t lo = 0u, hi = S - 1u;  // the last scene whose first chunk is not after c
+        while (lo < hi)
+        {
+            const uint32_t m = (lo + hi + 1u) / 2u;
+            if (sc_cb0[m] <= c) lo = m;
+            else hi = m - 1u;
+        }
+        cb_scene[c] = lo;
+        cb_slot0[c] = ptr[g.sc_v0[lo]] + 256u * (c - sc_cb0[lo]);
+    }
 }
 
 // t_c = sum_j w_j n.p_j over the contact's generalized DOFs, with p given by pfun.
@@ -1325,10 +1418,17 @@ LCSX_D float contact_t1(const ContactView& c, uint32_t k, PF pfun)
 {
     uint32_t r[8];
     float    w[8];
-    gdofs(c, k, r, w);
+    gdofs4(c, k, 0u, r, w);
     float4 nk = c.nk[k];
     f3     nn = mk(nk.x, nk.y, nk.z);
-    float  t  = w[0] * dot(nn, pfun(r[0]));
+    if (!c.gr)
+    {
+        // four vertices: their rows are requested together
+        const f3 p0 = pfun(r[0]), p1 = pfun(r[1]), p2 = pfun(r[2]), p3 = pfun(r[3]);
+        return ((w[0] * dot(nn, p0) + w[1] * dot(nn, p1)) + w[2] * dot(nn, p2)) + w[3] * dot(nn, p3);
+    }
+    gdofs4(c, k, 1u, r + 4, w + 4);
+    float t = w[0] * dot(nn, pfun(r[0]));
     for (int j = 1; j < 8; j++)
         if (r[j] != kInvalid) t = t + w[j] * dot(nn, pfun(r[j]));
     return t;
@@ -2253,13 +2353,13 @@ struct GridContacts
                 f3             sum, pr = mk(0.0f, 0.0f, 0.0f);
                 const uint32_t b = 256u * ch + (threadIdx.x & 192u);
                 auto           tf = [&](uint32_t k) {
-                    const uint4  ga = c.gr[2 * (size_t)k], gb = c.gr[2 * (size_t)k + 1];
-                    const float4 wa = c.gw[2 * (size_t)k], wb = c.gw[2 * (size_t)k + 1];
-                    const float4 nk = c.nk[k];
-                    const f3     nn = mk(nk.x, nk.y, nk.z);
+                    const float4   nk  = c.nk[k];
+                    const f3       nn  = mk(nk.x, nk.y, nk.z);
                     const uint32_t own = vc.row[b + lane_id()];
-                    const uint32_t ra[4] = {ga.x, ga.y, ga.z, ga.w}, rb[4] = {gb.x, gb.y, gb.z, gb.w};
-                    const float    fa[4] = {wa.x, wa.y, wa.z, wa.w}, fb[4] = {wb.x, wb.y, wb.z, wb.w};
+                    uint32_t       ra[4], rb[4];
+                    float          fa[4], fb[4];
+                    gdofs4(c, k, 0u, ra, fa);
+                    gdofs4(c, k, 1u, rb, fb);
                     const P4       A = rows4(a, zx, first, zep, p_old, beta, ra, bad);
                     float          t = fa[0] * dot(nn, A.p[0]);
 #pragma unroll
@@ -2647,7 +2747,7 @@ uint32_t launch_contact_triplets(const ContactView& c, uint32_t n_contacts, unsi
 void launch_contact_assemble(const ContactView& c, const VertContacts& vc, float* cgB, float* diag, uint32_t nv,
                              hipStream_t s)
 {
-    k_contact_assemble<<<grid_for(nv, kB), kB, 0, s>>>(c, vc, cgB, diag, nv);
+    k_contact_assemble<<<std::min(8192u, grid_for(nv, kB / 64u)), kB, 0, s>>>(c, vc, cgB, diag, nv);
 }
 void launch_pcg_init(const PcgArgs& a, hipStream_t s) { k_pcg_init<<<a.seg.n_rb, kB, 0, s>>>(a); }
 void launch_pcg_dir(const PcgArgs& a, const ContactView& c, const VertContacts& vc, unsigned max_chunks,

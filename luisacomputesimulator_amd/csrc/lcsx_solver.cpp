@@ -152,8 +152,11 @@ void Solver::alloc_collision(uint32_t vf, uint32_t ee, uint32_t nc)
     ccd_pairs_fresh = false;
     ccd_rest_ee.alloc(cap_ee);
     vc_list.alloc(slots_per_contact * (size_t)cap_c);
-    c_gr.alloc(2 * (size_t)cap_c);
-    c_gw.alloc(2 * (size_t)cap_c);
+    if (!S.bodies.empty())
+    {
+        c_gr.alloc(2 * (size_t)cap_c);
+        c_gw.alloc(2 * (size_t)cap_c);
+    }
     // per-block partial sums of the SpMV: row blocks + scene-aligned slot chunks (4 slots per contact)
     const size_t chunks = max_chunks(slots_per_contact * cap_c) + 1;
     part_pq.alloc(4 * (size_t)S.n_rb + chunks);  // four per row block (the SpMV's 64-row blocks), one per chunk
@@ -552,7 +555,7 @@ void Solver::dcd(bool from_ccd_pairs)
     a.fp64   = prm.precision >= 1;
     a.quadratic = prm.contact_energy_type == 0;
     a.out    = out;
-    a.vert_body = vert_body_d.p;
+    a.vert_body = S.bodies.empty() ? nullptr : vert_body_d.p;
     a.pairs = pairs_vf.p;
     a.pair_count = from_ccd_pairs ? &status.p->n_vf_ccd : &status.p->n_vf;
     a.pair_capacity = cap_vf;
@@ -565,8 +568,8 @@ void Solver::dcd(bool from_ccd_pairs)
     a.area_a = edge_area.p;
     a.area_b = edge_area.p;
     launch_dcd(a, 1, pair_grid(cap_ee), stream);
-    launch_contact_lift(contact_view(), pair_grid(cap_c), S.bodies.empty() ? nullptr : vert_body_d.p, bodies_d.p,
-                        body_X_d.p, c_gr.p, c_gw.p, stream);
+    if (!S.bodies.empty())
+        launch_contact_lift(contact_view(), pair_grid(cap_c), vert_body_d.p, bodies_d.p, body_X_d.p, c_gr.p, c_gw.p, stream);
     toc("dcd");
 }
 
@@ -888,8 +891,8 @@ void Solver::ccd_pass(int kind, bool rest, hipStream_t s)
     c.edges         = edges.p;
     c.offset        = offset.p;
     c.sst           = sst.p;
-    c.vert_scene    = vert_scene_d.p;
-    c.vert_body     = vert_body_d.p;
+    c.vert_scene    = S.nscenes > 1 ? vert_scene_d.p : nullptr;
+    c.vert_body     = S.bodies.empty() ? nullptr : vert_body_d.p;
     c.fp64          = prm.precision >= 1;
     c.budget        = ccd_budget;
     c.rest          = rest ? 1 : 0;
