@@ -416,28 +416,27 @@ void launch_pcg_spmv(const PcgArgs& a, const SellView& A, const VertContacts& vc
 void launch_pcg_update(const PcgArgs& a, hipStream_t s);
 
 // The PCG in one launch (lcsx_pcg_grid.h): limits, shape and workspace.
-constexpr uint32_t kGridRows  = 4096;  // rows whose p a workgroup holds: its own and those its columns name
-constexpr uint32_t kGridOwn   = 512;   // own rows of a workgroup
-constexpr uint32_t kGridVals  = 8192;  // partial sums of one kind
-constexpr uint32_t kGridWgs   = 256;   // workgroups: one per CU
+constexpr uint32_t kGridRows    = 4096;  // rows whose p a workgroup holds: its own and those its columns name
+constexpr uint32_t kGridOwn     = 512;   // own rows of a workgroup
+constexpr uint32_t kGridWgs     = 256;   // workgroups of a launch: one per CU
 constexpr uint32_t kGridThreads = 512;
-constexpr size_t   kGridWords = 2 * (size_t)kGridVals;  // 8-byte words posted by the workgroups
 struct GridSync
 {
-    unsigned long long* slots;  // kGridWords, zero before the first launch
-    unsigned long long* zx;     // 3 words per row, zero before the first launch: z as it is exchanged
-    uint32_t            epoch;  // of the launch's first iteration (from 2); later launches use later ones
+    unsigned long long* rz;    // words, zero before the first launch: one per row block,
+    unsigned long long* pq;    // four per row block and one per contact-slot chunk,
+    unsigned long long* zx;    // and three per row: z as it is exchanged
+    const uint2*        tab;   // per workgroup: its scene and its place in it (null: one scene)
+    uint32_t            epoch; // of the launch's first iteration (from 2); later launches use later ones
 };
 struct GridPlan
 {
-    unsigned wgs = 0;       // 0: the launches are used
-    int      U = 0, K = 0;  // row groups per thread and blocks per thread and row
+    int U = 0, K = 0;  // row groups per thread and blocks per thread and row (0: the launches are used)
+    uint32_t row_blocks() const { return (uint32_t)U * kGridThreads / 1024u; }  // of a workgroup
 };
-// The shape for n_rb row blocks of at most `width` blocks a row, with at most `chunks` contact-slot
-// chunks.
-GridPlan grid_plan(uint32_t n_rb, uint32_t width, uint32_t chunks);
-// Iterations [a.k, a.k + len) of a solve begun by launch_pcg_init (k_bsr_init), one scene.
-void launch_pcg_grid(const GridPlan& p, const PcgArgs& a, const SellView& A, const ContactView& c,
+// The shape for scenes of up to n_rb_most row blocks, n_rb in all, of at most `width` blocks a row.
+GridPlan grid_plan(uint32_t n_rb_most, uint32_t n_rb, uint32_t width);
+// Iterations [a.k, a.k + len) of a solve begun by launch_pcg_init, on `wgs` workgroups.
+void launch_pcg_grid(const GridPlan& p, unsigned wgs, const PcgArgs& a, const SellView& A, const ContactView& c,
                      const VertContacts& vc, const GridSync& g, uint32_t len, hipStream_t s);
 void launch_grid_clear(unsigned long long* words, size_t n, hipStream_t s);
 // One such launch runs at a time per GPU in a process (its workgroups wait for each other, so all

@@ -2279,13 +2279,17 @@ struct GridContacts
 {
     ContactView  c;
     VertContacts vc;
-    uint32_t     n = 0, nch = 0, end = 0;
-    LCSX_D void  begin(const PcgArgs& a)
+    uint32_t     c0 = 0, nch = 0, s0 = 0, end = 0, part = 0, parts = 1;  // the scene's chunks and slots
+    LCSX_D void  begin(const PcgArgs& a, uint32_t scene, uint32_t part_, uint32_t parts_)
     {
-        n   = min(*c.count, c.capacity);
-        nch = a.seg.sc_cb0[1];
-        end = vc.ptr[a.n];
+        c0    = a.seg.nscenes == 1u ? 0u : a.seg.sc_cb0[scene];
+        nch   = a.seg.sc_cb0[scene + 1] - c0;
+        s0    = vc.ptr[a.seg.nscenes == 1u ? 0u : a.seg.sc_v0[scene]];
+        end   = vc.ptr[a.seg.nscenes == 1u ? a.n : a.seg.sc_v0[scene + 1]];
+        part  = part_;
+        parts = parts_;
     }
+    LCSX_D uint32_t first() const { return c0; }
     LCSX_D uint32_t chunks() const { return nch; }
     // p = z + beta p_old of four rows at once (kInvalid: none), every load in flight before the first is
     // used
@@ -2343,7 +2347,7 @@ struct GridContacts
                       grid::Word* words, uint32_t epoch, float* sh, uint32_t& bad) const
     {
         const uint32_t gpw = blockDim.x >> 8, grp = threadIdx.x >> 8, wv = threadIdx.x >> 6;
-        for (uint32_t base = blockIdx.x * gpw; base < nch; base += gridDim.x * gpw)
+        for (uint32_t base = part * gpw; base < nch; base += parts * gpw)
         {
             const uint32_t ch  = base + grp;
             float          loc = 0.0f;
@@ -2351,7 +2355,7 @@ struct GridContacts
             {
                 uint32_t       row;
                 f3             sum, pr = mk(0.0f, 0.0f, 0.0f);
-                const uint32_t b = 256u * ch + (threadIdx.x & 192u);
+                const uint32_t b = s0 + 256u * ch + (threadIdx.x & 192u);
                 auto           tf = [&](uint32_t k) {
                     const float4   nk  = c.nk[k];
                     const f3       nn  = mk(nk.x, nk.y, nk.z);
@@ -2391,21 +2395,21 @@ struct GridContacts
             grid::stores_done();  // the runs' sums, before the word that announces them
             __syncthreads();
             if ((threadIdx.x & 255u) == 0u && ch < nch)
-                grid::post(words + ch, ((sh[wv] + sh[wv + 1]) + sh[wv + 2]) + sh[wv + 3], epoch);
+                grid::post(words + c0 + ch, ((sh[wv] + sh[wv + 1]) + sh[wv + 2]) + sh[wv + 3], epoch);
             __syncthreads();
         }
     }
     LCSX_D void poison(grid::Word* words) const
     {
         const uint32_t gpw = blockDim.x >> 8;
-        for (uint32_t base = blockIdx.x * gpw; base < nch; base += gridDim.x * gpw)
-            for (uint32_t ch = base; ch < min(base + gpw, nch); ch++) grid::post(words + ch, 0.0f, grid::kPoison);
+        for (uint32_t base = part * gpw; base < nch; base += parts * gpw)
+            for (uint32_t ch = base; ch < min(base + gpw, nch); ch++) grid::post(words + c0 + ch, 0.0f, grid::kPoison);
     }
     LCSX_D f3 fold(f3 q, uint32_t i) const
     {
         return fold_runs_of(
             q, [&](uint32_t e) { return grid::ld_row(reinterpret_cast<const float*>(vc.runsum), e); }, vc.ptr, i,
-            vc.ptr[0]);
+            s0);
     }
 };
 __global__ void k_grid_clear(unsigned long long* w, size_t n)
@@ -2814,28 +2818,25 @@ void launch_grid_clear(unsigned long long* w, size_t n, hipStream_t s)
 {
     if (n) k_grid_clear<<<std::min(1024u, grid_for(n, kB)), kB, 0, s>>>(w, n);
 }
-// One workgroup per row block up to 256 of them (one per CU), two row blocks each up to 512: a wait for
-// more workgroups costs more than the second block's product. Blocks per thread and row (K, four
-// threads a row) are what fits 256 registers beside the rows' vectors. Contact slots: at most two
-// chunks per 256 threads; each costs an iteration about 4 us, the launches' whole contact part 5-10 us.
-GridPlan grid_plan(uint32_t n_rb, uint32_t width, uint32_t chunks)
+// A workgroup takes one row block (256 rows) while one launch holds them all, otherwise two: a wait for
+// more workgroups costs more than the second block's product, and a batch needs half the launches.
+// Blocks per thread and row (K, four threads a row) are what fits 256 registers beside the rows'
+// vectors.
+GridPlan grid_plan(uint32_t n_rb_most, uint32_t n_rb, uint32_t width)
 {
-    GridPlan p;
-    const int      K = width <= 12u ? 3 : (width <= 16u ? 4 : (width <= 32u ? 8 : 0));
-    const int      U = n_rb <= kGridWgs ? 2 : 4;
-    const uint32_t G = U == 2 ? n_rb : (n_rb + 1u) / 2u;
-    if (K == 0 || n_rb == 0 || G > kGridWgs || (U == 4 && K > 3)) return p;
-    if (chunks > 2u * G * (kGridThreads / 256u) || 4u * n_rb + chunks > kGridVals) return p;
-    p.wgs = G;
-    p.U   = U;
-    p.K   = K;
+    GridPlan  p;
+    const int K = width <= 12u ? 3 : (width <= 16u ? 4 : (width <= 32u ? 8 : 0));
+    const int U = n_rb <= kGridWgs || K > 3 ? 2 : 4;
+    if (K == 0 || n_rb == 0 || n_rb_most > kGridWgs * (uint32_t)(U / 2)) return p;
+    p.U = U;
+    p.K = K;
     return p;
 }
 template <class Mat, class Ct, bool CT>
-static void grid_go(const GridPlan& p, const PcgArgs& a, const Mat& A, const Ct& ct, const GridSync& g, uint32_t len,
+static void grid_go(const GridPlan& p, unsigned wgs, const PcgArgs& a, const Mat& A, const Ct& ct, const GridSync& g, uint32_t len,
                     hipStream_t s)
 {
-    auto go = [&](auto kern) { kern<<<p.wgs, kGridThreads, 0, s>>>(a, A, ct, g, len); };
+    auto go = [&](auto kern) { kern<<<wgs, kGridThreads, 0, s>>>(a, A, ct, g, len); };
     if (p.U == 4) go(k_pcg_grid<Mat, 4, 3, CT, Ct>);
     else if (p.K == 3) go(k_pcg_grid<Mat, 2, 3, CT, Ct>);
     else if (p.K == 4) go(k_pcg_grid<Mat, 2, 4, CT, Ct>);
@@ -2843,7 +2844,7 @@ static void grid_go(const GridPlan& p, const PcgArgs& a, const Mat& A, const Ct&
     LCSX_HIP(hipGetLastError());
 }
 template <int LP>
-static void grid_lp(const GridPlan& p, const PcgArgs& a, const SellView& A, const ContactView& c,
+static void grid_lp(const GridPlan& p, unsigned wgs, const PcgArgs& a, const SellView& A, const ContactView& c,
                     const VertContacts& vc, const GridSync& g, uint32_t len, hipStream_t s)
 {
     const GridSell<LP> M{A, a.n};
@@ -2852,17 +2853,17 @@ static void grid_lp(const GridPlan& p, const PcgArgs& a, const SellView& A, cons
         GridContacts ct;
         ct.c  = c;
         ct.vc = vc;
-        grid_go<GridSell<LP>, GridContacts, true>(p, a, M, ct, g, len, s);
+        grid_go<GridSell<LP>, GridContacts, true>(p, wgs, a, M, ct, g, len, s);
     }
     else
-        grid_go<GridSell<LP>, NoContacts, false>(p, a, M, NoContacts{}, g, len, s);
+        grid_go<GridSell<LP>, NoContacts, false>(p, wgs, a, M, NoContacts{}, g, len, s);
 }
-void launch_pcg_grid(const GridPlan& p, const PcgArgs& a, const SellView& A, const ContactView& c,
+void launch_pcg_grid(const GridPlan& p, unsigned wgs, const PcgArgs& a, const SellView& A, const ContactView& c,
                      const VertContacts& vc, const GridSync& g, uint32_t len, hipStream_t s)
 {
-    if (A.val_p && A.bf16) grid_lp<2>(p, a, A, c, vc, g, len, s);
-    else if (A.val_p) grid_lp<1>(p, a, A, c, vc, g, len, s);
-    else grid_lp<0>(p, a, A, c, vc, g, len, s);
+    if (A.val_p && A.bf16) grid_lp<2>(p, wgs, a, A, c, vc, g, len, s);
+    else if (A.val_p) grid_lp<1>(p, wgs, a, A, c, vc, g, len, s);
+    else grid_lp<0>(p, wgs, a, A, c, vc, g, len, s);
 }
 namespace
 {

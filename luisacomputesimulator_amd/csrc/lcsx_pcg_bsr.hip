@@ -46,12 +46,12 @@ struct BsrWork
     float*    part_rz;
     float*    part_pq;  // four per row block: one per product block of 64 rows
     BsrState* st;
-    unsigned long long* words;  // of the one-launch form: kGridWords, then z's (3 per row); cleared by the init
+    unsigned long long* words;  // of the one-launch form (GridSync: rz, pq, zx); cleared by the init
     uint32_t            n_words;
 };
 
 constexpr uint32_t kGridBsrRows = 2 * kGridWgs * 256;  // most rows of the one-launch form
-constexpr uint32_t grid_words(uint32_t n) { return n <= kGridBsrRows ? (uint32_t)kGridWords + 3u * n : 0u; }
+constexpr uint32_t grid_words(uint32_t n) { return n <= kGridBsrRows ? 5u * ((n + kB - 1) / kB) + 3u * n : 0u; }
 
 constexpr uint32_t align_up(uint32_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
@@ -525,8 +525,7 @@ GridPlan bsr_plan(const lcsx_bsr* A, uint32_t nb)
 {
     const double mean = (double)A->nnz / A->n_rows;
     if (A->n_rows > (int)kGridBsrRows) return GridPlan{};
-    return grid_plan(nb, nb > kGridWgs ? (mean <= 12.0 ? 12u : 64u) : (mean <= 12.0 ? 16u : (mean <= 24.0 ? 32u : 64u)),
-                     0u);
+    return grid_plan(nb, nb, nb > kGridWgs ? (mean <= 12.0 ? 12u : 64u) : (mean <= 12.0 ? 16u : (mean <= 24.0 ? 32u : 64u)));
 }
 void launch_bsr_grid(const GridPlan& p, const lcsx_bsr* A, const BsrWork& w, const lcsx_pcg_options& o, float* x,
                      hipStream_t s)
@@ -547,8 +546,9 @@ void launch_bsr_grid(const GridPlan& p, const lcsx_bsr* A, const BsrWork& w, con
     a.abs_tol     = o.abs_tol;
     a.check_every = (uint32_t)o.check_every;
     const GridBsr  M{A->row_ptr, A->col, A->blocks, A->diag, w.st, (uint32_t)A->nnz};
-    const GridSync g{w.words, w.words + kGridWords, 2u};
-    auto go = [&](auto kern) { kern<<<p.wgs, kGridThreads, 0, s>>>(a, M, NoContacts{}, g, (uint32_t)o.max_iters); };
+    const GridSync g{w.words, w.words + w.nb, w.words + 5u * w.nb, nullptr, 2u};
+    const unsigned wgs = (w.nb + p.row_blocks() - 1u) / p.row_blocks();
+    auto go = [&](auto kern) { kern<<<wgs, kGridThreads, 0, s>>>(a, M, NoContacts{}, g, (uint32_t)o.max_iters); };
     if (p.U == 4) go(k_pcg_grid<GridBsr, 4, 3, false, NoContacts>);
     else if (p.K <= 4) go(k_pcg_grid<GridBsr, 2, 4, false, NoContacts>);
     else go(k_pcg_grid<GridBsr, 2, 8, false, NoContacts>);
@@ -567,7 +567,7 @@ lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_op
     {
         int dev = 0;
         gp      = bsr_plan(A, w.nb);
-        if (gp.wgs && (hipGetDevice(&dev) != hipSuccess || !lease.take(dev))) gp = GridPlan{};
+        if (gp.U && (hipGetDevice(&dev) != hipSuccess || !lease.take(dev))) gp = GridPlan{};
     }
     k_bsr_init<<<w.nb, kB, 0, s>>>(w, A->diag, b, x);
     LCSX_HIP(hipGetLastError());
@@ -575,9 +575,9 @@ lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_op
     int      issued = 0;
     while (issued < o.max_iters)
     {
-        const int chunk = gp.wgs ? o.max_iters : std::min(std::max(o.check_every, 8), o.max_iters - issued);
-        if (gp.wgs) launch_bsr_grid(gp, A, w, o, x, s);
-        for (int k = issued; !gp.wgs && k < issued + chunk; k++)
+        const int chunk = gp.U ? o.max_iters : std::min(std::max(o.check_every, 8), o.max_iters - issued);
+        if (gp.U) launch_bsr_grid(gp, A, w, o, x, s);
+        for (int k = issued; !gp.U && k < issued + chunk; k++)
         {
             k_bsr_dir<<<w.nb, kB, 0, s>>>(w, (uint32_t)k, (uint32_t)o.check_every, o.abs_tol, rel2);
             k_bsr_spmv<<<4 * w.nb, kProdB, 0, s>>>(w, (uint32_t)k, A->row_ptr, A->col, A->blocks, A->diag, (uint32_t)A->nnz);
@@ -587,7 +587,7 @@ lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_op
         issued += chunk;
         LCSX_HIP(hipMemcpyAsync(&h, w.st, sizeof(BsrState), hipMemcpyDeviceToHost, s));
         LCSX_HIP(hipStreamSynchronize(s));
-        if (gp.wgs && h.fail && !h.bad_index) return solve(A, b, x, o, s, base, res, false);
+        if (gp.U && h.fail && !h.bad_index) return solve(A, b, x, o, s, base, res, false);
         if (h.converged || h.bad_index) break;
     }
     if (h.bad_index) return arg_error("a block column or row range is outside the matrix");

@@ -6,7 +6,8 @@
 // the gaps between them. Here a workgroup owns one or two 256-row blocks. It reads their blocks,
 // vectors and preconditioner once, finds the rows outside its own that its blocks' columns name (a
 // hash table in LDS), and holds p of all of them in LDS, so the product reads registers and LDS only.
-// An iteration waits twice: for every 64-row chunk's p.q partial, and for every row block's r.z partial
+// A scene of a batch is solved by its own workgroups, which wait only for each other; a batch that needs
+// more workgroups than CUs takes several launches. An iteration waits twice: for every 64-row chunk's p.q partial, and for every row block's r.z partial
 // together with the z of the named rows. A partial is posted as one 8-byte word (value, epoch), and so
 // is every entry of z: the word that carries a value also says that it is there, so nothing has to be
 // ordered between the stores. Every workgroup adds the partials up itself.
@@ -108,13 +109,15 @@ LCSX_D f3 wait_z(const Word* zx, uint32_t n, uint32_t i, uint32_t epoch, uint32_
     }
 }
 
-// Waits for words [0, n) of `epoch` and adds them up as the launched kernels do: strided over the
-// first 256 threads, a butterfly per wavefront (the four wavefronts' sums go to red). Called by the
-// first four wavefronts. L.bad is set when a word was poisoned or the wait ran out.
+// Waits for words [0, n0) of s0, then [0, n1) of s1, of `epoch` and adds them up as the launched
+// kernels do: strided over the first 256 threads, a butterfly per wavefront (the four wavefronts' sums
+// go to red). Called by the first four wavefronts. L.bad is set when a word was poisoned or the wait ran
+// out.
 template <int kIn>  // words in flight per thread
-LCSX_D void wait_sum(const Word* s, uint32_t n, uint32_t epoch, Lds& L, float* red)
+LCSX_D void wait_sum(const Word* s0, uint32_t n0, const Word* s1, uint32_t n1, uint32_t epoch, Lds& L, float* red)
 {
-    float v = 0.0f;
+    const uint32_t n = n0 + n1;
+    float          v = 0.0f;
     for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 256u * kIn)
     {
         uint32_t tries = 0;
@@ -123,7 +126,10 @@ LCSX_D void wait_sum(const Word* s, uint32_t n, uint32_t epoch, Lds& L, float* r
             Word w[kIn];
 #pragma unroll
             for (int u = 0; u < kIn; u++)
-                w[u] = i0 + 256u * u < n ? peek(s + i0 + 256u * u) : (Word)epoch << 32;
+            {
+                const uint32_t i = i0 + 256u * u;
+                w[u]             = i < n ? peek(i < n0 ? s0 + i : s1 + (i - n0)) : (Word)epoch << 32;
+            }
             bool ok = true, gone = ++tries > kPolls || *(volatile uint32_t*)&L.bad != 0u;
 #pragma unroll
             for (int u = 0; u < kIn; u++)
@@ -191,12 +197,20 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
     constexpr uint32_t M = U * gpw, R = 64u * M;          // chunks and rows of a workgroup
     static_assert(M % 4u == 0u && M <= T / 64u && R <= kGridOwn, "whole row blocks, one wavefront per chunk");
     const uint32_t t = threadIdx.x, lane = lane_id(), wv = t >> 6, j = lane >> 4, n = a.n;
-    const uint32_t n_rb = a.seg.n_rb, b0 = blockIdx.x * (M / 4u), nb = min(M / 4u, n_rb - b0), nc = 4u * nb;
-    const uint32_t own0 = blockIdx.x * R;
-    PcgState*      st = a.s;
-    if (st->converged) return;  // set by an earlier launch: every workgroup reads the same
-    Word* const S_pq = g.slots;
-    Word* const S_rz = S_pq + kGridVals;
+    // this workgroup's scene, its place in it, the scene's rows [.., end) and row blocks [rb0, rb0 + nrb)
+    const bool     one   = g.tab == nullptr;
+    const uint2    me    = one ? make_uint2(0u, blockIdx.x) : g.tab[blockIdx.x];
+    const uint32_t scene = me.x, part = me.y;
+    const uint32_t rb0 = one ? 0u : a.seg.sc_rb0[scene], nrb = (one ? a.seg.n_rb : a.seg.sc_rb0[scene + 1]) - rb0;
+    const uint32_t own0 = (one ? 0u : a.seg.sc_v0[scene]) + part * R, end = one ? n : a.seg.sc_v0[scene + 1];
+    const uint32_t b0 = rb0 + part * (M / 4u), nb = min(M / 4u, rb0 + nrb - b0), nc = 4u * nb;
+    const uint32_t parts = (nrb + M / 4u - 1u) / (M / 4u);
+    PcgState*      st = a.s + scene;
+    if (st->converged) return;  // set by an earlier launch: every workgroup of the scene reads the same
+    Word* const S_pq = g.pq + 4u * rb0;  // the scene's words
+    Word* const S_rz = g.rz + rb0;
+    Word* const S_ch = g.pq + 4u * a.seg.n_rb;
+    const float* const rz_part = a.part_rz + rb0;
     // ---- this thread's blocks, and the rows outside its own that they name
     typename Mat::Raw W[U][K];
     uint32_t          ci[U][K];
@@ -213,7 +227,7 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
     {
         const uint32_t lc = (uint32_t)u * gpw + (wv >> 2);
         const uint32_t i  = own0 + 64u * lc + 16u * (wv & 3u) + (lane & 15u);
-        const bool     in = lc < nc && i < n;
+        const bool     in = lc < nc && i < end;
         typename Mat::Row r{};
         if (in)
         {
@@ -270,7 +284,7 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
     __syncthreads();
     // ---- this thread's row (the first nc wavefronts: one chunk each) and p of all named rows
     const uint32_t row = own0 + t;
-    const bool     rv  = wv < nc && row < n;
+    const bool     rv  = wv < nc && row < end;
     m3             D{}, Mi{};
     f3             xr{}, r{}, z{}, p{};
     if (rv && ok)
@@ -289,7 +303,7 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
     if (t < 256u)
     {
         float v = 0.0f;
-        for (uint32_t b = t; b < n_rb; b += 256u) v = v + a.part_rz[b];
+        for (uint32_t b = t; b < nrb; b += 256u) v = v + rz_part[b];
         v = wave_sum(v);
         if (lane == 0) L.red[0][wv] = v;
     }
@@ -301,7 +315,7 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
     float*   p_cur = a.p_old;
     float*   p_nxt = a.p_new;
     bool     stop  = false;
-    ct.begin(a);
+    ct.begin(a, scene, part, parts);
     for (uint32_t e = t; e < nhalo; e += T)
     {
         const f3 ze = ld3(a.z, L.halo[e]);
@@ -312,7 +326,7 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
         const uint32_t ep    = g.epoch + it;
         const bool     check = (k % a.check_every) == 0u;
         stop                 = !(rz == rz) || (check && (rz < a.abs_tol || rz <= a.rel2 * rz0));
-        if (blockIdx.x == 0 && t == 0)
+        if (part == 0u && t == 0)
         {
             st->rz[k & 1u] = rz;
             if (k == 0u) st->rz0 = rz;
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
         {
             const uint32_t lc = (uint32_t)u * gpw + (wv >> 2);
             const uint32_t lr = 64u * lc + 16u * (wv & 3u) + (lane & 15u);
-            const bool     in = lc < nc && own0 + lr < n;
+            const bool     in = lc < nc && own0 + lr < end;
             f3             y  = mk(0.0f, 0.0f, 0.0f);
             if (in && j == 0u) y = ld3(L.q, lr);
 #pragma unroll
@@ -373,13 +387,13 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
             if (lane == 0) L.sh[u][wv] = loc;
         }
         __syncthreads();
-        if (t < nc) post(S_pq + 4u * b0 + t, sum4(&L.sh[t / gpw][4u * (t % gpw)]), ep);
+        if (t < nc) post(S_pq + 4u * (b0 - rb0) + t, sum4(&L.sh[t / gpw][4u * (t % gpw)]), ep);
         if (CT)
         {
-            ct.slots(a, g.zx, it == 0u, ep - 1u, p_cur, beta, S_pq + 4u * n_rb, ep, L.cs, L.bad_tc);
+            ct.slots(a, g.zx, it == 0u, ep - 1u, p_cur, beta, S_ch, ep, L.cs, L.bad_tc);
             __syncthreads();
         }
-        if (t < 256u) wait_sum<4 * U / 2>(S_pq, 4u * n_rb + ct.chunks(), ep, L, L.red[1]);
+        if (t < 256u) wait_sum<4 * U / 2>(S_pq, 4u * nrb, S_ch + ct.first(), ct.chunks(), ep, L, L.red[1]);
         __syncthreads();
         ok = (L.bad | L.bad_tc) == 0u;
         if (!ok) break;
@@ -401,9 +415,9 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
         loc = wave_sum(loc);
         if (lane == 0) L.cs[wv] = loc;
         __syncthreads();
-        if (t < nb) post(S_rz + b0 + t, sum4(&L.cs[4u * t]), ep);
+        if (t < nb) post(S_rz + (b0 - rb0) + t, sum4(&L.cs[4u * t]), ep);
         // ---- r.z of all row blocks, and the named rows' z, waited for by the other wavefronts meanwhile
-        if (t < 256u) wait_sum<U / 2>(S_rz, n_rb, ep, L, L.red[0]);
+        if (t < 256u) wait_sum<U / 2>(S_rz, nrb, nullptr, 0u, ep, L, L.red[0]);
         for (uint32_t e = (t + 256u) % T; e < nhalo; e += T) st3(L.z, e, wait_z(g.zx, n, L.halo[e], ep, L.bad));
         __syncthreads();
         ok = L.bad == 0u;
@@ -417,11 +431,11 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
     if (!ok)
     {
         // no workgroup may wait for this one any longer
-        if (t < nc) post(S_pq + 4u * b0 + t, 0.0f, kPoison);
-        if (t < nb) post(S_rz + b0 + t, 0.0f, kPoison);
+        if (t < nc) post(S_pq + 4u * (b0 - rb0) + t, 0.0f, kPoison);
+        if (t < nb) post(S_rz + (b0 - rb0) + t, 0.0f, kPoison);
         if (t == 0)
         {
-            ct.poison(S_pq + 4u * n_rb);
+            ct.poison(S_ch);
             __hip_atomic_store(&st->fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
@@ -439,7 +453,8 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
 // Solves without contacts.
 struct NoContacts
 {
-    LCSX_D void     begin(const PcgArgs&) {}
+    LCSX_D void     begin(const PcgArgs&, uint32_t, uint32_t, uint32_t) {}
+    LCSX_D uint32_t first() const { return 0u; }
     LCSX_D uint32_t chunks() const { return 0u; }
     LCSX_D void     slots(const PcgArgs&, const grid::Word*, bool, uint32_t, const float*, float, grid::Word*, uint32_t,
                           float*, uint32_t&) const

@@ -193,11 +193,7 @@ void Solver::init()
     minv.alloc(9 * (size_t)nv);
     sell_val.alloc(9 * (size_t)std::max(S.nblocks, 1u));
     part_rz.alloc(S.n_rb + 1);
-    sell_width = 0;
-    for (size_t k = 0; k + 1 < S.sl_off.size(); k++) sell_width = std::max(sell_width, S.sl_off[k + 1] - S.sl_off[k]);
-    pcg_grid = true;
-    grid_slots.free();
-    grid_zx.free();
+    plan_grid();
     // scene tables
     const uint32_t ns = S.nscenes;
     sc_v0_d.upload(S.sc_v0, stream);
@@ -252,6 +248,54 @@ void Solver::init()
     LCSX_HIP(hipStreamSynchronize(stream));
     inited = true;
     frame  = 0;
+}
+
+// The one-launch PCG's shape, and the scenes dealt to launches ("rounds") of at most kGridWgs
+// workgroups, the largest scenes first into the first round that still holds them. Up to two rounds: a
+// solve takes 1.12 ms in one round of 121,000 rows (1.88 with three launches per iteration), 3.4 ms in two
+// of 236,000 rows (4.0) and as long as the launches, 4.3 ms, in three of 306,000.
+void Solver::plan_grid()
+{
+    pcg_grid = true;
+    grid_slots.free();
+    grid_zx.free();
+    uint32_t width = 0, most = 0;
+    for (size_t k = 0; k + 1 < S.sl_off.size(); k++) width = std::max(width, S.sl_off[k + 1] - S.sl_off[k]);
+    for (uint32_t sc = 0; sc < S.nscenes; sc++) most = std::max(most, S.sc_rb0[sc + 1] - S.sc_rb0[sc]);
+    grid_shape = grid_plan(most, S.n_rb, width);
+    grid_round.clear();
+    if (!grid_shape.U) return;
+    constexpr size_t kRounds = 2;
+    const uint32_t per = grid_shape.row_blocks();
+    auto           wgs = [&](uint32_t sc) { return (S.sc_rb0[sc + 1] - S.sc_rb0[sc] + per - 1) / per; };
+    std::vector<uint32_t> order(S.nscenes);
+    for (uint32_t sc = 0; sc < S.nscenes; sc++) order[sc] = sc;
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return wgs(x) > wgs(y); });
+    std::vector<uint32_t> used, round(S.nscenes);
+    for (uint32_t sc : order)
+    {
+        size_t r = 0;
+        while (r < used.size() && used[r] + wgs(sc) > kGridWgs) r++;
+        if (r == used.size()) used.push_back(0u);
+        used[r] += wgs(sc);
+        round[sc] = (uint32_t)r;
+    }
+    if (used.size() > kRounds)
+    {
+        grid_shape = GridPlan{};
+        return;
+    }
+    grid_round.push_back(0u);
+    std::vector<uint2> tab;
+    for (size_t r = 0; r < used.size(); r++)
+    {
+        for (uint32_t sc : order)
+            if (round[sc] == r)
+                for (uint32_t k = 0; k < wgs(sc); k++) tab.push_back(make_uint2(sc, k));
+        grid_round.push_back((uint32_t)tab.size());
+    }
+    if (S.nscenes > 1) grid_tab.upload(tab, stream);
+    LCSX_HIP(hipStreamSynchronize(stream));
 }
 
 void Solver::upload_state_constants()
@@ -607,17 +651,19 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     const unsigned mc = vc.ptr ? max_chunks(vc.nslots) : 0u;
     launch_pcg_init(a, stream);
     host_pcg.assign(ns, PcgState{});
-    // one launch for all iterations up to the next residual replacement, or three per iteration
+    // one launch (per round of scenes) for all iterations up to the next residual replacement, or three
+    // per iteration. Contact slots beyond two chunks per 256 threads stay with the launches: each chunk
+    // costs an iteration of the one-launch form about 4 us, the launches' whole contact part 5-10 us.
     GridPlan  gp;
     GridLease lease;
-    if (pcg_grid && ns == 1 && !use_graphs && spmv_sample == 0)
+    const uint32_t gw = grid_round.empty() ? 0u : grid_round.back();
+    if (pcg_grid && grid_shape.U && !use_graphs && spmv_sample == 0 && mc <= 2u * gw * (kGridThreads / 256u) &&
+        lease.take(device))
+        gp = grid_shape;
+    const size_t grid_words = 5 * (size_t)S.n_rb + 2 * (size_t)gw * (kGridThreads / 256u);
+    if (gp.U && (!grid_slots.p || grid_epoch > 0xf0000000u))
     {
-        gp = grid_plan(S.n_rb, sell_width, mc);
-        if (gp.wgs && !lease.take(device)) gp = GridPlan{};
-    }
-    if (gp.wgs && (!grid_slots.p || grid_epoch > 0xf0000000u))
-    {
-        if (!grid_slots.p) grid_slots.alloc(kGridWords);
+        if (!grid_slots.p) grid_slots.alloc(grid_words);
         if (!grid_zx.p) grid_zx.alloc(3 * (size_t)S.nv);
         launch_grid_clear(grid_slots.p, grid_slots.n, stream);
         launch_grid_clear(grid_zx.p, grid_zx.n, stream);
@@ -630,18 +676,22 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     {
         // one host check per convergence-test interval (at least kPcgChunk launches), chunks
         // ending at the residual replacements
-        int chunk = std::min(gp.wgs ? max_iters : std::max(kPcgChunk, a.check_every > 1 ? (int)a.check_every : 0),
+        int chunk = std::min(gp.U ? max_iters : std::max(kPcgChunk, a.check_every > 1 ? (int)a.check_every : 0),
                              max_iters - issued);
         if (replace_every > 0) chunk = std::min(chunk, replace_every - issued % replace_every);
-        if (gp.wgs)
+        if (gp.U)
         {
             PcgArgs b = a;
             b.p_old   = p[par].p;
             b.p_new   = p[1 - par].p;
             b.k       = (uint32_t)issued;
-            const GridSync g{grid_slots.p, grid_zx.p, grid_epoch};
+            for (size_t r = 0; r + 1 < grid_round.size(); r++)
+            {
+                const uint32_t w0 = grid_round[r];
+                const GridSync g{grid_slots.p, grid_slots.p + S.n_rb, grid_zx.p, ns > 1 ? grid_tab.p + w0 : nullptr, grid_epoch};
+                launch_pcg_grid(gp, grid_round[r + 1] - w0, b, A, cv, vc, g, (uint32_t)chunk, stream);
+            }
             grid_epoch += (uint32_t)chunk;
-            launch_pcg_grid(gp, b, A, cv, vc, g, (uint32_t)chunk, stream);
             par = (par + chunk) & 1;
             if (timing) times["pcg_grid"].second += 1;  // launches of this form (no time of its own)
         }
@@ -726,7 +776,9 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
         }
         LCSX_HIP(hipStreamSynchronize(stream));
         flush_events();
-        if (gp.wgs && host_pcg[0].fail)
+        bool gave_up = false;
+        for (const PcgState& h : host_pcg) gave_up = gave_up || (gp.U && h.fail);
+        if (gave_up)
         {
             // a wait ran out or the gathered rows do not fit: the launches from the start, from now on
             pcg_grid = false;

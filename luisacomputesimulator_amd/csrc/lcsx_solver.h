@@ -188,13 +188,16 @@ struct Solver
     // PCG in one launch (lcsx_pcg_grid.h), the default where it fits; off while the caller chooses
     // the form of the launches (set_graphs, set_spmv_shape) or times them, and after it gave up once
     bool                     pcg_grid = true;
-    uint32_t                 sell_width = 0;  // most off-diagonal blocks of a row
+    GridPlan                 grid_shape;      // U 0: the rows or scenes do not fit
+    std::vector<uint32_t>    grid_round;      // workgroups of round r: [grid_round[r], grid_round[r + 1])
+    DBuf<uint2>              grid_tab;        // per workgroup: scene, place in it (several scenes)
     DBuf<unsigned long long> grid_slots, grid_zx;
     uint32_t                 grid_epoch = 0;
     // runtime mappings chosen by autotune() (defaults: the measured best on the 88K-vertex tube)
     // ACCD iterations per pair in the first CCD pass; pairs that need more run again in a second
     // pass over a compact list, so long iterations do not hold whole wavefronts
     int         ccd_budget            = 32;
+    void                     plan_grid();
     bool        contact_t_per_contact = true;  // one scene: t_c by one thread per contact
     int         query_variant         = kQueryDefault;  // LBVH traversal shape (lbvh_query)
     int         spmv_shape            = kSpmvShapeDefault;  // PCG SpMV mapping (launch_pcg_spmv)

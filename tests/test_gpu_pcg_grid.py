@@ -74,6 +74,27 @@ def test_one_launch_equals_launches(require_gpu, name, precision):
         assert contacts > 0
 
 
+def batch(sizes):
+    return [scenes.square_cloth(n, seed=k) if k % 2 else
+            scenes.cloth_on_sphere(n, 0.02, -0.01, seed=k, sphere_subdiv=2, height=0.3015) for k, n in enumerate(sizes)]
+
+
+# scenes of unequal sizes in one launch, scenes dealt to two, and more rows than two launches hold
+@pytest.mark.parametrize("sizes,one_launch", [((2, 9, 33, 17, 24), True), ((220, 33, 220, 221), True),
+                                              ((220,) * 6, False)])
+def test_batch_one_launch_equals_launches(require_gpu, sizes, one_launch):
+    one, launches = (NewtonSolver.from_scenes(batch(sizes)) for _ in range(2))
+    launches.set_graphs(False)
+    frames = 4 if max(sizes) < 100 else 1
+    for f in range(frames):
+        one.physics_step_gpu(1)
+        launches.physics_step_gpu(1)
+        print(f"[gpu-grid] batch {sizes} frame {f}: {one.stats()['pcg_iters_total']}", flush=True)
+        assert one.stats()["pcg_iters_total"] == launches.stats()["pcg_iters_total"]
+        assert np.array_equal(one.get_simulation_results(), launches.get_simulation_results())
+    assert ("pcg_grid" in one.kernel_times()) == one_launch
+
+
 def banded(n, half, seed):
     """A diagonally dominant block-CSR system: row i has the columns i - half .. i + half but itself."""
     rng = np.random.default_rng(seed)
