@@ -17,6 +17,7 @@ constexpr float kEpsilon        = 1.19209290E-7f;  // FLT_EPSILON (reference Cor
 constexpr float kLineSearchMaxT = 1.25f;           // ACCD step cap (reference accd.hpp:47)
 constexpr float kCcdReduction   = 0.01f;           // ACCD gap reduction (reference accd.hpp:46)
 constexpr uint32_t kInvalid     = 0xffffffffu;
+constexpr uint32_t kClusterLeaves = 1024;  // positions of a block of the solver's hierarchies (ClusterTree)
 
 struct f3
 {

@@ -110,6 +110,7 @@ struct Lbvh
     // (true, for sorted self-queries)
     int                   sorted_keys = 0;
     uint32_t*         sorted_to_orig = nullptr;  // points into vals[?] after construct
+    DBuf<uint32_t>    leaf_of;                   // its inverse: the sorted leaf of an element
     // traversal stack entries past a query's LDS part (grown by lbvh_query as needed)
     mutable DBuf<uint32_t> spill;
     // per inner node: the 4-wide record (the slots of both children's packed records; a leaf
@@ -179,5 +180,35 @@ struct QueryArgs
 constexpr int kQueryVariants = 10;
 constexpr int kQueryDefault  = 7;
 void lbvh_query(const Lbvh& t, const QueryArgs& a, hipStream_t s);
+
+// The hierarchy that the solver's broad phases walk in the shapes that share a query among lanes: over
+// the elements in a static order that keeps a mesh's neighbours together (Setup::cluster), so its
+// topology is made once and only its boxes change. Every scene starts a block of kClusterLeaves positions.
+struct ClusterQuery
+{
+    const uint32_t* order;  // queries (points, or edges), every scene padded with kInvalid to whole wavefronts
+    uint32_t        n;      // of them, padding included
+    const uint32_t* edges;  // null: points
+    const uint32_t* vert_scene;
+    const uint8_t*  active;
+    const float *   x0, *x1, *offset, *dhat;
+    uint32_t*       pairs;
+    uint32_t        capacity;
+    uint32_t*       count;
+};
+struct ClusterTree
+{
+    int              arity  = 3;
+    uint32_t         blocks = 0;
+    const uint32_t*  prims  = nullptr;  // device, arity per element (not owned)
+    DBuf<uint32_t>   elem, scene_block;  // element at a position (kInvalid: none); first block of each scene, and the end
+    DBuf<float4>     rec, top;           // records, blocks' boxes
+    void init(int arity_, const uint32_t* device_prims, const std::vector<uint32_t>& order,
+              const std::vector<uint32_t>& scene_block_, hipStream_t s);
+    // leaf_of: the elements' keys (null: their ids)
+    void refit(const float* x0, const float* x1, const float* pad, const uint32_t* leaf_of, hipStream_t s);
+    void query(const ClusterQuery& a, const uint32_t* leaf_of, hipStream_t s) const;
+};
+bool query_by_clusters(int variant);  // whether a traversal shape is one of those
 
 }  // namespace lcsx

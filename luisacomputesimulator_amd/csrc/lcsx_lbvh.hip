@@ -164,7 +164,7 @@ __global__ __launch_bounds__(1024) void k_build_small(uint32_t n, uint32_t ni, i
                                                        uint32_t* __restrict__ gbox, uint64_t* __restrict__ morton_sorted,
                                                        uint32_t* __restrict__ sorted, uint2* __restrict__ children,
                                                        uint32_t* __restrict__ object_idx, uint32_t* __restrict__ parent,
-                                                       uint32_t* __restrict__ tcount)
+                                                       uint32_t* __restrict__ tcount, uint32_t* __restrict__ leaf_of)
 {
     constexpr uint32_t kN = 1024u * kPer;
     __shared__ uint32_t skey[kN];
@@ -310,6 +310,7 @@ __global__ __launch_bounds__(1024) void k_build_small(uint32_t n, uint32_t ni, i
             morton_sorted[l]   = ((uint64_t)key[i] << 32) | (uint64_t)o;
             children[ni + l]   = make_uint2(o, o);
             object_idx[ni + l] = o;
+            leaf_of[o]         = l;
             if (n == 1u) parent[ni + l] = kInvalid;
         }
     }
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(kBlock) void k_leaves(uint32_t n, uint32_t ni, cons
                                                     const uint32_t* __restrict__ seg_of_leaf,
                                                     const uint32_t* __restrict__ seg_tab, uint64_t* __restrict__ morton_sorted,
                                                     uint2* __restrict__ children, uint32_t* __restrict__ object_idx,
-                                                    uint32_t* __restrict__ parent)
+                                                    uint32_t* __restrict__ parent, uint32_t* __restrict__ leaf_of)
 {
     uint32_t l = blockIdx.x * kBlock + threadIdx.x;
     if (l >= n) return;
@@ -427,6 +428,7 @@ __global__ __launch_bounds__(kBlock) void k_leaves(uint32_t n, uint32_t ni, cons
     morton_sorted[l] = ((uint64_t)skeys[l] << 32) | (uint64_t)(o - seg_tab[4 * g]);
     children[ni + l] = make_uint2(o, o);
     object_idx[ni + l] = o;
+    leaf_of[o]         = l;
     if (seg_tab[4 * g + 1] == 1u) parent[ni + l] = kInvalid;  // a one-leaf segment: the leaf is its root
 }
 
@@ -1021,8 +1023,6 @@ constexpr QueryShape kQueryShapes[kQueryVariants] = {{2, 32, 256, 1}, {2, 16, 51
 
 // Copies a wavefront's staged pairs to the global list: one atomic reserves the range, lanes
 // copy in strides of 64. Called by all 64 lanes.
-// kOrder: the staged pairs are (query, leaf) of a self-query, stored as (lower id, higher id)
-template <bool kOrder = false>
 LCSX_D void flush_pairs(const uint2* buf, uint32_t nbuf, uint32_t* count, uint32_t capacity, uint32_t* pairs)
 {
     __builtin_amdgcn_wave_barrier();
@@ -1032,8 +1032,7 @@ LCSX_D void flush_pairs(const uint2* buf, uint32_t nbuf, uint32_t* count, uint32
     for (uint32_t k = lane_id(); k < nbuf; k += 64u)
         if (base + k < capacity)
         {
-            uint2 v = buf[k];
-            if (kOrder) v = make_uint2(min(v.x, v.y), max(v.x, v.y));
+            const uint2 v = buf[k];
             pairs[2 * (size_t)(base + k)]     = v.x;
             pairs[2 * (size_t)(base + k) + 1] = v.y;
         }
@@ -1228,7 +1227,7 @@ __global__ __launch_bounds__(kQueryBlock) void k_query(QueryArgs a, const float4
 // each lane walks its own query), and the group shares one stack (64 entries, the first kS in LDS)
 // and one step count. Same leaves as the other shapes; a full stack ends the query after the
 // step's leaves are emitted, reported through *overflow.
-template <int kS, int kBuf, int kL, bool kSelf>
+template <int kS, int kBuf, int kL>
 __global__ __launch_bounds__(kQueryBlock) void k_query_coop(QueryArgs a, const float4* __restrict__ packed4,
                                                              uint32_t n_inner, const uint32_t* __restrict__ roots,
                                                              const NodeBox* __restrict__ nodes,
@@ -1261,51 +1260,20 @@ __global__ __launch_bounds__(kQueryBlock) void k_query_coop(QueryArgs a, const f
     };
     const uint32_t qi     = xcd_block(blockIdx.x, gridDim.x) * kGroups + grp;
     bool           active = qi < a.n_queries;
-    // kSelf: the sorted self-query of the edge tree (QueryEdges with sorted_self), an instance of its own
-    constexpr bool self = kSelf;
-    const uint32_t q      = (self && active) ? a.order[qi] : qi;
-    const uint32_t fk     = self ? qi : q;
-    // the filter flag is the same for every lane of the launch (kept in scalar registers)
-    const bool     filt = a.mode == QueryEdges || (a.mode == QueryBoxes && a.edge_filter != 0);
+    const uint32_t q      = qi;
+    const bool     filt = a.edge_filter != 0;
     f3             lo = mk(0.0f, 0.0f, 0.0f), hi = mk(0.0f, 0.0f, 0.0f);
     if (active)
     {
-        if (a.mode == QueryVerts)
-        {
-            f3    p0 = ld3(a.x0, q), p1 = ld3(a.x1, q);
-            float t  = a.offset[q] + a.dhat[q];
-            lo       = vmin(p0, p1) - mk(t, t, t);
-            hi       = vmax(p0, p1) + mk(t, t, t);
-        }
-        else if (a.mode == QueryEdges)
-        {
-            uint32_t e0 = a.edges[2 * q], e1 = a.edges[2 * q + 1];
-            f3       s0 = ld3(a.x0, e0), s1 = ld3(a.x0, e1), t0 = ld3(a.x1, e0), t1 = ld3(a.x1, e1);
-            float    t  = a.offset[e0] + a.dhat[e0];
-            lo          = vmin(vmin(s0, s1), vmin(t0, t1)) - mk(t, t, t);
-            hi          = vmax(vmax(s0, s1), vmax(t0, t1)) + mk(t, t, t);
-        }
-        else
-        {
-            lo = ld3(a.boxes, 2 * q);
-            hi = ld3(a.boxes, 2 * q + 1);
-        }
+        lo = ld3(a.boxes, 2 * q);
+        hi = ld3(a.boxes, 2 * q + 1);
     }
-    uint32_t root = kInvalid;
-    if (active)
-    {
-        uint32_t g = 0;
-        if (a.vert_scene && a.mode != QueryBoxes) g = a.vert_scene[a.mode == QueryVerts ? q : a.edges[2 * q]];
-        root = roots[g];
-        if (root == kInvalid || (a.active && a.active[g] == 0)) active = false;
-        if (a.mode == QueryVerts && a.row_kind && a.row_kind[q] >= 2u) active = false;
-    }
+    const uint32_t root = roots[0];  // a tree queried with boxes is one segment
+    if (root == kInvalid) active = false;
     // rank of this lane among the set lanes of a ballot below it
     auto rank = [](uint64_t bal) -> uint32_t {
         return __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
     };
-    // staged as (query, leaf); a self-query's pairs are ordered (lower id first) when flushed, once
-    // per staged pair instead of on every step
     auto pair_of = [&](uint32_t o) { return make_uint2(q, o); };
     int      sp     = 0;
     uint32_t visits = 0;
@@ -1320,10 +1288,9 @@ __global__ __launch_bounds__(kQueryBlock) void k_query_coop(QueryArgs a, const f
             {
                 const NodeBox  B   = nodes[root];
                 const uint32_t el  = children[root].x;
-                const uint32_t key = self ? root - n_inner : el;
-                e0 = overlap4(make_float4(B.lo.x, B.lo.y, B.lo.z, 0.0f), make_float4(B.hi.x, B.hi.y, B.hi.z, 0.0f), lo,
+                                e0 = overlap4(make_float4(B.lo.x, B.lo.y, B.lo.z, 0.0f), make_float4(B.hi.x, B.hi.y, B.hi.z, 0.0f), lo,
                               hi) &&
-                     (!filt || fk < key);
+                     (!filt || q < el);
                 o0 = el;
             }
             active = false;
@@ -1377,7 +1344,7 @@ __global__ __launch_bounds__(kQueryBlock) void k_query_coop(QueryArgs a, const f
             // bitwise, not short-circuit, so the conditions stay lane masks in scalar registers
             code[u]      = __float_as_uint(r[2 * u].w);
             const bool h = work & overlap4(r[2 * u], r[2 * u + 1], lo, hi) &
-                           ((fk < __float_as_uint(r[2 * u + 1].w)) | !filt);
+                           ((q < __float_as_uint(r[2 * u + 1].w)) | !filt);
             inner_hit[u] = h & ((int)code[u] >= 0);
             e[u]         = h & ((int)code[u] < 0);
             gm[u]        = (uint32_t)(__ballot(inner_hit[u]) >> (lane_id() & ~(uint32_t)(kL - 1))) & kGMask;
@@ -1413,11 +1380,358 @@ __global__ __launch_bounds__(kQueryBlock) void k_query_coop(QueryArgs a, const f
         }
         if (nbuf > (uint32_t)(kBuf - 64 * kU))
         {
-            flush_pairs<kSelf>(buf[wv], nbuf, a.count, a.capacity, a.pairs);
+            flush_pairs(buf[wv], nbuf, a.count, a.capacity, a.pairs);
             nbuf = 0;
         }
     }
-    if (nbuf) flush_pairs<kSelf>(buf[wv], nbuf, a.count, a.capacity, a.pairs);
+    if (nbuf) flush_pairs(buf[wv], nbuf, a.count, a.capacity, a.pairs);
+}
+
+// ---- The solver's own hierarchy (ClusterTree). A block is kClusterLeaves consecutive positions of the
+// static order and a complete 4-ary tree over them: 256 records of four leaves, 64 of four of those, and
+// so on to one, kClusterRecords records of the packed4 layout in a row, children at fixed places. Above
+// the blocks there is only the list of their boxes, which a wavefront tests 64 at a time.
+// Unions drop NaNs (fminf, fmaxf), so a vertex gone astray hides no other.
+LCSX_D f3 umin(f3 a, f3 b) { return mk(fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z)); }
+LCSX_D f3 umax(f3 a, f3 b) { return mk(fmaxf(a.x, b.x), fmaxf(a.y, b.y), fmaxf(a.z, b.z)); }
+constexpr uint32_t kClusterRecords = 341;  // 256 + 64 + 16 + 4 + 1
+static_assert(kClusterLeaves == 1024, "kClusterRecords");
+
+// One workgroup per block: a thread makes the record of its four positions, then each level's boxes go
+// into their parents' records, all in LDS; the block leaves as one stretch of 43 KB. Bound by the gathered
+// loads of the elements' vertices. 187,000 faces and 281,000 edges: 11 us on average (the LBVH's leaves,
+// treelets and top: 54).
+__global__ __launch_bounds__(256) void k_cluster_refit(int arity, const uint32_t* __restrict__ prims,
+                                                       const uint32_t* __restrict__ elem, const uint32_t* __restrict__ leaf_of,
+                                                       const float* __restrict__ x0, const float* __restrict__ x1,
+                                                       const float* __restrict__ pad, float4* __restrict__ rec,
+                                                       float4* __restrict__ top)
+{
+    __shared__ float4 img[8 * kClusterRecords];
+    const uint32_t    t = threadIdx.x, blk = blockIdx.x;
+    const float       inf = __int_as_float(0x7f800000);
+    f3                lo = mk(inf, inf, inf), hi = mk(-inf, -inf, -inf);
+    uint32_t          key = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++)
+    {
+        const uint32_t at = blk * kClusterLeaves + 4 * t + k;
+        const uint32_t el = elem[at];  // kInvalid: a position between two scenes
+        float4         l  = make_float4(inf, inf, inf, __uint_as_float(0x80000000u));
+        float4         h  = make_float4(-inf, -inf, -inf, 0.0f);
+        if (el != kInvalid)
+        {
+            const NodeBox  B = leaf_box(at, arity, prims, elem, x0, x1, pad);
+            const uint32_t w = leaf_of ? leaf_of[el] : el;
+            l   = make_float4(B.lo.x, B.lo.y, B.lo.z, __uint_as_float(0x80000000u | el));
+            h   = make_float4(B.hi.x, B.hi.y, B.hi.z, __uint_as_float(w));
+            lo  = umin(lo, mk(l.x, l.y, l.z));
+            hi  = umax(hi, mk(h.x, h.y, h.z));
+            key = max(key, w);
+        }
+        img[8 * t + 2 * k]     = l;
+        img[8 * t + 2 * k + 1] = h;
+    }
+    // this thread's box, as a slot of its parent's record; then the next level's first threads
+    uint32_t node = t, base = 256, cnt = 256;
+    while (true)
+    {
+        if (t < cnt)
+        {
+            const float4 l = make_float4(lo.x, lo.y, lo.z, __uint_as_float(blk * kClusterRecords + node));
+            const float4 h = make_float4(hi.x, hi.y, hi.z, __uint_as_float(key));
+            if (cnt == 1u)
+            {
+                top[2 * blk]     = l;
+                top[2 * blk + 1] = h;
+            }
+            else
+            {
+                img[8 * (base + t / 4u) + 2 * (t & 3u)]     = l;
+                img[8 * (base + t / 4u) + 2 * (t & 3u) + 1] = h;
+            }
+        }
+        __syncthreads();
+        if (cnt == 1u) break;
+        cnt /= 4u;
+        node = base + t;
+        if (t < cnt)
+        {
+            lo  = mk(inf, inf, inf);
+            hi  = mk(-inf, -inf, -inf);
+            key = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++)
+            {
+                const float4 l = img[8 * node + 2 * k], h = img[8 * node + 2 * k + 1];
+                lo  = umin(lo, mk(l.x, l.y, l.z));
+                hi  = umax(hi, mk(h.x, h.y, h.z));
+                key = max(key, __float_as_uint(h.w));
+            }
+        }
+        base += cnt;
+    }
+    float4* const out = rec + (size_t)blk * (8 * kClusterRecords);
+    for (uint32_t k = t; k < 8 * kClusterRecords; k += 256u) out[k] = img[k];
+}
+
+// One wavefront per 16 consecutive points or edges of the static order: they visit nearly the same nodes,
+// so the wavefront walks the tree once for all of them, up to 32 nodes a step (four lanes test the slots of
+// a record against the queries' joint boxes), lists the leaves met in LDS and tests each of them against
+// the queries, four leaves at a time in the four quarters of the wavefront. In the LBVH (whose Morton box,
+// as the reference's, covers the first third of a cloth's edges, so the rest is sorted along two axes or
+// one) a query's own walk visited 15 to 250 records one after the other.
+// The order's curve jumps now and then, and one joint box over a jump would cover much of the mesh: the
+// queries are cut at the three largest jumps into four joint boxes (64 queries on a 161 x 161 cloth and its
+// sphere met 299 leaves with one box, 152 with four, 147 with eight).
+// 16 queries: 64 leave a small mesh with a few long wavefronts (a 33 x 33 cloth: 39 us, 14 with 16), and
+// their 64 box tests per leaf met are mostly misses; 8 walk the top of the tree twice as often (edges
+// of the batch below: 1310 us against 680, before the reservations were shared).
+// kEdges: an edge keeps the leaves whose key is above its own: the LBVH's sorted leaf where the pair test
+// is symmetric (sorted_ee), so that each pair is tested from the same side as in a query of the LBVH, or
+// the element id.
+// Per query of edges and of points: 24 scenes of 306,000 vertices, 6.5 M and 2.4 M pairs: 226 and 87 us
+// (1162 and 307 in the LBVH with four lanes per query); 297 x 297 tube in wide contact bands: 273 and 92 us
+// (497 and 176).
+constexpr int kGroupStack = 384, kGroupLeaves = 160, kGroupBuf = 768, kGroupCuts = 3;
+constexpr uint32_t kGroup = 16;  // queries of a wavefront
+constexpr int kGroupWaves = 8;
+constexpr int kGroupTests = 4;  // leaves read together per quarter, ahead of their tests
+template <bool kEdges>
+__global__ __launch_bounds__(64 * kGroupWaves) void k_query_group(ClusterQuery a, const float4* __restrict__ rec,
+                                                              const float4* __restrict__ top,
+                                                              const uint32_t* __restrict__ scene_block,
+                                                              const uint32_t* __restrict__ leaf_of)
+{
+    constexpr int kWaves = kGroupWaves, kBoxes = kGroupCuts + 1;
+    constexpr uint32_t kShares = 64u / kGroup;
+    static_assert(kGroup <= 16 && kGroupTests * 64 <= kGroupBuf, "a pair's query takes 4 bits, its element 28 (Lbvh::init)");
+    static_assert(kGroupLeaves % (kGroupTests * kShares) == 0, "the last batch of tests stays in the list");
+    __shared__ uint32_t stack_[kWaves][kGroupStack];
+    __shared__ float4   leaf_[kWaves][2 * kGroupLeaves];
+    __shared__ uint32_t buf_[kWaves][kGroupBuf];  // pairs: query in the top 4 bits, element below
+    __shared__ uint32_t n_[kWaves], base_;
+    const uint32_t      wv = threadIdx.x >> 6, lane = lane_id(), g = lane >> 2, j = lane & 3u;
+    const uint32_t      li = lane & (kGroup - 1u), part = lane / kGroup;  // query, share of the leaves
+    uint32_t* const     stack = stack_[wv];
+    float4* const       leaf  = leaf_[wv];
+    uint32_t* const     buf   = buf_[wv];
+    const uint32_t      at    = (xcd_block(blockIdx.x, gridDim.x) * kWaves + wv) * kGroup;
+    const float         inf   = __int_as_float(0x7f800000);
+    auto rank = [](uint64_t bal) -> uint32_t {
+        return __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+    };
+    // this lane's query (the lists are padded to whole wavefronts per scene)
+    const uint32_t q = at < a.n ? a.order[at + li] : kInvalid;
+    bool           live = __ballot(q != kInvalid) != 0ull;  // uniform across the wavefront
+    f3       lo = mk(inf, inf, inf), hi = mk(-inf, -inf, -inf);
+    uint32_t own = kInvalid, sc = 0;  // key above which leaves are kept (kEdges), scene
+    if (q != kInvalid)
+    {
+        const uint32_t e0 = kEdges ? a.edges[2 * q] : q;
+        const float    t  = a.offset[e0] + a.dhat[e0];
+        if (kEdges)
+        {
+            const uint32_t e1 = a.edges[2 * q + 1];
+            const f3       s0 = ld3(a.x0, e0), s1 = ld3(a.x0, e1), t0 = ld3(a.x1, e0), t1 = ld3(a.x1, e1);
+            lo  = vmin(vmin(s0, s1), vmin(t0, t1)) - mk(t, t, t);
+            hi  = vmax(vmax(s0, s1), vmax(t0, t1)) + mk(t, t, t);
+            own = leaf_of ? leaf_of[q] : q;
+        }
+        else
+        {
+            const f3 p0 = ld3(a.x0, q), p1 = ld3(a.x1, q);
+            lo = vmin(p0, p1) - mk(t, t, t);
+            hi = vmax(p0, p1) + mk(t, t, t);
+        }
+        if (a.vert_scene) sc = a.vert_scene[e0];
+    }
+    // a scene's first position is a multiple of 64, so lane 0 holds a query of it
+    sc = (uint32_t)__builtin_amdgcn_readfirstlane((int)sc);
+    live = live && !(a.active && a.active[sc] == 0);
+    // ---- joint boxes: lanes [start, ...) up to the next cut share one
+    uint64_t cuts = 1ull;  // bit l: a joint box starts at lane l
+    {
+        const f3 ln = mk(__shfl_down(lo.x, 1), __shfl_down(lo.y, 1), __shfl_down(lo.z, 1));
+        const f3 hn = mk(__shfl_down(hi.x, 1), __shfl_down(hi.y, 1), __shfl_down(hi.z, 1));
+        const f3 e  = vmax(hi, hn) - vmin(lo, ln);
+        // the extent of this lane's and the next one's joint box, with the lane in the low bits
+        uint32_t d = (__float_as_uint(fmaxf(fmaxf(fmaxf(e.x, e.y), e.z), 0.0f)) & ~63u) | li;
+        if (li == kGroup - 1u) d = 0u;
+#pragma unroll
+        for (int c = 0; c < kGroupCuts; c++)
+        {
+            uint32_t m = d;
+            for (int o = kGroup / 2; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+            const uint32_t cut = (uint32_t)__builtin_amdgcn_readfirstlane((int)(m & 63u));
+            cuts |= 2ull << cut;
+            if (li == cut) d = 0u;
+        }
+    }
+    f3 ulo[kBoxes], uhi[kBoxes];
+    {
+        const uint32_t start = 63u - (uint32_t)__clzll((long long)(cuts & (~0ull >> (63u - li))));
+        f3             l = lo, h = hi;
+#pragma unroll
+        for (uint32_t o = 1; o < kGroup; o <<= 1)
+        {
+            const f3 lp = mk(__shfl_up(l.x, o), __shfl_up(l.y, o), __shfl_up(l.z, o));
+            const f3 hp = mk(__shfl_up(h.x, o), __shfl_up(h.y, o), __shfl_up(h.z, o));
+            if (li >= start + o)
+            {
+                l = umin(l, lp);
+                h = umax(h, hp);
+            }
+        }
+        uint64_t left = cuts;
+#pragma unroll
+        for (int c = 0; c < kBoxes; c++)
+        {
+            // the box that starts at the lowest bit ends before the next one
+            const bool any = left != 0ull;
+            left &= left - 1ull;
+            const int last = left ? __ffsll((long long)left) - 2 : (int)kGroup - 1;
+            auto      part = [&](float v, float none) {
+                const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), last));
+                return any ? r : none;
+            };
+            ulo[c] = mk(part(l.x, inf), part(l.y, inf), part(l.z, inf));
+            uhi[c] = mk(part(h.x, -inf), part(h.y, -inf), part(h.z, -inf));
+        }
+    }
+    uint32_t first = own;  // a subtree whose largest key is not above the smallest own one holds no pair
+    if (kEdges)
+        for (int o = kGroup / 2; o > 0; o >>= 1) first = min(first, (uint32_t)__shfl_xor((int)first, o));
+    auto met = [&](float4 b0, float4 b1) {
+        bool h = false;
+#pragma unroll
+        for (int c = 0; c < kBoxes; c++) h = h | overlap4(b0, b1, ulo[c], uhi[c]);
+        return kEdges ? h & (first < __float_as_uint(b1.w)) : h;
+    };
+    uint32_t sp = 0, nleaf = 0, nbuf = 0;  // uniform across the wavefront
+    auto     write = [&](uint32_t to) {
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t k0 = 0; k0 < nbuf; k0 += 64u)
+        {
+            const uint32_t k = k0 + lane, v = buf[min(k, nbuf - 1u)];
+            const uint32_t e0 = __shfl(q, (int)(v >> 28)), e1 = v & 0x0fffffffu;
+            if (k < nbuf && to + k < a.capacity)
+            {
+                a.pairs[2 * (size_t)(to + k)]     = kEdges ? min(e0, e1) : e0;
+                a.pairs[2 * (size_t)(to + k) + 1] = kEdges ? max(e0, e1) : e1;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto test_leaves = [&]() {
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t c0 = part; c0 - part < nleaf; c0 += kGroupTests * kShares)
+        {
+            float4   b0[kGroupTests], b1[kGroupTests];
+            uint64_t bal[kGroupTests];
+            uint32_t total = 0;
+#pragma unroll
+            for (int u = 0; u < kGroupTests; u++)  // (past the last leaf: any entry of the list, dropped)
+            {
+                b0[u] = leaf[2 * (c0 + u * kShares)];
+                b1[u] = leaf[2 * (c0 + u * kShares) + 1];
+            }
+#pragma unroll
+            for (int u = 0; u < kGroupTests; u++)
+            {
+                bool e = overlap4(b0[u], b1[u], lo, hi) & (c0 + u * kShares < nleaf);
+                if (kEdges) e = e & (own < __float_as_uint(b1[u].w));
+                bal[u] = __ballot(e);
+                total += (uint32_t)__popcll(bal[u]);
+            }
+            if (nbuf + total > (uint32_t)kGroupBuf)
+            {
+                uint32_t to = 0;
+                if (lane == 0u) to = count_reserve(a.count, nbuf);
+                write(__shfl(to, 0));
+                nbuf = 0;
+            }
+#pragma unroll
+            for (int u = 0; u < kGroupTests; u++)
+            {
+                if ((bal[u] >> lane) & 1ull)
+                    buf[nbuf + rank(bal[u])] = li << 28 | (__float_as_uint(b0[u].w) & 0x0fffffffu);
+                nbuf += (uint32_t)__popcll(bal[u]);
+            }
+        }
+        nleaf = 0;
+        __builtin_amdgcn_wave_barrier();
+    };
+    // ---- the walk: the scene's blocks while few nodes are at hand, else up to 32 nodes a step
+    uint32_t       blk = live ? scene_block[sc] : 0u;
+    const uint32_t end = live ? scene_block[sc + 1] : 0u;
+    while (true)
+    {
+        if (sp < 16u && blk < end)
+        {
+            bool   h  = false;
+            float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (blk + lane < end)
+            {
+                r0 = top[2 * (blk + lane)];
+                h  = met(r0, top[2 * (blk + lane) + 1]);
+            }
+            const uint64_t bal = __ballot(h);
+            if (h) stack[sp + rank(bal)] = __float_as_uint(r0.w);
+            sp += (uint32_t)__popcll(bal);
+            blk += 64u;
+            __builtin_amdgcn_wave_barrier();
+            continue;
+        }
+        if (sp == 0u) break;
+        // Up to 32 nodes: sp stays below 384. At most 224 entries remain under the 32, and 128 come on top of
+        // them; beyond 256 one node is taken at a time, which adds at most 3 for each of the 4 levels below it.
+        const uint32_t take = sp > 256u ? 1u : min(sp, 32u);
+        sp -= take;
+        float4 r0[2], r1[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+        {
+            const uint32_t k  = g + 16u * u;
+            const uint32_t nd = k < take ? stack[sp + k] : 0u;
+            const float4*  P  = rec + (nd * 8u + 2u * j);
+            r0[u] = P[0];
+            r1[u] = P[1];
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+        {
+            const bool     h      = (g + 16u * u < take) & met(r0[u], r1[u]);
+            const bool     isleaf = (int)__float_as_uint(r0[u].w) < 0;
+            const uint64_t bi = __ballot(h & !isleaf), bl = __ballot(h & isleaf);
+            if (h & !isleaf) stack[sp + rank(bi)] = __float_as_uint(r0[u].w);
+            sp += (uint32_t)__popcll(bi);
+            if (h & isleaf)
+            {
+                leaf[2 * (nleaf + rank(bl))]     = r0[u];
+                leaf[2 * (nleaf + rank(bl)) + 1] = r1[u];
+            }
+            nleaf += (uint32_t)__popcll(bl);
+        }
+        if (nleaf > (uint32_t)kGroupLeaves - 128u) test_leaves();
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (nleaf) test_leaves();
+    // one reservation for the workgroup: single ones queue at the counter, 11 ns each, which was all of the
+    // time with one per wavefront (58,000 of them: 680 us)
+    if (lane == 0u) n_[wv] = nbuf;
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        uint32_t n = 0;
+        for (int w = 0; w < kWaves; w++) n += n_[w];
+        base_ = n ? count_reserve(a.count, n) : 0u;
+    }
+    __syncthreads();
+    uint32_t to = base_;
+    for (uint32_t w = 0; w < wv; w++) to += n_[w];
+    write(to);
 }
 
 template <int V>
@@ -1426,12 +1740,8 @@ void launch_query_shape(const Lbvh& t, const QueryArgs& a, uint32_t grid, hipStr
     constexpr QueryShape Q = kQueryShapes[V];
     if constexpr (Q.lanes >= 2)
     {
-        if (a.mode == QueryEdges && a.sorted_self)
-            k_query_coop<Q.lds_stack, Q.buf, Q.lanes, true><<<grid, kQueryBlock, 0, s>>>(
-                a, t.packed4.p, t.ni, t.roots.p, t.nodes.p, t.children.p, t.spill.p);
-        else
-            k_query_coop<Q.lds_stack, Q.buf, Q.lanes, false><<<grid, kQueryBlock, 0, s>>>(
-                a, t.packed4.p, t.ni, t.roots.p, t.nodes.p, t.children.p, t.spill.p);
+        k_query_coop<Q.lds_stack, Q.buf, Q.lanes><<<grid, kQueryBlock, 0, s>>>(
+            a, t.packed4.p, t.ni, t.roots.p, t.nodes.p, t.children.p, t.spill.p);
     }
     else
         k_query<Q.wide, Q.lds_stack, Q.buf><<<grid, kQueryBlock, 0, s>>>(a, Q.wide == 4 ? t.packed4.p : t.packed.p, t.ni,
@@ -1497,6 +1807,7 @@ void Lbvh::init(int arity_, const uint32_t* device_prims, uint32_t n_leaves, con
     morton_sorted.alloc(n);
     parent.alloc(n_nodes());
     object_idx.alloc(n_nodes());
+    leaf_of.alloc(n);
     children.alloc(n_nodes());
     nodes.alloc(n_nodes());
     packed.alloc(4 * (size_t)(ni ? ni : 1));
@@ -1537,7 +1848,7 @@ void Lbvh::construct(const float* x, const uint32_t* verts_per_seg, hipStream_t 
         sorted_to_orig = vals[0].p;
         auto go        = [&](auto kern) {
             kern<<<1, 1024, 0, s>>>(n, ni, arity, prims, x, cover_h[0], gbox.p, morton_sorted.p, sorted_to_orig, children.p,
-                                    object_idx.p, parent.p, tcount.p);
+                                    object_idx.p, parent.p, tcount.p, leaf_of.p);
         };
         if (n <= 4096u) go(k_build_small<4>);
         else go(k_build_small<8>);
@@ -1567,7 +1878,7 @@ void Lbvh::construct(const float* x, const uint32_t* verts_per_seg, hipStream_t 
     }
     sorted_to_orig = vals[cur].p;
     k_leaves<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, ni, keys[cur].p, vals[cur].p, seg_of_leaf.p, seg_tab.p,
-                                                    morton_sorted.p, children.p, object_idx.p, parent.p);
+                                                    morton_sorted.p, children.p, object_idx.p, parent.p, leaf_of.p);
     k_fill_u32<<<1, kBlock, 0, s>>>(tcount.p, 2u, 0u);
     finish(s);
 }
@@ -1693,6 +2004,47 @@ void lbvh_query(const Lbvh& t, const QueryArgs& a, hipStream_t s)
     case 8: launch_query_shape<8>(t, a, grid, s); break;
     default: launch_query_shape<9>(t, a, grid, s); break;
     }
+    LCSX_HIP(hipGetLastError());
+}
+
+bool query_by_clusters(int variant)
+{
+    const int v = variant >= 0 && variant < kQueryVariants ? variant : kQueryDefault;
+    return kQueryShapes[v].lanes >= 2;
+}
+
+void ClusterTree::init(int arity_, const uint32_t* device_prims, const std::vector<uint32_t>& order,
+                       const std::vector<uint32_t>& scene_block_, hipStream_t s)
+{
+    arity  = arity_;
+    prims  = device_prims;
+    blocks = (uint32_t)(order.size() / kClusterLeaves);
+    if (blocks > 0xffffffffu / (8u * kClusterRecords))  // records are addressed in 32 bits
+    {
+        set_error("broad phase: too many elements");
+        throw CapacityFailure();
+    }
+    elem.upload(order, s);
+    scene_block.upload(scene_block_, s);
+    if (!blocks) return;
+    rec.alloc(8 * (size_t)kClusterRecords * blocks);
+    top.alloc(2 * (size_t)blocks);
+}
+
+void ClusterTree::refit(const float* x0, const float* x1, const float* pad, const uint32_t* leaf_of, hipStream_t s)
+{
+    if (!blocks) return;
+    k_cluster_refit<<<blocks, 256, 0, s>>>(arity, prims, elem.p, leaf_of, x0, x1, pad, rec.p, top.p);
+    LCSX_HIP(hipGetLastError());
+}
+
+void ClusterTree::query(const ClusterQuery& a, const uint32_t* leaf_of, hipStream_t s) const
+{
+    if (!blocks || !a.n) return;
+    const uint32_t per  = kGroup * kGroupWaves;  // queries of a block
+    const uint32_t grid = (a.n + per - 1) / per;
+    if (a.edges) k_query_group<true><<<grid, 64 * kGroupWaves, 0, s>>>(a, rec.p, top.p, scene_block.p, leaf_of);
+    else k_query_group<false><<<grid, 64 * kGroupWaves, 0, s>>>(a, rec.p, top.p, scene_block.p, leaf_of);
     LCSX_HIP(hipGetLastError());
 }
 

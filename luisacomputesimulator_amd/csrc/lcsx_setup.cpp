@@ -145,6 +145,109 @@ void animate_target(const lcsx_fixed_anim& a, float t, const float in[3], float 
     out[2] = p.z;
 }
 
+// Sorts n ids by their 30-bit codes, equal ones by id (they come in ascending order): three stable
+// counting passes, or std::sort for few.
+static void sort_by_code(uint32_t* id, const std::vector<uint32_t>& code, size_t n, std::vector<uint32_t>& tmp)
+{
+    if (n < 1024)
+    {
+        std::stable_sort(id, id + n, [&](uint32_t x, uint32_t y) { return code[x] < code[y]; });
+        return;
+    }
+    tmp.resize(std::max(tmp.size(), n));
+    uint32_t *from = id, *to = tmp.data();
+    for (int shift = 0; shift < 30; shift += 10)
+    {
+        uint32_t at[1024] = {}, sum = 0;
+        for (size_t i = 0; i < n; i++) at[(code[from[i]] >> shift) & 1023u]++;
+        for (uint32_t& c : at) std::swap(c, sum), sum += c;
+        for (size_t i = 0; i < n; i++) to[at[(code[from[i]] >> shift) & 1023u]++] = from[i];
+        std::swap(from, to);
+    }
+    std::copy(from, from + n, id);  // (three passes end in tmp)
+}
+
+void Setup::cluster()
+{
+    // per mesh: the rest pose's box (a cube of its largest side, so that distances along the axes count alike)
+    uint32_t nm = 0;
+    for (uint32_t i = 0; i < nv; i++) nm = std::max(nm, vert_mesh[i] + 1u);
+    std::vector<float>    lo(3 * (size_t)nm, 3.0e38f), hi(3 * (size_t)nm, -3.0e38f), scale(nm);
+    std::vector<uint32_t> mesh_scene(nm, 0);
+    auto                  point = [&](uint32_t i) { return row_kind[i] < 2; };
+    for (uint32_t i = 0; i < nv; i++)
+    {
+        const uint32_t m = vert_mesh[i];
+        mesh_scene[m]    = vert_scene[i];
+        for (uint32_t k = 0; point(i) && k < 3; k++)
+        {
+            lo[3 * m + k] = std::min(lo[3 * m + k], rest_x[3 * i + k]);
+            hi[3 * m + k] = std::max(hi[3 * m + k], rest_x[3 * i + k]);
+        }
+    }
+    for (uint32_t m = 0; m < nm; m++)
+    {
+        float side = 1e-12f;
+        for (uint32_t k = 0; k < 3; k++) side = std::max(side, hi[3 * m + k] - lo[3 * m + k]);
+        scale[m] = 1024.0f / side;
+    }
+    auto spread = [](uint32_t v) {  // ten bits, two zeros between any two
+        v = (v | (v << 16)) & 0x030000ffu;
+        v = (v | (v << 8)) & 0x0300f00fu;
+        v = (v | (v << 4)) & 0x030c30c3u;
+        return (v | (v << 2)) & 0x09249249u;
+    };
+    auto morton = [&](uint32_t m, const float c[3]) {
+        uint32_t code = 0;
+        for (uint32_t k = 0; k < 3; k++)
+        {
+            const float v = (c[k] - lo[3 * m + k]) * scale[m];
+            code |= spread(v > 0.0f ? (uint32_t)std::min(v, 1023.0f) : 0u) << (2 - k);
+        }
+        return code;
+    };
+    // the elements of all meshes, each mesh's along its curve, every scene padded to whole units (the meshes
+    // are numbered scene by scene); arity 0: points
+    std::vector<uint32_t> code, id, first, tmp;
+    auto ordered = [&](uint32_t n, uint32_t arity, const std::vector<uint32_t>& prims, uint32_t unit,
+                       std::vector<uint32_t>& out, std::vector<uint32_t>* block) {
+        auto mesh = [&](uint32_t i) { return vert_mesh[arity ? prims[arity * i] : i]; };
+        code.resize(n);
+        first.assign(nm + 1, 0);
+        for (uint32_t i = 0; i < n; i++)
+        {
+            if (!arity && !point(i)) continue;
+            float c[3] = {0.0f, 0.0f, 0.0f};
+            for (uint32_t k = 0; k < 3; k++)
+                if (!arity) c[k] = rest_x[3 * i + k];
+                else
+                    for (uint32_t a = 0; a < arity; a++) c[k] += rest_x[3 * prims[arity * i + a] + k] / (float)arity;
+            code[i] = morton(mesh(i), c);
+            first[mesh(i) + 1]++;
+        }
+        for (uint32_t m = 0; m < nm; m++) first[m + 1] += first[m];
+        id.resize(first[nm]);
+        std::vector<uint32_t> at(first.begin(), first.end() - 1);
+        for (uint32_t i = 0; i < n; i++)
+            if (arity || point(i)) id[at[mesh(i)]++] = i;
+        uint32_t m = 0;
+        for (uint32_t sc = 0; sc < nscenes; sc++)
+        {
+            if (block) block->push_back((uint32_t)(out.size() / unit));
+            for (; m < nm && mesh_scene[m] <= sc; m++)
+            {
+                sort_by_code(id.data() + first[m], code, first[m + 1] - first[m], tmp);
+                out.insert(out.end(), id.begin() + first[m], id.begin() + first[m + 1]);
+            }
+            while (out.size() % unit) out.push_back(kInvalid);
+        }
+        if (block) block->push_back((uint32_t)(out.size() / unit));
+    };
+    ordered(nv, 0, faces, 64, cluster_v, nullptr);
+    ordered(nf, 3, faces, kClusterLeaves, cluster_f, &cluster_f_block);
+    ordered(ne, 2, edges, kClusterLeaves, cluster_e, &cluster_e_block);
+}
+
 void Setup::build(const std::vector<MeshDesc>& meshes)
 {
     *this = Setup();
@@ -518,6 +621,7 @@ void Setup::build(const std::vector<MeshDesc>& meshes)
             for (uint32_t jj = 0; jj < 4; jj++)
                 if (ii != jj) b.blk[k++] = slot_of(b.row0 + ii, b.row0 + jj);
     }
+    cluster();
 }
 
 // Shell body (RigidMaterial is_shell, init_sim_data.cpp:600-640): mass carried by the vertices

@@ -76,9 +76,16 @@ struct Setup
     std::vector<uint32_t> vert_body;  // per row: body id (rigid vertex or body row) or ~0u
     std::vector<float>    body_X;     // per row: body-frame position of a rigid vertex (3)
 
+    // points (rows of kind 0 and 1), faces and edges, mesh by mesh and along a Morton curve through each
+    // mesh's rest pose: neighbours in these lists are neighbours in space, however a mesh moves. Every scene
+    // is padded with kInvalid, to whole wavefronts of 64 points and whole blocks of kClusterLeaves elements;
+    // _block: the first block of each scene, and the end.
+    std::vector<uint32_t> cluster_v, cluster_f, cluster_e, cluster_f_block, cluster_e_block;
+
     void build(const std::vector<MeshDesc>& meshes);
 
 private:
+    void cluster();
     void rigid_shell_mass(const Body& b, uint32_t mi, const std::vector<float>& vvol, const std::vector<float>& body_vol,
                           const std::vector<float>& body_mass, float& m, float mx[3], float mxx[3][3], float& vol) const;
     void rigid_solid_mass(const Body& b, uint32_t mi, const std::vector<uint32_t>& face_mesh_, float& m, float mx[3],

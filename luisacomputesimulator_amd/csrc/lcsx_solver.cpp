@@ -330,6 +330,10 @@ void Solver::upload_state_constants()
     blk_contrib.upload(S.blk_contrib, s);
     fixed_ids.upload(S.fixed_verts, s);
     row_kind_d.upload(S.row_kind, s);
+    cluster_vert.upload(S.cluster_v, s);
+    n_cluster_vert = (uint32_t)S.cluster_v.size();
+    cluster_face.init(3, faces.p, S.cluster_f, S.cluster_f_block, s);
+    cluster_edge.init(2, edges.p, S.cluster_e, S.cluster_e_block, s);
     vert_body_d.upload(S.vert_body, s);
     body_X_d.upload(S.body_X, s);
     static_assert(sizeof(BodyDev) == sizeof(Setup::Body), "body record layout");
@@ -524,12 +528,36 @@ void Solver::material()
     toc("material");
 }
 
+ClusterQuery Solver::cluster_query(const float* x0) const
+{
+    ClusterQuery c{};
+    c.vert_scene = vert_scene_d.p;
+    c.active     = active_d.p;
+    c.x0         = x0;
+    c.x1         = x.p;
+    c.offset     = offset.p;
+    c.dhat       = dhat.p;
+    return c;
+}
+
 void Solver::query_faces(bool ccd)
 {
     if (S.nf == 0) return;
     const float* x0 = ccd ? x_iter.p : x.p;
     Status*      st = status.p;
     tree_face.refit(x0, x.p, offset.p, stream);
+    if (query_by_clusters(query_variant))
+    {
+        ClusterQuery c = cluster_query(x0);
+        c.order        = cluster_vert.p;
+        c.n            = n_cluster_vert;
+        c.pairs        = pairs_vf.p;
+        c.capacity     = cap_vf;
+        c.count        = ccd ? &st->n_vf_ccd : &st->n_vf;
+        cluster_face.refit(x0, x.p, offset.p, nullptr, stream);
+        cluster_face.query(c, nullptr, stream);
+        return;
+    }
     QueryArgs q{};
     q.vert_scene = vert_scene_d.p;
     q.active     = active_d.p;
@@ -554,6 +582,20 @@ void Solver::query_edges(bool ccd)
     const float* x0 = ccd ? x_iter.p : x.p;
     Status*      st = status.p;
     tree_edge.refit(x0, x.p, offset.p, stream);
+    if (query_by_clusters(query_variant))
+    {
+        ClusterQuery    c       = cluster_query(x0);
+        const uint32_t* leaf_of = sorted_ee ? tree_edge.leaf_of.p : nullptr;
+        c.order                 = cluster_edge.elem.p;
+        c.n                     = cluster_edge.blocks * kClusterLeaves;
+        c.edges                 = edges.p;
+        c.pairs                 = pairs_ee.p;
+        c.capacity              = cap_ee;
+        c.count                 = ccd ? &st->n_ee_ccd : &st->n_ee;
+        cluster_edge.refit(x0, x.p, offset.p, leaf_of, stream);
+        cluster_edge.query(c, leaf_of, stream);
+        return;
+    }
     QueryArgs q{};
     q.vert_scene = vert_scene_d.p;
     q.active     = active_d.p;

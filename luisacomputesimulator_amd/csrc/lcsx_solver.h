@@ -46,6 +46,10 @@ struct Solver
     DBuf<float>    face_stage, hinge_stage, spring_stage;
     Lbvh           tree_face, tree_edge;
     bool           sorted_ee = false;  // edge-edge candidates by the sorted self-query
+    ClusterTree    cluster_face, cluster_edge;
+    DBuf<uint32_t> cluster_vert;  // points in the order of their queries
+    uint32_t       n_cluster_vert = 0;
+    ClusterQuery   cluster_query(const float* x0) const;
     // collision buffers
     DBuf<uint32_t> pairs_vf, pairs_ee;
     uint32_t       cap_vf = 0, cap_ee = 0, cap_c = 0;
@@ -193,11 +197,11 @@ struct Solver
     DBuf<uint2>              grid_tab;        // per workgroup: scene, place in it (several scenes)
     DBuf<unsigned long long> grid_slots, grid_zx;
     uint32_t                 grid_epoch = 0;
+    void                     plan_grid();
     // runtime mappings chosen by autotune() (defaults: the measured best on the 88K-vertex tube)
     // ACCD iterations per pair in the first CCD pass; pairs that need more run again in a second
     // pass over a compact list, so long iterations do not hold whole wavefronts
     int         ccd_budget            = 32;
-    void                     plan_grid();
     bool        contact_t_per_contact = true;  // one scene: t_c by one thread per contact
     int         query_variant         = kQueryDefault;  // LBVH traversal shape (lbvh_query)
     int         spmv_shape            = kSpmvShapeDefault;  // PCG SpMV mapping (launch_pcg_spmv)

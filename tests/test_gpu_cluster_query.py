@@ -1,0 +1,65 @@
+"""The broad phase over the solver's own hierarchies (clusters in the rest pose's order, 16 queries per
+wavefront) against one walk of the LBVH per query (traversal shape 1): the same candidate pairs, as sets,
+at the start and after the meshes have moved."""
+import numpy as np
+import pytest
+
+from luisacomputesimulator_amd import NewtonSolver, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def mixed_dhat():
+    """Two offsets in one scene: the edge pairs are kept by element id."""
+    sc = scenes.cloth_on_sphere(17, 0.02, -0.01, seed=3, sphere_subdiv=2, height=0.3015)
+    sc.meshes[0].material.thickness *= 1.5
+    return sc
+
+
+def boxes():
+    sc = scenes.cloth_rigid_coupling(n=17, boxes=2, seed=3, box_region=((-0.25, 0.25), (0.32, 0.5), (-0.25, 0.25)))
+    for m in sc.meshes[1:]:
+        m.verts[:, 1] -= np.float32(m.verts[:, 1].min() - (0.2 + 1.3e-3))
+    return sc
+
+
+# edges per scene: 5 (one record and a part), 1008 and 1121 (around a block of 1024 positions), 70,000 (more
+# than 64 blocks: the list of blocks takes two steps), long edges beside short ones, several scenes
+CASES = {
+    "square_2": lambda: [scenes.square_cloth(2)],
+    "square_19": lambda: [scenes.square_cloth(19)],
+    "square_20": lambda: [scenes.square_cloth(20)],
+    "square_155": lambda: [scenes.square_cloth(155)],
+    "sphere_24": lambda: [scenes.cloth_on_sphere(24, 0.02, -0.01, seed=4, sphere_subdiv=2, height=0.3015)],
+    "tube": lambda: [scenes.cylinder_tube(rings=96, per_ring=96, cyl_radius=0.1084, cyl_segments=96, cyl_rings=5)],
+    "mixed_dhat": lambda: [mixed_dhat()],
+    "boxes": lambda: [boxes()],
+    "batch": lambda: [scenes.square_cloth(2), scenes.square_cloth(33),
+                      scenes.cloth_on_sphere(17, 0.05, -0.03, seed=1, sphere_subdiv=2, height=0.3015)],
+}
+
+
+def pairs(s, key):
+    p = s.read(key).reshape(-1, 2)
+    return p[np.lexsort((p[:, 1], p[:, 0]))]
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_clusters_find_the_pairs_of_the_lbvh(require_gpu, name):
+    scs = CASES[name]()
+    s = NewtonSolver.from_scenes(scs) if len(scs) > 1 else NewtonSolver.from_scene(scs[0])
+    for frame in range(2):
+        for stage in ("frame_begin", "predict", "iter_begin"):
+            s.stage(stage)
+        for stage in ("broad_phase_dcd", "broad_phase_ccd"):
+            got = []
+            for shape in (7, 1):
+                s.set_query_shape(shape)
+                s.stage(stage)
+                got.append([pairs(s, "pairs_vf"), pairs(s, "pairs_ee")])
+            print(f"[gpu-cluster] {name} frame {frame} {stage}: {len(got[0][0])} vf, {len(got[0][1])} ee", flush=True)
+            for a, b in zip(*got):
+                assert len(np.unique(a, axis=0)) == len(a)
+                assert np.array_equal(a, b)
+        s.set_query_shape(7)
+        s.physics_step_gpu(3)
