@@ -125,7 +125,8 @@ struct Lbvh
     // min(n_g, 256 ceil(verts_g / 256)) leaves (lbvh.cpp:958, 968)
     void construct(const float* x, const uint32_t* verts_per_seg, hipStream_t s);
     void finish(hipStream_t s);  // construct, from the sorted leaves on
-    void refit(const float* x0, const float* x1, const float* pad, hipStream_t s);
+    // wide: with the 4-wide records
+    void refit(const float* x0, const float* x1, const float* pad, hipStream_t s, bool wide = true);
     uint32_t n_inner() const { return ni; }
     uint32_t n_nodes() const { return n + ni; }
 };

@@ -693,6 +693,7 @@ LCSX_D void inner_box(uint32_t p, uint32_t ni, const uint2* __restrict__ childre
     P[1]      = pa1;
     P[2]      = pb0;
     P[3]      = pb1;
+    if (!packed4) return;
     float4* Q = packed4 + 8 * (size_t)p;
     if (c.x < ni)
     {
@@ -781,6 +782,9 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
     {
         p  = order[k];
         tc = top_child[k];
+        // top nodes below these levels (a larger top): refit before, read as what lies outside
+        if (tc.z >= T) tc.x &= 0x7fffffffu;
+        if (tc.w >= T) tc.y &= 0x7fffffffu;
         // the slot of a child outside the top
         auto outside = [&](uint32_t c, int side) {
             const NodeBox B = nodes[c];
@@ -855,6 +859,7 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
     P[1]      = pa1;
     P[2]      = pb0;
     P[3]      = pb1;
+    if (!packed4) return;
     float4* Q = packed4 + 8 * (size_t)p;
     const uint32_t cs[2] = {tc.x, tc.y}, ks[2] = {tc.z, tc.w};
     for (int side = 0; side < 2; side++)
@@ -967,7 +972,7 @@ __global__ __launch_bounds__(kTreeletBlock) void k_refit_treelets(const uint32_t
             return make_float4(ib[t][l], ib[t + 1][l], ib[t + 2][l], __uint_as_float(hi ? ikey[l] : c));
         };
         float4* const Q = packed4 + 8 * (size_t)first;
-        for (uint32_t i = k; i < 8u * cnt; i += kN)
+        for (uint32_t i = k; packed4 && i < 8u * cnt; i += kN)
         {
             const uint32_t c = ich[(i >> 2) & 1u][i >> 3], sub = (i >> 1) & 1u;
             const bool     hi = (i & 1u) != 0u;
@@ -1926,30 +1931,37 @@ void Lbvh::finish(hipStream_t s)
     LCSX_HIP(hipGetLastError());
 }
 
-void Lbvh::refit(const float* x0, const float* x1, const float* pad, hipStream_t s)
+void Lbvh::refit(const float* x0, const float* x1, const float* pad, hipStream_t s, bool wide)
 {
     if (n == 0) return;
     k_refit_leaves<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, ni, arity, prims, sorted_to_orig, x0, x1, pad, nodes.p);
     if (ni == 0) return;
+    float4* const p4 = wide ? packed4.p : nullptr;
     // uncounted: about one workgroup per treelet, each taking every grid-th one
     const uint32_t tgrid = counted ? ntreelets : n / 384u + 1u;
     if (tgrid)
         k_refit_treelets<<<tgrid, kTreeletBlock, 0, s>>>(tcount.p, troots.p, tsize.p, tfirst.p, tleaf.p, parent.p, ni,
-                                                         children.p, nodes.p, packed.p, packed4.p, sorted_keys);
-    // the nodes above the treelets (none up to kTreeletLeaves leaves)
-    if (n > kTreeletLeaves && (!counted || (ntop && ntop <= kTopLds)))
-        k_refit_top<<<1, 1024, 0, s>>>(top_order.p, top_level_ptr.p, kMaxLevels - 1u, ni, top_child.p, children.p, nodes.p,
-                                       packed.p, packed4.p, sorted_keys);
-    else if (ntop > kTopLds)
-        for (int h = (int)kMaxLevels - 1; h >= 0; h--)
-        {
-            const uint32_t b = top_lvp_h[h], e = top_lvp_h[h + 1];
-            if (e > b)
-                k_refit_range<<<grid_for(e - b, kBlock), kBlock, 0, s>>>(top_order.p + b, e - b, ni, children.p, nodes.p,
-                                                                         packed.p, packed4.p, sorted_keys);
-        }
+                                                         children.p, nodes.p, packed.p, p4, sorted_keys);
+    // the nodes above the treelets (none up to kTreeletLeaves leaves): the levels nearest the roots that one
+    // workgroup's LDS holds together in one launch, the levels below them one by one before it (24 scenes:
+    // 58 us of launches per refit where every level had its own, now 25)
+    if (n > kTreeletLeaves && (!counted || ntop))
+    {
+        uint32_t levels = kMaxLevels;
+        if (counted && ntop > kTopLds)
+            for (; top_lvp_h[levels] > kTopLds; levels--)
+            {
+                const uint32_t b = top_lvp_h[levels - 1], e = top_lvp_h[levels];
+                if (e > b)
+                    k_refit_range<<<grid_for(e - b, kBlock), kBlock, 0, s>>>(top_order.p + b, e - b, ni, children.p, nodes.p,
+                                                                             packed.p, p4, sorted_keys);
+            }
+        if (levels)
+            k_refit_top<<<1, 1024, 0, s>>>(top_order.p, top_level_ptr.p, levels - 1u, ni, top_child.p, children.p, nodes.p,
+                                           packed.p, p4, sorted_keys);
+    }
     LCSX_HIP(hipGetLastError());
-    wide_ready = true;
+    wide_ready = wide;
 }
 
 uint32_t sort_hist_words(uint32_t n)

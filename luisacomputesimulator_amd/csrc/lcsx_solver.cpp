@@ -545,7 +545,7 @@ void Solver::query_faces(bool ccd)
     if (S.nf == 0) return;
     const float* x0 = ccd ? x_iter.p : x.p;
     Status*      st = status.p;
-    tree_face.refit(x0, x.p, offset.p, stream);
+    tree_face.refit(x0, x.p, offset.p, stream, !query_by_clusters(query_variant));
     if (query_by_clusters(query_variant))
     {
         ClusterQuery c = cluster_query(x0);
@@ -581,7 +581,7 @@ void Solver::query_edges(bool ccd)
     if (S.ne == 0) return;
     const float* x0 = ccd ? x_iter.p : x.p;
     Status*      st = status.p;
-    tree_edge.refit(x0, x.p, offset.p, stream);
+    tree_edge.refit(x0, x.p, offset.p, stream, !query_by_clusters(query_variant));
     if (query_by_clusters(query_variant))
     {
         ClusterQuery    c       = cluster_query(x0);
