@@ -694,15 +694,22 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     launch_pcg_init(a, stream);
     host_pcg.assign(ns, PcgState{});
     // one launch (per round of scenes) for all iterations up to the next residual replacement, or three
-    // per iteration. Contact slots beyond two chunks per 256 threads stay with the launches: each chunk
-    // costs an iteration of the one-launch form about 4 us, the launches' whole contact part 5-10 us.
+    // per iteration. The launches' time hardly depends on the contacts, the one launch's does. One row
+    // block per workgroup: up to two slot chunks per 256 threads (a 200 x 200 cloth on a sphere, 300
+    // iterations: 1.35 ms against 2.02 at 4,276 contacts; a 100 x 100 tube 1.30 against 1.56 at 13,000). Two
+    // row blocks per workgroup spill with contacts (94,000 rows, 100 iterations: 1.09 against 1.94 ms
+    // without contacts, 1.95 against 2.05 with 215, 2.19 against 2.09 with 1,172, 2.87 against 2.22 with
+    // 18,000): a chunk per scene and one for 16 workgroups, or 8 in a batch, whose scenes wait for their own
+    // chunks only (202,000 rows with a chunk for 11 workgroups: 2.48 against 2.99).
     GridPlan  gp;
     GridLease lease;
     const uint32_t gw = grid_round.empty() ? 0u : grid_round.back();
-    if (pcg_grid && grid_shape.U && !use_graphs && spmv_sample == 0 && mc <= 2u * gw * (kGridThreads / 256u) &&
+    const uint32_t grid_chunks = 2u * gw * (kGridThreads / 256u);  // that the words are for
+    const uint32_t most_chunks = grid_shape.U == 2 ? grid_chunks : std::min(grid_chunks, ns + gw / (ns == 1u ? 16u : 8u));
+    if (pcg_grid && grid_shape.U && !use_graphs && spmv_sample == 0 && mc <= most_chunks &&
         lease.take(device))
         gp = grid_shape;
-    const size_t grid_words = 5 * (size_t)S.n_rb + 2 * (size_t)gw * (kGridThreads / 256u);
+    const size_t grid_words = 5 * (size_t)S.n_rb + grid_chunks;
     if (gp.U && (!grid_slots.p || grid_epoch > 0xf0000000u))
     {
         if (!grid_slots.p) grid_slots.alloc(grid_words);
