@@ -298,7 +298,9 @@ lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on);
  * 32 stack entries in LDS, 512 pairs staged; 7 is the default. 9: two lanes per query on the 128 B
  * records (lane j tests grandchildren 2j and 2j + 1), 16 stack entries in LDS, 512 pairs staged
  * (faster where the queries fill the GPU, as in large batches). Before a tree's
- * first refit the 4-wide shapes run as the binary shape 1 or 3. */
+ * first refit the 4-wide shapes run as the binary shape 1 or 3. That is how a standalone tree is
+ * queried; in a solver 7, 8 and 9 all walk its own hierarchies, 16 neighbouring queries per
+ * wavefront, whose walks have no stack to overflow. */
 lcsx_status lcsx_solver_set_query_shape(lcsx_solver* s, int shape);
 /* Mapping of the PCG block SpMV (no counterpart in the reference; every shape gives the same
  * bits, the blocks of a row being added in the same order). 0: three blocks per lane and pass with

@@ -402,9 +402,9 @@ class NewtonSolver:
         _check(self.lib.lcsx_solver_set_graphs(self.h, int(on)))
 
     def set_query_shape(self, shape: int) -> None:
-        """Broad-phase traversal shape (0..3 binary steps, 4..6 four-wide steps, 7..8 four-wide
-        steps with four lanes per query, 9 with two lanes per query; different LDS stack entries
-        and per-wavefront pair staging; every shape finds the same pairs)."""
+        """Broad-phase traversal shape (0..3 binary steps, 4..6 four-wide steps of the LBVH with
+        different LDS stack entries and per-wavefront pair staging; 7..9 the solver's own
+        hierarchies, 16 queries per wavefront; every shape finds the same pairs)."""
         _check(self.lib.lcsx_solver_set_query_shape(self.h, int(shape)))
 
     def set_spmv_shape(self, shape: int) -> None:
