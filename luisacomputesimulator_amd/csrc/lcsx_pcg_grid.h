@@ -270,8 +270,9 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
             }
         }
     __syncthreads();
-    const uint32_t nhalo = L.nhalo;
-    bool           ok    = L.bad == 0u && R + nhalo <= kGridRows;
+    // more named rows than there is room for: halo holds the first ones only, and none is read
+    bool           ok    = L.bad == 0u && L.nhalo <= kGridRows - R;
+    const uint32_t nhalo = ok ? L.nhalo : 0u;
     if (ok)
     {
 #pragma unroll

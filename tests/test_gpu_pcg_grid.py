@@ -146,23 +146,78 @@ def test_block_csr_solve(require_gpu, n, half):
     assert res["iters"] == 100 and err < 1e-4
 
 
-def test_block_csr_scattered_columns(require_gpu):
-    """Columns all over the matrix: a workgroup names more rows than it can hold and the solve starts over
-    with the launches. Against numpy's 64-bit solution."""
-    n, rng = 20000, np.random.default_rng(5)
-    i = np.repeat(np.arange(n), 14)
+def named_rows(ptr, cols, rows):
+    """The most rows outside its own that the columns of one workgroup (of `rows` rows) name."""
+    n, most = len(ptr) - 1, 0
+    for r in range(0, n, rows):
+        c = np.unique(cols[ptr[r]:ptr[min(r + rows, n)]])
+        most = max(most, int(np.count_nonzero((c < r) | (c >= r + rows))))
+    return most
+
+
+def widened(ptr, cols, blocks, diag):
+    """The same system with 40 zero blocks more in its last row: wider than any one-launch shape, so the solve
+    takes the launches, where a zero block adds nothing."""
+    extra = np.arange(40) % (len(ptr) - 1)
+    ptr = ptr.copy()
+    ptr[-1] += len(extra)
+    return BsrSystem(ptr, np.concatenate([cols, extra]), np.concatenate([blocks, np.zeros((40, 3, 3), np.float32)]), diag)
+
+
+# columns all over the matrix: a workgroup of 256 rows holds p of 3,840 others, one of 512 rows (above 65,536
+# rows) of 3,584; the last two fit
+@pytest.mark.parametrize("n,width,fits", [(60000, 20, False), (100000, 10, False), (20000, 14, True), (70000, 6, True)])
+def test_block_csr_scattered_columns(require_gpu, n, width, fits):
+    """A workgroup that names more rows than it can hold gives up before it reads any of them, and the solve is
+    the launches'. Bit for bit against the launches, and against the dominance of the diagonal."""
+    rng = np.random.default_rng(n + width)
+    i = np.repeat(np.arange(n), width)
     c = rng.integers(0, n, size=i.size)
     c = np.where(c == i, (c + 1) % n, c)
+    ptr = np.arange(n + 1) * width
+    room = 3840 if n <= 65536 else 3584
+    named = named_rows(ptr, c, 4096 - room)
+    print(f"[gpu-grid] scattered n {n}, {width} blocks a row: {named} rows named, room for {room}", flush=True)
+    assert (named <= room) == fits
     blocks = np.tile(-0.01 * np.eye(3, dtype=np.float32), (i.size, 1, 1))
+    blocks *= (1.0 + 0.5 * np.sin(np.arange(i.size, dtype=np.float32)))[:, None, None]
     diag = np.tile(np.eye(3, dtype=np.float32), (n, 1, 1))
     b = rng.normal(size=(n, 3)).astype(np.float32)
-    x, res = pcg_solve_bsr(BsrSystem(np.arange(n + 1) * 14, c, blocks, diag), b, max_iters=4, check_every=4, abs_tol=0.0)
+    opt = dict(max_iters=4, check_every=4, abs_tol=0.0)
+    x, res = pcg_solve_bsr(BsrSystem(ptr, c, blocks, diag), b, **opt)
     assert res["iters"] == 4 and np.isfinite(x).all()
+    y, launched = pcg_solve_bsr(widened(ptr, c, blocks, diag), b, **opt)
+    assert np.array_equal(x, y) and res == launched
     # the matrix is not symmetric: only that four iterations reduce the residual as the dominance says
     r = b - x.astype(np.float64)
     for d in range(3):
-        r[:, d] += 0.01 * np.bincount(i, weights=x[c, d].astype(np.float64), minlength=n)
+        r[:, d] -= np.bincount(i, weights=blocks[:, d, d].astype(np.float64) * x[c, d], minlength=n)
     assert np.linalg.norm(r) < 0.02 * np.linalg.norm(b)
+
+
+def test_shuffled_cloth_takes_the_launches(require_gpu):
+    """A cloth whose vertices are numbered at random, as a mesh file may have them: the one-launch form gives up
+    in its first solve, and the frame is the launches', bit for bit."""
+    def solver():
+        sc = scenes.square_cloth(257)
+        m, perm = sc.meshes[0], np.random.default_rng(7).permutation(257 * 257)
+        place = np.empty_like(perm)
+        place[perm] = np.arange(len(perm))
+        m.verts, m.tris = m.verts[perm], place[m.tris].astype(np.int32)
+        return NewtonSolver.from_scene(sc)
+
+    one, launches = solver(), solver()
+    csr = one.read("csr").astype(np.int64)
+    n = 257 * 257
+    named = named_rows(csr[:n + 1] - (n + 1), csr[n + 1:], 512)
+    print(f"[gpu-grid] shuffled cloth: {named} rows named", flush=True)
+    assert named > 3584
+    launches.set_graphs(False)
+    for g in (one, launches):
+        g.physics_step_gpu(1)
+    assert one.stats()["pcg_iters_total"] == launches.stats()["pcg_iters_total"]
+    assert one.kernel_times()["pcg_grid"][1] == 1
+    assert np.array_equal(one.get_simulation_results(), launches.get_simulation_results())
 
 
 def test_block_csr_bad_index_in_the_middle(require_gpu):
