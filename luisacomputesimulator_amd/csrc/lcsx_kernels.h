@@ -344,7 +344,8 @@ void launch_dcd(const DcdArgs& a, int kind, unsigned grid, hipStream_t s);
 // tmp: one word per slot (scratch of the slot ordering)
 void launch_contact_adjacency(const ContactView& c, uint32_t nv, unsigned grid, uint32_t* cnt, uint32_t* ptr,
                               uint32_t* list, uint32_t* row, float4* coef, uint32_t* tmp, const SegView& g,
-                              uint32_t* sc_cb0, uint32_t* cb_scene, uint32_t* cb_slot0, hipStream_t s);
+                              uint32_t* sc_cb0, uint32_t* cb_scene, uint32_t* cb_slot0, bool repeats,
+                              hipStream_t s);
 // Scratch of the contact-triplet assembly (grown on demand; not used by the Newton loop).
 struct ContactTripletBufs
 {

@@ -1252,14 +1252,24 @@ __global__ __launch_bounds__(kB) void k_vc_fill(ContactView c, const uint32_t* _
     }
 }
 
-// Each row's slots in a fixed order: by the contact's vertex ids (with the type bit; a contact names
-// a row once). The narrow phase appends contacts with atomics, so contact ids differ from run to run;
+// Each row's slots in a fixed order: by the contact's vertex ids (with the type bit). The narrow phase
+// appends contacts with atomics, so contact ids differ from run to run;
 // ordering the slots by content makes every per-row sum (contact gradient and Hessian, the SpMV's
 // contact runs) add its terms in the same order in every run, so a state and its contact set give
-// the same rounding. A slot's place is its rank among its row's slots, whose keys are unique. One
+// the same rounding. A slot's place is its rank among its row's slots. One
 // thread per slot walks a short row by itself; the slots of a longer one (a collider vertex has
 // hundreds) are compared by their wavefront together, 64 of the row's keys at a time from registers
 // (2.8M slots: 678 us when every thread walked its row, now 316).
+// kTies: meshes that list an edge or a face twice, or an element that names a vertex twice
+// (Setup::repeats), give slots of one row with equal ids. Those are ordered by their entry, their
+// contact's k2 (the listings differ in area) and the contact's id, so every slot still has a place of its own.
+LCSX_D bool tie_less(const ContactView& c, uint32_t y, uint32_t x)
+{
+    if ((y & 7u) != (x & 7u)) return (y & 7u) < (x & 7u);
+    const uint32_t ky = __float_as_uint(c.nk[y >> 3].w), kx = __float_as_uint(c.nk[x >> 3].w);
+    return ky != kx ? ky < kx : y < x;
+}
+template <bool kTies>
 __global__ __launch_bounds__(kB) void k_vc_rank(ContactView c, const uint32_t* __restrict__ ptr,
                                                  const uint32_t* __restrict__ row, const uint32_t* __restrict__ total,
                                                  const uint32_t* __restrict__ list, uint32_t* __restrict__ out)
@@ -1275,13 +1285,21 @@ __global__ __launch_bounds__(kB) void k_vc_rank(ContactView c, const uint32_t* _
         const uint64_t hx = ((uint64_t)kx.x << 32) | kx.y, lx = ((uint64_t)kx.z << 32) | kx.w;
         auto less = [&](uint64_t hy, uint64_t ly) { return (hy < hx) | ((hy == hx) & (ly < lx)); };
         uint32_t rank = 0u;
-        if (on && m <= kShort)
+        if (kTies && on)
+            for (uint32_t t = 0; t < m; t++)
+            {
+                const uint32_t y  = list[b + t];
+                const uint4    ky = c.idx[y >> 3];
+                const uint64_t hy = ((uint64_t)ky.x << 32) | ky.y, ly = ((uint64_t)ky.z << 32) | ky.w;
+                if (less(hy, ly) || (hy == hx && ly == lx && y != x && tie_less(c, y, x))) rank++;
+            }
+        if (!kTies && on && m <= kShort)
             for (uint32_t t = 0; t < m; t++)
             {
                 const uint4 ky = c.idx[list[b + t] >> 3];
                 rank += less(((uint64_t)ky.x << 32) | ky.y, ((uint64_t)ky.z << 32) | ky.w) ? 1u : 0u;
             }
-        for (uint64_t todo = __ballot(on && m > kShort); todo != 0ull;)
+        for (uint64_t todo = __ballot(!kTies && on && m > kShort); todo != 0ull;)
         {
             const int      lead = __ffsll((unsigned long long)todo) - 1;
             const uint32_t rb = (uint32_t)__builtin_amdgcn_readlane((int)b, lead);
@@ -2712,14 +2730,15 @@ void launch_dcd(const DcdArgs& a, int kind, unsigned grid, hipStream_t s)
 }
 void launch_contact_adjacency(const ContactView& c, uint32_t nv, unsigned grid, uint32_t* cnt, uint32_t* ptr,
                               uint32_t* list, uint32_t* row, float4* coef, uint32_t* tmp, const SegView& g,
-                              uint32_t* sc_cb0, uint32_t* cb_scene, uint32_t* cb_slot0, hipStream_t s)
+                              uint32_t* sc_cb0, uint32_t* cb_scene, uint32_t* cb_slot0, bool repeats, hipStream_t s)
 {
     k_fill_u32<<<grid_for(nv + 1, kB), kB, 0, s>>>(cnt, nv + 1, 0u);
     k_vc_count<<<grid, kB, 0, s>>>(c, cnt);
     launch_scan_excl_u32(cnt, ptr, nv, list, s);  // list: scratch for the tile sums (refilled below)
     k_fill_u32<<<grid_for(nv + 1, kB), kB, 0, s>>>(cnt, nv + 1, 0u);
     k_vc_fill<<<grid, kB, 0, s>>>(c, ptr, cnt, list, row);
-    k_vc_rank<<<4 * grid, kB, 0, s>>>(c, ptr, row, ptr + nv, list, tmp);
+    if (repeats) k_vc_rank<true><<<4 * grid, kB, 0, s>>>(c, ptr, row, ptr + nv, list, tmp);
+    else k_vc_rank<false><<<4 * grid, kB, 0, s>>>(c, ptr, row, ptr + nv, list, tmp);
     k_vc_coeffs<<<4 * grid, kB, 0, s>>>(c, ptr, nv, tmp, list, coef);
     k_chunk_table<<<1, 1024, 0, s>>>(g, ptr, sc_cb0, cb_scene, cb_slot0);
 }

@@ -316,6 +316,12 @@ void Setup::build(const std::vector<MeshDesc>& meshes)
     nf = (uint32_t)(faces.size() / 3);
     ne = (uint32_t)(edges.size() / 2);
     nh = (uint32_t)(hinges.size() / 4);
+    // (edges are sorted within a mesh; two listings of a face are the two sides of a hinge, unless a third
+    // face makes its edge a repeated one; a face that names a vertex twice has the edge of that vertex)
+    for (uint32_t e = 0; e < ne; e++)
+        repeats = repeats || edges[2 * e] == edges[2 * e + 1] ||
+                  (e && edges[2 * e] == edges[2 * e - 2] && edges[2 * e + 1] == edges[2 * e - 1]);
+    for (uint32_t h = 0; h < nh; h++) repeats = repeats || hinges[4 * h + 2] == hinges[4 * h + 3];
 
     // scene ranges (meshes arrive in non-decreasing scene order) and scene-aligned row blocks
     nscenes = meshes.empty() ? 1u : meshes.back().scene + 1u;

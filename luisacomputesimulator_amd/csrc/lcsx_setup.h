@@ -76,6 +76,10 @@ struct Setup
     std::vector<uint32_t> vert_body;  // per row: body id (rigid vertex or body row) or ~0u
     std::vector<float>    body_X;     // per row: body-frame position of a rigid vertex (3)
 
+    // an edge or a face listed twice (an edge of three or more faces is), or an element that names a vertex
+    // twice: contacts of one row may then have equal vertex ids
+    bool repeats = false;
+
     // points (rows of kind 0 and 1), faces and edges, mesh by mesh and along a Morton curve through each
     // mesh's rest pose: neighbours in these lists are neighbours in space, however a mesh moves. Every scene
     // is padded with kInvalid, to whole wavefronts of 64 points and whole blocks of kClusterLeaves elements;

@@ -679,7 +679,7 @@ void Solver::contact_assemble()
     // the run sums are free until the PCG: their words hold the ordered slot list meanwhile
     launch_contact_adjacency(contact_view(), S.nv, pair_grid(cap_c), vc_cnt.p, vc_ptr.p, vc_list.p, vc_row.p, vc_coef.p,
                              reinterpret_cast<uint32_t*>(vc_runsum.p), seg_view(true), sc_cb0_d.p, cb_scene_d.p,
-                             cb_slot0_d.p, stream);
+                             cb_slot0_d.p, S.repeats, stream);
     vc_ready = true;
     VertContacts vc{vc_ptr.p, vc_list.p, vc_row.p, vc_coef.p, vc_tc.p, 0u, vc_ptr.p + S.nv};  // assembly walks the per-row lists
     launch_contact_assemble(contact_view(), vc, cgB.p, diag.p, S.nv, stream);
