@@ -1612,13 +1612,16 @@ std::string Solver::autotune()
             }
         }
         ccd_budget = best < kTuneMargin * cur ? bb : b0;
-        // the swept broad phase's traversal shape (LDS stack entries, pair staging)
+        // the swept broad phase's traversal shape (LDS stack entries, pair staging). The shapes that walk the
+        // solver's own hierarchies are one code path here: one of them is timed, so that noise picks none
         best         = 1e30f;
         cur          = 1e30f;
         const int v0 = query_variant;
         int       vb = query_variant;
+        const int vc = query_by_clusters(v0) ? v0 : kQueryDefault;
         for (int v = 0; v < kQueryVariants; v++)
         {
+            if (query_by_clusters(v) && v != vc) continue;
             query_variant = v;
             line_search();
             read_status();

@@ -47,3 +47,15 @@ def test_autotune_in_contact(require_gpu):
         err = np.abs(xa - xb).max() / np.abs(xb).max()
         print(f"[gpu-autotune] frame {f}: rel diff {err:.3e}, contacts {a.stats()['num_contacts']}", flush=True)
         assert err < 1e-4
+
+
+@pytest.mark.parametrize("shape", [7, 9])
+def test_autotune_times_one_shape_of_the_solvers_hierarchies(require_gpu, shape):
+    """Shapes 7 to 9 walk the same hierarchies in a solver: the one in use (or 7) stands for them."""
+    g = NewtonSolver.from_scene(scenes.square_cloth(17))
+    g.set_query_shape(shape)
+    g.physics_step_gpu(1)
+    rep = g.autotune()
+    timed = [int(k.split("=")[1][:-1]) for k in rep if k.startswith("line_search[query=")]
+    print(f"[gpu-autotune] shapes timed {timed}, chosen {rep['chosen']['query']}", flush=True)
+    assert timed == list(range(7)) + [shape] and rep["chosen"]["query"] in timed
