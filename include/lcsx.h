@@ -397,6 +397,16 @@ lcsx_status lcsx_pcg_solve_bsr_noalloc(const lcsx_bsr* A, const float* device_b,
  * row on `stream`. Bad indices as in lcsx_pcg_solve_bsr. */
 lcsx_status lcsx_spmv_bsr(const lcsx_bsr* A, const float* device_x, float* device_y, void* stream);
 
+/* No counterpart in the reference: how many solves of this process on a device took which form
+ * (lcsx_pcg_solve_bsr, its no-alloc form and the solvers'; all give the same bits). counts[0]: one launch,
+ * to its end. counts[1]: began as one launch, but a row has more blocks, or 256 (512) rows name more others,
+ * than it holds. counts[2]: began as one launch, but its workgroups did not all run at once (another process
+ * on the GPU, a stream restricted to some CUs), found after about 0.14 s; the next 1024 solves on the device,
+ * then 2048 and so on, take the launches at once. counts[3]: would have fitted, but another solve was
+ * running in that form or it was such a next one. Solves of 1 to 3 ran as three launches per iteration, as
+ * did the uncounted ones, which the form does not take by their size. */
+lcsx_status lcsx_pcg_form_counts(int device, uint64_t counts[4]);
+
 /* ConjugateGradientSolver::device_solve(stream, func_spmv, func_compute_energy) (precond_cg.h:41-43,
  * precond_cg.cpp:626-771) in its operator form: the caller supplies the product q = A p as a
  * function, the library runs the same block-Jacobi PCG around it (x0 = 0, the safe divisions, the

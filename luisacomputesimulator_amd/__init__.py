@@ -126,6 +126,7 @@ _SIGS = {
                                      C.c_void_p, C.POINTER(lcsx_pcg_result)]),
     "lcsx_pcg_solve_bsr_noalloc": (C.c_int, [C.POINTER(lcsx_bsr), C.c_void_p, C.c_void_p,
                                              C.POINTER(lcsx_pcg_options), C.c_void_p, C.POINTER(lcsx_pcg_result)]),
+    "lcsx_pcg_form_counts": (C.c_int, [C.c_int, C.POINTER(C.c_uint64)]),
     "lcsx_spmv_bsr": (C.c_int, [C.POINTER(lcsx_bsr), C.c_void_p, C.c_void_p, C.c_void_p]),
     "lcsx_pcg_solve_op": (C.c_int, [C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                     C.POINTER(lcsx_pcg_options), C.c_void_p, C.POINTER(lcsx_pcg_result)]),
@@ -484,6 +485,14 @@ def pcg_solve_bsr(system: "BsrSystem", b, max_iters: int = 100, check_every: int
     fn = lib.lcsx_pcg_solve_bsr_noalloc if no_alloc else lib.lcsx_pcg_solve_bsr
     _check(fn(C.byref(system.c), bd.ptr, xd.ptr, C.byref(o), None, C.byref(r)))
     return xd.numpy().reshape(-1, 3), {f: getattr(r, f) for f, _ in lcsx_pcg_result._fields_}
+
+
+def pcg_form_counts(device: int = 0) -> Dict[str, int]:
+    """Solves of this process on a device: in one launch to their end, and as launches because the rows did not
+    fit it, a wait ran out in it, or another solve held it (lcsx_pcg_form_counts)."""
+    c = (C.c_uint64 * 4)()
+    _check(load_library().lcsx_pcg_form_counts(device, c))
+    return dict(zip(("one_launch", "unfit", "waited", "refused"), map(int, c)))
 
 
 def spmv_bsr(system: "BsrSystem", x) -> np.ndarray:

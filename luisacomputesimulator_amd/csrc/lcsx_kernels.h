@@ -50,7 +50,7 @@ struct PcgState
     float    rz[2], rz0;
     uint32_t converged, iters, nan;
     uint32_t bad_index;  // block-CSR solves: a column or row range lies outside the matrix
-    uint32_t fail;       // the one-launch form gave up (lcsx_pcg_grid.h); the solve starts over
+    uint32_t fail;       // the one-launch form gave up (kGridUnfit, kGridWaited); the solve starts over
 };
 
 // SELL-16 block matrix: rows in slices of 16; slice s stores sl_off[s + 1] - sl_off[s] block
@@ -419,8 +419,12 @@ void launch_pcg_update(const PcgArgs& a, hipStream_t s);
 // The PCG in one launch (lcsx_pcg_grid.h): limits, shape and workspace.
 constexpr uint32_t kGridRows    = 4096;  // rows whose p a workgroup holds: its own and those its columns name
 constexpr uint32_t kGridOwn     = 512;   // own rows of a workgroup
-constexpr uint32_t kGridWgs     = 256;   // workgroups of a launch: one per CU
+constexpr uint32_t kGridWgs     = 256;   // most workgroups of a launch: one per CU of the GPU (grid_wgs)
 constexpr uint32_t kGridThreads = 512;
+constexpr uint32_t kGridPolls   = 200000;  // polls of one wait (about 0.7 us each)
+// Why a launch gave up: a row has more blocks, or a workgroup names more rows, than the shape holds; or a
+// wait ran out.
+constexpr uint32_t kGridUnfit = 1, kGridWaited = 2;
 struct GridSync
 {
     unsigned long long* rz;    // words, zero before the first launch: one per row block,
@@ -428,26 +432,41 @@ struct GridSync
     unsigned long long* zx;    // and three per row: z as it is exchanged
     const uint2*        tab;   // per workgroup: its scene and its place in it (null: one scene)
     uint32_t            epoch; // of the launch's first iteration (from 2); later launches use later ones
+    uint32_t            polls; // of one wait before the launch gives up
 };
 struct GridPlan
 {
     int U = 0, K = 0;  // row groups per thread and blocks per thread and row (0: the launches are used)
     uint32_t row_blocks() const { return (uint32_t)U * kGridThreads / 1024u; }  // of a workgroup
 };
-// The shape for scenes of up to n_rb_most row blocks, n_rb in all, of at most `width` blocks a row.
-GridPlan grid_plan(uint32_t n_rb_most, uint32_t n_rb, uint32_t width);
+// Workgroups that a launch may have on a device: its CUs, at most kGridWgs (0: none, as with no device).
+uint32_t grid_wgs(int device);
+// The shape for scenes of up to n_rb_most row blocks, n_rb in all, of at most `width` blocks a row, in
+// launches of up to `wgs` workgroups.
+GridPlan grid_plan(uint32_t n_rb_most, uint32_t n_rb, uint32_t width, uint32_t wgs);
 // Iterations [a.k, a.k + len) of a solve begun by launch_pcg_init, on `wgs` workgroups.
 void launch_pcg_grid(const GridPlan& p, unsigned wgs, const PcgArgs& a, const SellView& A, const ContactView& c,
                      const VertContacts& vc, const GridSync& g, uint32_t len, hipStream_t s);
 void launch_grid_clear(unsigned long long* words, size_t n, hipStream_t s);
 // One such launch runs at a time per GPU in a process (its workgroups wait for each other, so all
-// must be resident); without the lease a solve uses the launches, which give the same bits.
+// must be resident); without the lease a solve uses the launches, which give the same bits. Where a wait has
+// run out (another process holds CUs of the GPU, or the stream may use some of them only) the next solves on
+// that GPU get no lease: 1024 of them, and twice as many after every further wait, since a wait that runs out
+// costs about 0.14 s, as much as a hundred solves.
 struct GridLease
 {
     int  dev = -1;
     bool take(int device);
+    void outcome(uint32_t fail, bool remember = true);  // of the solve (0: it ran to its end)
     ~GridLease();
 };
+// Solves of a device since the process began: in one launch, given up as unfit, given up on a wait, and
+// refused a lease.
+struct GridCounts
+{
+    uint64_t one, unfit, waited, refused;
+};
+GridCounts grid_counts(int device);
 // Mixed precision: FP16 copy of the off-diagonal blocks with a power-of-two scale per block.
 void launch_energy(const EnergyArgs& a, unsigned contact_grid, uint32_t nscenes, hipStream_t s);
 void launch_pack_fp16(uint32_t nslices, uint32_t n, const uint32_t* sl_off, uint32_t nblocks, const float* val,

@@ -2316,7 +2316,7 @@ struct GridContacts
         f3 p[4];
     };
     LCSX_D P4 rows4(const PcgArgs& a, const grid::Word* zx, bool first, uint32_t zep, const float* p_old, float beta,
-                    const uint32_t (&r)[4], uint32_t& bad) const
+                    const uint32_t (&r)[4], uint32_t polls, uint32_t& bad) const
     {
         P4 o;
         if (first)
@@ -2347,7 +2347,7 @@ struct GridContacts
             for (int j = 0; j < 4; j++)
 #pragma unroll
                 for (int d = 0; d < 3; d++) ok = ok && (r[j] == kInvalid || grid::epoch_of(w[j][d]) == zep);
-            if (!ok && tries > grid::kPolls) bad = 1u;
+            if (!ok && tries > polls) bad = 1u;
             if (ok || *(volatile uint32_t*)&bad != 0u)
             {
 #pragma unroll
@@ -2360,9 +2360,9 @@ struct GridContacts
     // The runs of this workgroup's 256-slot chunks and their p.q partials. p of other workgroups' rows
     // is z + beta p_old again, and every slot evaluates its contact's t_c itself (contact_t1's
     // expression, so the same bits): a wait of all workgroups for the t_c would cost more than the
-    // repetition as long as the contacts are few (grid_plan's limit).
+    // repetition as long as the contacts are few (the limit in Solver::pcg_run).
     LCSX_D void slots(const PcgArgs& a, const grid::Word* zx, bool first, uint32_t zep, const float* p_old, float beta,
-                      grid::Word* words, uint32_t epoch, float* sh, uint32_t& bad) const
+                      grid::Word* words, uint32_t epoch, float* sh, uint32_t polls, uint32_t& bad) const
     {
         const uint32_t gpw = blockDim.x >> 8, grp = threadIdx.x >> 8, wv = threadIdx.x >> 6;
         for (uint32_t base = part * gpw; base < nch; base += parts * gpw)
@@ -2382,7 +2382,7 @@ struct GridContacts
                     float          fa[4], fb[4];
                     gdofs4(c, k, 0u, ra, fa);
                     gdofs4(c, k, 1u, rb, fb);
-                    const P4       A = rows4(a, zx, first, zep, p_old, beta, ra, bad);
+                    const P4       A = rows4(a, zx, first, zep, p_old, beta, ra, polls, bad);
                     float          t = fa[0] * dot(nn, A.p[0]);
 #pragma unroll
                     for (int j = 0; j < 4; j++)
@@ -2392,7 +2392,7 @@ struct GridContacts
                     }
                     if (rb[0] != kInvalid || rb[1] != kInvalid || rb[2] != kInvalid || rb[3] != kInvalid)
                     {
-                        const P4 B = rows4(a, zx, first, zep, p_old, beta, rb, bad);
+                        const P4 B = rows4(a, zx, first, zep, p_old, beta, rb, polls, bad);
 #pragma unroll
                         for (int j = 0; j < 4; j++)
                         {
@@ -2841,12 +2841,12 @@ void launch_grid_clear(unsigned long long* w, size_t n, hipStream_t s)
 // more workgroups costs more than the second block's product, and a batch needs half the launches.
 // Blocks per thread and row (K, four threads a row) are what fits 256 registers beside the rows'
 // vectors.
-GridPlan grid_plan(uint32_t n_rb_most, uint32_t n_rb, uint32_t width)
+GridPlan grid_plan(uint32_t n_rb_most, uint32_t n_rb, uint32_t width, uint32_t wgs)
 {
     GridPlan  p;
     const int K = width <= 12u ? 3 : (width <= 16u ? 4 : (width <= 32u ? 8 : 0));
-    const int U = n_rb <= kGridWgs || K > 3 ? 2 : 4;
-    if (K == 0 || n_rb == 0 || n_rb_most > kGridWgs * (uint32_t)(U / 2)) return p;
+    const int U = n_rb <= wgs || K > 3 ? 2 : 4;
+    if (K == 0 || n_rb == 0 || n_rb_most > wgs * (uint32_t)(U / 2)) return p;
     p.U = U;
     p.K = K;
     return p;
@@ -2886,17 +2886,67 @@ void launch_pcg_grid(const GridPlan& p, unsigned wgs, const PcgArgs& a, const Se
 }
 namespace
 {
-std::atomic<bool> g_grid_busy[64];
+constexpr int kGridDevices = 64;
+struct GridDevice
+{
+    std::atomic<bool>     busy{false};
+    std::atomic<uint32_t> cus{0};            // 0: not asked yet
+    std::atomic<uint32_t> skip{0}, back{0};  // solves without a lease still to come, and after the next wait
+    std::atomic<uint64_t> one{0}, unfit{0}, waited{0}, refused{0};
+};
+GridDevice g_grid[kGridDevices];
+}  // namespace
+uint32_t grid_wgs(int device)
+{
+    if (device < 0 || device >= kGridDevices) return 0u;
+    uint32_t cus = g_grid[device].cus.load();
+    if (!cus)
+    {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) return 0u;
+        cus = (uint32_t)n;
+        g_grid[device].cus.store(cus);
+    }
+    return std::min(cus, kGridWgs);
 }
 bool GridLease::take(int device)
 {
-    if (device < 0 || device >= 64 || g_grid_busy[device].exchange(true)) return false;
+    if (device < 0 || device >= kGridDevices) return false;
+    GridDevice& d = g_grid[device];
+    uint32_t    s = d.skip.load();
+    while (s && !d.skip.compare_exchange_weak(s, s - 1u)) {}
+    if (s || d.busy.exchange(true))
+    {
+        d.refused++;
+        return false;
+    }
     dev = device;
     return true;
 }
+void GridLease::outcome(uint32_t fail, bool remember)
+{
+    if (dev < 0) return;
+    GridDevice& d = g_grid[dev];
+    if (!fail) d.one++;
+    else if (fail & kGridUnfit) d.unfit++;
+    else
+    {
+        d.waited++;
+        if (!remember) return;
+        const uint32_t b = std::max(d.back.load(), 1024u);
+        d.skip.store(b);
+        d.back.store(std::min(2u * b, 1u << 20));
+    }
+}
 GridLease::~GridLease()
 {
-    if (dev >= 0) g_grid_busy[dev].store(false);
+    if (dev >= 0) g_grid[dev].busy.store(false);
+}
+GridCounts grid_counts(int device)
+{
+    if (device < 0 || device >= kGridDevices) return GridCounts{};
+    const GridDevice& d = g_grid[device];
+    return GridCounts{d.one.load(), d.unfit.load(), d.waited.load(), d.refused.load()};
 }
 void launch_spmv(const SellView& A, const ContactView& c, const VertContacts& vc, unsigned contact_grid, const float* p,
                  float* y, uint32_t n, hipStream_t s)

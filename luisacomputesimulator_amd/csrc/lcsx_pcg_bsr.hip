@@ -521,11 +521,12 @@ struct GridBsr
 // The shape of the one-launch form. The widest row is not known here: cloth-like matrices have rows
 // of up to one and a half times the mean (a row with more blocks than the shape holds makes the kernel
 // give up before its first iteration).
-GridPlan bsr_plan(const lcsx_bsr* A, uint32_t nb)
+GridPlan bsr_plan(const lcsx_bsr* A, uint32_t nb, uint32_t wgs)
 {
     const double mean = (double)A->nnz / A->n_rows;
     if (A->n_rows > (int)kGridBsrRows) return GridPlan{};
-    return grid_plan(nb, nb, nb > kGridWgs ? (mean <= 12.0 ? 12u : 64u) : (mean <= 12.0 ? 16u : (mean <= 24.0 ? 32u : 64u)));
+    return grid_plan(nb, nb, nb > wgs ? (mean <= 12.0 ? 12u : 64u) : (mean <= 12.0 ? 16u : (mean <= 24.0 ? 32u : 64u)),
+                     wgs);
 }
 void launch_bsr_grid(const GridPlan& p, const lcsx_bsr* A, const BsrWork& w, const lcsx_pcg_options& o, float* x,
                      hipStream_t s)
@@ -546,7 +547,7 @@ void launch_bsr_grid(const GridPlan& p, const lcsx_bsr* A, const BsrWork& w, con
     a.abs_tol     = o.abs_tol;
     a.check_every = (uint32_t)o.check_every;
     const GridBsr  M{A->row_ptr, A->col, A->blocks, A->diag, w.st, (uint32_t)A->nnz};
-    const GridSync g{w.words, w.words + w.nb, w.words + 5u * w.nb, nullptr, 2u};
+    const GridSync g{w.words, w.words + w.nb, w.words + 5u * w.nb, nullptr, 2u, kGridPolls};
     const unsigned wgs = (w.nb + p.row_blocks() - 1u) / p.row_blocks();
     auto go = [&](auto kern) { kern<<<wgs, kGridThreads, 0, s>>>(a, M, NoContacts{}, g, (uint32_t)o.max_iters); };
     if (p.U == 4) go(k_pcg_grid<GridBsr, 4, 3, false, NoContacts>);
@@ -566,8 +567,8 @@ lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_op
     if (one_launch && o.max_iters > 0)
     {
         int dev = 0;
-        gp      = bsr_plan(A, w.nb);
-        if (gp.U && (hipGetDevice(&dev) != hipSuccess || !lease.take(dev))) gp = GridPlan{};
+        if (hipGetDevice(&dev) == hipSuccess) gp = bsr_plan(A, w.nb, grid_wgs(dev));
+        if (gp.U && !lease.take(dev)) gp = GridPlan{};
     }
     k_bsr_init<<<w.nb, kB, 0, s>>>(w, A->diag, b, x);
     LCSX_HIP(hipGetLastError());
@@ -587,6 +588,7 @@ lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_op
         issued += chunk;
         LCSX_HIP(hipMemcpyAsync(&h, w.st, sizeof(BsrState), hipMemcpyDeviceToHost, s));
         LCSX_HIP(hipStreamSynchronize(s));
+        if (gp.U && !h.bad_index) lease.outcome(h.fail);
         if (gp.U && h.fail && !h.bad_index) return solve(A, b, x, o, s, base, res, false);
         if (h.converged || h.bad_index) break;
     }
@@ -667,6 +669,17 @@ extern "C" void lcsx_pcg_options_default(lcsx_pcg_options* o)
     o->check_every = 25;
     o->rel_tol     = 0.0f;
     o->abs_tol     = 1e-10f;
+}
+
+extern "C" lcsx_status lcsx_pcg_form_counts(int device, uint64_t counts[4])
+{
+    if (!counts || device < 0) return arg_error("invalid arguments");
+    const GridCounts g = grid_counts(device);
+    counts[0]          = g.one;
+    counts[1]          = g.unfit;
+    counts[2]          = g.waited;
+    counts[3]          = g.refused;
+    return LCSX_OK;
 }
 
 extern "C" lcsx_status lcsx_pcg_solve_bsr(const lcsx_bsr* A, const float* device_b, float* device_x,

@@ -250,7 +250,7 @@ void Solver::init()
     frame  = 0;
 }
 
-// The one-launch PCG's shape, and the scenes dealt to launches ("rounds") of at most kGridWgs
+// The one-launch PCG's shape, and the scenes dealt to launches ("rounds") of at most grid_wgs
 // workgroups, the largest scenes first into the first round that still holds them. Up to two rounds: a
 // solve takes 1.12 ms in one round of 121,000 rows (1.88 with three launches per iteration), 3.4 ms in two
 // of 236,000 rows (4.0) and as long as the launches, 4.3 ms, in three of 306,000.
@@ -262,7 +262,8 @@ void Solver::plan_grid()
     uint32_t width = 0, most = 0;
     for (size_t k = 0; k + 1 < S.sl_off.size(); k++) width = std::max(width, S.sl_off[k + 1] - S.sl_off[k]);
     for (uint32_t sc = 0; sc < S.nscenes; sc++) most = std::max(most, S.sc_rb0[sc + 1] - S.sc_rb0[sc]);
-    grid_shape = grid_plan(most, S.n_rb, width);
+    const uint32_t limit = grid_wgs(device);
+    grid_shape = grid_plan(most, S.n_rb, width, limit);
     grid_round.clear();
     if (!grid_shape.U) return;
     constexpr size_t kRounds = 2;
@@ -275,7 +276,7 @@ void Solver::plan_grid()
     for (uint32_t sc : order)
     {
         size_t r = 0;
-        while (r < used.size() && used[r] + wgs(sc) > kGridWgs) r++;
+        while (r < used.size() && used[r] + wgs(sc) > limit) r++;
         if (r == used.size()) used.push_back(0u);
         used[r] += wgs(sc);
         round[sc] = (uint32_t)r;
@@ -687,7 +688,7 @@ void Solver::contact_assemble()
 }
 
 int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const VertContacts& vc, int max_iters,
-                    int replace_every)
+                    int replace_every, bool one_launch)
 {
     const uint32_t ns = S.nscenes;
     const unsigned mc = vc.ptr ? max_chunks(vc.nslots) : 0u;
@@ -706,7 +707,7 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     const uint32_t gw = grid_round.empty() ? 0u : grid_round.back();
     const uint32_t grid_chunks = 2u * gw * (kGridThreads / 256u);  // that the words are for
     const uint32_t most_chunks = grid_shape.U == 2 ? grid_chunks : std::min(grid_chunks, ns + gw / (ns == 1u ? 16u : 8u));
-    if (pcg_grid && grid_shape.U && !use_graphs && spmv_sample == 0 && mc <= most_chunks &&
+    if (one_launch && pcg_grid && grid_shape.U && !use_graphs && spmv_sample == 0 && mc <= most_chunks &&
         lease.take(device))
         gp = grid_shape;
     const size_t grid_words = 5 * (size_t)S.n_rb + grid_chunks;
@@ -737,7 +738,8 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
             for (size_t r = 0; r + 1 < grid_round.size(); r++)
             {
                 const uint32_t w0 = grid_round[r];
-                const GridSync g{grid_slots.p, grid_slots.p + S.n_rb, grid_zx.p, ns > 1 ? grid_tab.p + w0 : nullptr, grid_epoch};
+                const GridSync g{grid_slots.p, grid_slots.p + S.n_rb, grid_zx.p, ns > 1 ? grid_tab.p + w0 : nullptr, grid_epoch,
+                                 kGridPolls};
                 launch_pcg_grid(gp, grid_round[r + 1] - w0, b, A, cv, vc, g, (uint32_t)chunk, stream);
             }
             grid_epoch += (uint32_t)chunk;
@@ -825,14 +827,16 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
         }
         LCSX_HIP(hipStreamSynchronize(stream));
         flush_events();
-        bool gave_up = false;
-        for (const PcgState& h : host_pcg) gave_up = gave_up || (gp.U && h.fail);
+        uint32_t gave_up = 0u;
+        for (const PcgState& h : host_pcg) gave_up |= gp.U ? h.fail : 0u;
         if (gave_up)
         {
-            // a wait ran out or the gathered rows do not fit: the launches from the start, from now on
-            pcg_grid = false;
+            // the launches from the start; from now on, if the rows do not fit (the pattern stays what it is)
+            lease.outcome(gave_up);
+            if (gave_up & kGridUnfit) grid_shape = GridPlan{};
             grid_slots.free();
-            return pcg_run(a, A, cv, vc, max_iters, replace_every);
+            if (timing) times["pcg_grid_gave_up"].second += 1;
+            return pcg_run(a, A, cv, vc, max_iters, replace_every, false);
         }
         bool done = true;
         for (const PcgState& h : host_pcg)
@@ -848,6 +852,7 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
         }
         if (done || nan) break;
     }
+    if (gp.U && issued > 0) lease.outcome(0u);
     if (nan)
     {
         set_error("NaN/Inf in the PCG iteration");

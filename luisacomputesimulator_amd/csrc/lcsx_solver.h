@@ -147,7 +147,7 @@ struct Solver
     // residual is replaced by the true one (FP32 blocks) after every replace_every iterations.
     // Returns the iterations run.
     int         pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const VertContacts& vc, int max_iters,
-                        int replace_every);
+                        int replace_every, bool one_launch = true);
     void        account_spmv(uint32_t iters, uint32_t nslots);
     VertContacts vert_contacts();
     unsigned    pair_grid(uint32_t cap) const;

@@ -5,7 +5,7 @@ launches; a solver left alone takes the one-launch form wherever the system fits
 import numpy as np
 import pytest
 
-from luisacomputesimulator_amd import BsrSystem, LcsxError, NewtonSolver, pcg_solve_bsr, scenes
+from luisacomputesimulator_amd import BsrSystem, LcsxError, NewtonSolver, pcg_form_counts, pcg_solve_bsr, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -112,16 +112,43 @@ def banded(n, half, seed):
     return BsrSystem(ptr, c, blocks, diag.astype(np.float32)), (i, c, blocks, diag), rng.normal(size=(n, 3))
 
 
+def counted(fn):
+    """fn's result, and the forms of the PCG that it was counted in."""
+    before = pcg_form_counts()
+    out = fn()
+    return out, {k: v - before[k] for k, v in pcg_form_counts().items() if v != before[k]}
+
+
+def widened(ptr, cols, blocks, diag):
+    """The same system with 40 zero blocks more in its last row: wider than any one-launch shape, so the solve
+    takes the launches, where a zero block adds nothing."""
+    extra = np.arange(40) % (len(ptr) - 1)
+    ptr = ptr.copy()
+    ptr[-1] += len(extra)
+    return BsrSystem(ptr, np.concatenate([cols, extra]), np.concatenate([blocks, np.zeros((40, 3, 3), np.float32)]), diag)
+
+
 # one row, around a row block's and a workgroup's edge, two row blocks per workgroup (above 65536), and
 # rows wider than any shape holds (24 blocks a row above 65536 rows, 40 below)
 @pytest.mark.parametrize("n,half", [(1, 1), (255, 2), (256, 6), (257, 6), (1000, 6), (1025, 11), (65536, 6), (65537, 6),
                                     (131072, 3), (70000, 12), (3000, 20)])
 def test_block_csr_solve(require_gpu, n, half):
     """The residual of 100 iterations against the FP64 recurrence's own, and the solution against the
-    64-bit iterate (1e-4: 100 FP32 iterations of a system of condition below 1e3)."""
+    64-bit iterate (1e-4: 100 FP32 iterations of a system of condition below 1e3). The form that ran, and the
+    launches' bits."""
     sysm, (i, c, blocks, diag), b = banded(n, half, n)
     b = b.astype(np.float32)
-    x, res = pcg_solve_bsr(sysm, b, max_iters=100, check_every=25, abs_tol=0.0)
+    (x, res), form = counted(lambda: pcg_solve_bsr(sysm, b, max_iters=100, check_every=25, abs_tol=0.0))
+    # (the shapes are for a mean of up to 24 blocks a row, or 12 above 65,536 rows)
+    one = len(c) <= (24 if n <= 65536 else 12) * n
+    assert form == ({"one_launch": 1} if one else {})
+    if one:
+        ptr = np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))])
+        wide = widened(ptr, c, blocks, diag.astype(np.float32))
+        (y, launched), form = counted(lambda: pcg_solve_bsr(wide, b, max_iters=100, check_every=25, abs_tol=0.0))
+        # (40 blocks more in a tiny matrix are more than any shape's mean)
+        assert form == ({"unfit": 1} if len(c) + 40 <= (24 if n <= 65536 else 12) * n else {})
+        assert np.array_equal(x, y) and res == launched
     B, D, inv = blocks.astype(np.float64), diag.astype(np.float32).astype(np.float64), None
     inv = np.linalg.inv(D)
 
@@ -155,15 +182,6 @@ def named_rows(ptr, cols, rows):
     return most
 
 
-def widened(ptr, cols, blocks, diag):
-    """The same system with 40 zero blocks more in its last row: wider than any one-launch shape, so the solve
-    takes the launches, where a zero block adds nothing."""
-    extra = np.arange(40) % (len(ptr) - 1)
-    ptr = ptr.copy()
-    ptr[-1] += len(extra)
-    return BsrSystem(ptr, np.concatenate([cols, extra]), np.concatenate([blocks, np.zeros((40, 3, 3), np.float32)]), diag)
-
-
 # columns all over the matrix: a workgroup of 256 rows holds p of 3,840 others, one of 512 rows (above 65,536
 # rows) of 3,584; the last two fit
 @pytest.mark.parametrize("n,width,fits", [(60000, 20, False), (100000, 10, False), (20000, 14, True), (70000, 6, True)])
@@ -184,7 +202,8 @@ def test_block_csr_scattered_columns(require_gpu, n, width, fits):
     diag = np.tile(np.eye(3, dtype=np.float32), (n, 1, 1))
     b = rng.normal(size=(n, 3)).astype(np.float32)
     opt = dict(max_iters=4, check_every=4, abs_tol=0.0)
-    x, res = pcg_solve_bsr(BsrSystem(ptr, c, blocks, diag), b, **opt)
+    (x, res), form = counted(lambda: pcg_solve_bsr(BsrSystem(ptr, c, blocks, diag), b, **opt))
+    assert form == ({"one_launch": 1} if fits else {"unfit": 1})
     assert res["iters"] == 4 and np.isfinite(x).all()
     y, launched = pcg_solve_bsr(widened(ptr, c, blocks, diag), b, **opt)
     assert np.array_equal(x, y) and res == launched
@@ -216,7 +235,7 @@ def test_shuffled_cloth_takes_the_launches(require_gpu):
     for g in (one, launches):
         g.physics_step_gpu(1)
     assert one.stats()["pcg_iters_total"] == launches.stats()["pcg_iters_total"]
-    assert one.kernel_times()["pcg_grid"][1] == 1
+    assert one.kernel_times()["pcg_grid"][1] == 1 and one.kernel_times()["pcg_grid_gave_up"][1] == 1
     assert np.array_equal(one.get_simulation_results(), launches.get_simulation_results())
 
 
