@@ -278,15 +278,22 @@ lcsx_status lcsx_solver_kernel_times(lcsx_solver* s, char* buf, size_t buf_len, 
  * around it, which is why level 2 samples. */
 lcsx_status lcsx_solver_set_timing(lcsx_solver* s, int level);
 /* PCG launch mode (no counterpart in the reference, whose backend records its own command
- * lists). A solver on which neither this nor lcsx_solver_set_spmv_shape was called runs a solve of one
- * scene as a single launch where the system fits (up to 131,072 rows of at most 12 blocks, 65,536 of at
- * most 32, and contacts that are few beside the rows), otherwise as three launches per iteration. This
- * call selects the launches: 1 captures each convergence-test interval of PCG iterations as a hipGraph
- * and replays it; 0 launches every kernel directly. Every form adds up the same terms in the same
- * order. On MI355X the replay does not shorten the device time of a solve (the gaps between
+ * lists). A solver on which neither this nor lcsx_solver_set_spmv_shape was called runs a solve as a
+ * single launch where the system fits (lcsx_solver_set_one_launch), otherwise as three launches per
+ * iteration. This call selects the launches: 1 captures each convergence-test interval of PCG iterations
+ * as a hipGraph and replays it; 0 launches every kernel directly. Every form adds up the same terms in the
+ * same order. On MI355X the replay does not shorten the device time of a solve (the gaps between
  * dependent kernels remain) and each new chunk shape costs a capture. Timing level 2 always launches
  * directly (its events are attached to the SpMV launches). */
 lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on);
+/* The PCG in one launch (no counterpart in the reference). on 1, the default: a solve runs as a single
+ * launch where the system fits (a scene of up to 131,072 rows of at most 12 blocks or 65,536 of at most 32,
+ * a batch in up to two such launches, and contacts that are few beside the rows), whatever
+ * lcsx_solver_set_graphs and lcsx_solver_set_spmv_shape say of the solves that do not; this takes back
+ * their choice of the launches. 0: launches only. polls bounds each wait of its workgroups for each other,
+ * at about 0.7 us a poll (0: 200,000); past it the solve starts over as launches. With another bound than
+ * the default the solver keeps to the launches after that, until this is called again. */
+lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on, uint32_t polls);
 /* LBVH traversal shape of the solver's broad-phase queries (no counterpart in the reference; the
  * same pairs in every shape). Binary steps (one 64 B record, two children tested per step, the
  * reference's 32-entry stack): 0 keeps the whole stack in LDS and stages 256 pairs per wavefront

@@ -785,6 +785,14 @@ lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on)
     return LCSX_OK;
 }
 
+lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on, uint32_t polls)
+{
+    if (!s || (on != 0 && on != 1)) return arg_error("invalid arguments");
+    s->s.pcg_grid   = on == 1;
+    s->s.grid_polls = polls ? polls : kGridPolls;
+    return LCSX_OK;
+}
+
 lcsx_status lcsx_solver_set_query_shape(lcsx_solver* s, int shape)
 {
     if (!s || shape < 0 || shape >= kQueryVariants) return arg_error("invalid arguments");

@@ -256,7 +256,6 @@ void Solver::init()
 // of 236,000 rows (4.0) and as long as the launches, 4.3 ms, in three of 306,000.
 void Solver::plan_grid()
 {
-    pcg_grid = true;
     grid_slots.free();
     grid_zx.free();
     uint32_t width = 0, most = 0;
@@ -707,7 +706,7 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     const uint32_t gw = grid_round.empty() ? 0u : grid_round.back();
     const uint32_t grid_chunks = 2u * gw * (kGridThreads / 256u);  // that the words are for
     const uint32_t most_chunks = grid_shape.U == 2 ? grid_chunks : std::min(grid_chunks, ns + gw / (ns == 1u ? 16u : 8u));
-    if (one_launch && pcg_grid && grid_shape.U && !use_graphs && spmv_sample == 0 && mc <= most_chunks &&
+    if (one_launch && pcg_grid && grid_shape.U && spmv_sample == 0 && mc <= most_chunks &&
         lease.take(device))
         gp = grid_shape;
     const size_t grid_words = 5 * (size_t)S.n_rb + grid_chunks;
@@ -739,7 +738,7 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
             {
                 const uint32_t w0 = grid_round[r];
                 const GridSync g{grid_slots.p, grid_slots.p + S.n_rb, grid_zx.p, ns > 1 ? grid_tab.p + w0 : nullptr, grid_epoch,
-                                 kGridPolls};
+                                 grid_polls};
                 launch_pcg_grid(gp, grid_round[r + 1] - w0, b, A, cv, vc, g, (uint32_t)chunk, stream);
             }
             grid_epoch += (uint32_t)chunk;
@@ -831,9 +830,11 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
         for (const PcgState& h : host_pcg) gave_up |= gp.U ? h.fail : 0u;
         if (gave_up)
         {
-            // the launches from the start; from now on, if the rows do not fit (the pattern stays what it is)
-            lease.outcome(gave_up);
+            // the launches from the start; from now on, if the rows do not fit (the pattern stays what it is) or
+            // a wait of the caller's bound ran out (which says nothing about the device)
+            lease.outcome(gave_up, grid_polls == kGridPolls);
             if (gave_up & kGridUnfit) grid_shape = GridPlan{};
+            else if (grid_polls != kGridPolls) pcg_grid = false;
             grid_slots.free();
             if (timing) times["pcg_grid_gave_up"].second += 1;
             return pcg_run(a, A, cv, vc, max_iters, replace_every, false);

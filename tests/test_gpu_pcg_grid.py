@@ -79,6 +79,75 @@ def batch(sizes):
             scenes.cloth_on_sphere(n, 0.02, -0.01, seed=k, sphere_subdiv=2, height=0.3015) for k, n in enumerate(sizes)]
 
 
+def test_forms_of_the_launches_and_back(require_gpu):
+    """set_graphs and set_spmv_shape choose the launches, before or after the solver is initialised, and
+    set_one_launch the default form again; with graphs the solves that fit run in one launch all the same."""
+    def forms(g):
+        return set(counted(lambda: g.physics_step_gpu(1))[1])
+
+    g = NewtonSolver.from_scene(scenes.square_cloth(17))
+    assert forms(g) == {"one_launch"}
+    for choose in (lambda: g.set_graphs(False), lambda: g.set_spmv_shape(3), lambda: g.set_one_launch(False),
+                   lambda: g.set_graphs(True)):
+        choose()
+        assert forms(g) == set()
+        g.set_one_launch()
+        assert forms(g) == {"one_launch"}
+    sc = scenes.square_cloth(17)
+    h = NewtonSolver(sc.params)
+    mid = h.register_mesh("square", sc.meshes[0].verts, sc.meshes[0].tris, sc.meshes[0].material)
+    h.set_graphs(False)
+    h.init_solver()
+    assert mid == 0 and forms(h) == set()
+    with pytest.raises(LcsxError):
+        g.set_one_launch(2)
+
+
+@pytest.mark.parametrize("name", ["square_33", "tube_contact"])
+def test_a_wait_that_runs_out_starts_over(require_gpu, name):
+    """Waits bounded to one poll run out at once; the solve is the launches' then, bit for bit, and the solver
+    keeps to them until it is told otherwise. Other solvers are not kept from the form."""
+    a, b, c = (NewtonSolver.from_scene(CASES[name][0]()) for _ in range(3))
+    a.set_one_launch(True, 1)
+    b.set_graphs(False)
+    (_, forms), _ = counted(lambda: a.physics_step_gpu(1)), b.physics_step_gpu(1)
+    assert forms == {"waited": 1} and a.kernel_times()["pcg_grid_gave_up"][1] == 1
+    assert np.array_equal(a.get_simulation_results(), b.get_simulation_results())
+    assert set(counted(lambda: c.physics_step_gpu(1))[1]) == {"one_launch"}
+    a.set_one_launch()
+    assert set(counted(lambda: a.physics_step_gpu(1))[1]) == {"one_launch"}
+    b.physics_step_gpu(1)
+    assert np.array_equal(a.get_simulation_results(), b.get_simulation_results())
+
+
+def test_a_refused_lease_takes_the_launches(require_gpu):
+    """While another solve of the process holds the device's one-launch form (its lease is taken here through the
+    library's C++ symbols), solvers' and block-CSR solves run as launches, with the same bits."""
+    import ctypes as C
+
+    from luisacomputesimulator_amd import load_library
+
+    lib = load_library()
+    take, drop = lib._ZN4lcsx9GridLease4takeEi, lib._ZN4lcsx9GridLeaseD1Ev
+    take.restype, take.argtypes, drop.restype, drop.argtypes = C.c_bool, [C.c_void_p, C.c_int], None, [C.c_void_p]
+    sysm, _, b = banded(1000, 6, 3)
+    solve = lambda: pcg_solve_bsr(sysm, b.astype(np.float32), max_iters=60, check_every=1, abs_tol=0.0)
+    (x, res), form = counted(solve)
+    assert form == {"one_launch": 1}
+    g, h = (NewtonSolver.from_scene(CASES["tube_contact"][0]()) for _ in range(2))
+    g.physics_step_gpu(1)
+    lease = C.c_int(-1)
+    assert take(C.byref(lease), 0)
+    try:
+        (y, launched), form = counted(solve)
+        _, forms = counted(lambda: h.physics_step_gpu(1))
+    finally:
+        drop(C.byref(lease))
+    assert form == {"refused": 1} and set(forms) == {"refused"}
+    assert np.array_equal(x, y) and res == launched
+    assert np.array_equal(g.get_simulation_results(), h.get_simulation_results())
+
+
 # scenes of unequal sizes in one launch, scenes dealt to two, and more rows than two launches hold
 @pytest.mark.parametrize("sizes,one_launch", [((2, 9, 33, 17, 24), True), ((220, 33, 220, 221), True),
                                               ((220,) * 6, False)])
