@@ -6,6 +6,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <optional>
 
 namespace lcsx
 {
@@ -1490,7 +1491,9 @@ void Solver::spmv_dx(bool lp)
 // launch mode (direct or captured graphs), with one scene the form of the contact t_c kernel (one
 // thread per contact or per slot chunk), the SpMV mapping and the broad-phase traversal shape.
 // None of them changes a result: the step bound is a minimum over the same pairs, and the PCG
-// runs the same arithmetic. The state
+// runs the same arithmetic. The PCG's settings are those of its launches and are timed as launches, also
+// where the present system would run in one: they are for the solves that do not fit it, and choosing
+// them leaves that rule as it is. The state
 // (positions, velocities, statistics, timings) is restored afterwards.
 std::string Solver::autotune()
 {
@@ -1542,6 +1545,14 @@ std::string Solver::autotune()
         update_contacts(false);
     }
     contact_assemble();
+    struct Launched  // launches only, while this lives
+    {
+        bool&      flag;
+        const bool was;
+        explicit Launched(bool& f) : flag(f), was(f) { f = false; }
+        ~Launched() { flag = was; }
+    };
+    std::optional<Launched> launched(std::in_place, pcg_grid);
     // PCG: launch mode x contact t_c form. A candidate replaces the current setting only when it
     // is faster by more than kTuneMargin (timings repeat to within ~2%)
     constexpr float kTuneMargin = 0.97f;
@@ -1593,6 +1604,7 @@ std::string Solver::autotune()
         }
         spmv_shape = best < kTuneMargin * cur ? sb : s0;
     }
+    launched.reset();
     pcg();
     // line search: CCD first-pass budget
     if (prm.use_ccd_linesearch && prm.use_self_collision)

@@ -3,7 +3,7 @@ solver's state, so a tuned solver's frames equal an untuned one's."""
 import numpy as np
 import pytest
 
-from luisacomputesimulator_amd import NewtonSolver, scenes
+from luisacomputesimulator_amd import NewtonSolver, pcg_form_counts, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +59,25 @@ def test_autotune_times_one_shape_of_the_solvers_hierarchies(require_gpu, shape)
     timed = [int(k.split("=")[1][:-1]) for k in rep if k.startswith("line_search[query=")]
     print(f"[gpu-autotune] shapes timed {timed}, chosen {rep['chosen']['query']}", flush=True)
     assert timed == list(range(7)) + [shape] and rep["chosen"]["query"] in timed
+
+
+def test_autotune_times_the_launches_and_keeps_the_one_launch(require_gpu):
+    """The PCG's tuned settings are the launches': no candidate runs in one launch (the line search's state takes
+    one solve after them), and whatever is chosen, the next frame's solves do."""
+    g = NewtonSolver.from_scene(scenes.square_cloth(33))
+    g.physics_step_gpu(1)
+    before = pcg_form_counts()
+    rep = g.autotune()
+    tuned = pcg_form_counts()
+    g.physics_step_gpu(1)
+    after = pcg_form_counts()
+    print(f"[gpu-autotune] chosen {rep['chosen']}, counts {before} {tuned} {after}", flush=True)
+    assert tuned["one_launch"] - before["one_launch"] == 1
+    assert after["one_launch"] - tuned["one_launch"] == g.stats()["newton_iters"]
+    assert all(tuned[k] == before[k] == after[k] for k in ("unfit", "waited", "refused"))
+    h = NewtonSolver.from_scene(scenes.square_cloth(17))
+    h.set_graphs(False)  # a choice of the launches stays one
+    h.physics_step_gpu(1)
+    h.autotune()
+    h.physics_step_gpu(1)
+    assert pcg_form_counts() == after
