@@ -711,7 +711,8 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
         lease.take(device))
         gp = grid_shape;
     const size_t grid_words = 5 * (size_t)S.n_rb + grid_chunks;
-    if (gp.U && (!grid_slots.p || grid_epoch > 0xf0000000u))
+    // (a solve's epochs stay below kPoison, whatever its cap)
+    if (gp.U && (!grid_slots.p || (uint64_t)grid_epoch + (uint64_t)std::max(max_iters, 0) > 0xfffffff0u))
     {
         if (!grid_slots.p) grid_slots.alloc(grid_words);
         if (!grid_zx.p) grid_zx.alloc(3 * (size_t)S.nv);

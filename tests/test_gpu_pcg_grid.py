@@ -120,6 +120,30 @@ def test_a_wait_that_runs_out_starts_over(require_gpu, name):
     assert np.array_equal(a.get_simulation_results(), b.get_simulation_results())
 
 
+def test_an_iteration_cap_of_all_integers(require_gpu):
+    """pcg_iter_count as a program sets it that wants no cap: every solve takes as many epochs of the exchanged
+    words as its cap, so they are cleared before the numbers run out. Two solves without contacts, whose numbers
+    end a wrap, then one with contacts (words that no solve has written yet), and again."""
+    def solver(cap):
+        sc = tube_on_ring()
+        sc.params.pcg_iter_count, sc.params.pcg_check_every, sc.params.pcg_rel_tol = cap, 1, 1e-3
+        return NewtonSolver.from_scene(sc)
+
+    a, b = solver(2 ** 31 - 1), solver(1000)
+    b.set_graphs(False)
+    for rep in range(3):
+        for s in ("frame_begin", "predict", "iter_begin", "material", "pcg", "pcg", "update_contacts", "contact_assemble",
+                  "pcg"):
+            b.stage(s)
+            assert b.stats()["pcg_iters"] < 1000  # so does a, whose iterations are the same
+            _, form = counted(lambda: a.stage(s))
+            assert form == ({"one_launch": 1} if s == "pcg" else {})
+            assert s != "pcg" or np.array_equal(a.read("dx"), b.read("dx")), rep
+        contacts = len(b.read("contact_idx")) // 4
+        print(f"[gpu-grid] cap 2^31 - 1: {b.stats()['pcg_iters']} iterations, {contacts} contacts", flush=True)
+        assert contacts > 0
+
+
 def test_a_refused_lease_takes_the_launches(require_gpu):
     """While another solve of the process holds the device's one-launch form (its lease is taken here through the
     library's C++ symbols), solvers' and block-CSR solves run as launches, with the same bits."""
