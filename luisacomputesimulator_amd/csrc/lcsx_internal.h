@@ -138,8 +138,8 @@ void     launch_scan_excl_u32(const uint32_t* in, uint32_t* out, uint32_t n, uin
 
 // Stable LSD radix sort of n entries by the key pair (hi, lo), moving a 32-bit value along: lo, hi
 // and val are ping-pong pairs of n-entry buffers, sorted on their low lo_bits / hi_bits bits;
-// hist holds sort_hist_words(n) words, tmp scan_tmp_words(sort_hist_words(n)). Returns the index
-// (0 or 1) of the buffers that hold the result.
+// hist holds sort_hist_words(n) words, tmp scan_tmp_words(sort_hist_words(n)), or those of a larger n
+// (neither shrinks as n grows). Returns the index (0 or 1) of the buffers that hold the result.
 uint32_t sort_hist_words(uint32_t n);
 int      launch_sort_key_pairs(uint32_t* lo[2], uint32_t* hi[2], uint32_t* val[2], uint32_t n, int lo_bits, int hi_bits,
                                uint32_t* hist, uint32_t* tmp, hipStream_t s);

@@ -6,6 +6,7 @@
 // and copies keys twice per tree and frame), the refit climbs subtrees of up to 1024 leaves in LDS
 // instead of the whole tree with a float-flag spin protocol, and pair lists are appended with one
 // atomic per staged batch.
+#include <algorithm>
 #include "lcsx_internal.h"
 #include "lcsx_physics.h"
 
@@ -320,7 +321,8 @@ __global__ __launch_bounds__(1024) void k_build_small(uint32_t n, uint32_t ni, i
 // Keys per thread of a pass over n keys: a tile's rounds are serial, so few keys want small tiles
 // (187,088 leaves: 17 us a scatter with 16 keys per thread in 46 workgroups, 10 us with 8 in 92), as
 // long as one workgroup can still scan the tiles' counts.
-int sort_items(uint32_t n) { return n <= 65536u ? 4 : (n <= 294912u ? 8 : kSortItems); }
+constexpr uint32_t kSort4 = 65536, kSort8 = 294912;  // most keys with 4 and with 8 per thread
+int sort_items(uint32_t n) { return n <= kSort4 ? 4 : (n <= kSort8 ? 8 : kSortItems); }
 
 // Histogram of the digit (dig >> shift) & 255 per tile.
 template <int kItems>
@@ -1966,8 +1968,12 @@ void Lbvh::refit(const float* x0, const float* x1, const float* pad, hipStream_t
 
 uint32_t sort_hist_words(uint32_t n)
 {
-    const uint32_t tile = (uint32_t)(kBlock * sort_items(n));
-    return 256u * ((n + tile - 1u) / tile) + 1u;
+    // for any count up to n: a count with smaller tiles has more of them
+    auto words = [](uint32_t k) {
+        const uint32_t tile = (uint32_t)(kBlock * sort_items(k));
+        return 256u * ((k + tile - 1u) / tile) + 1u;
+    };
+    return std::max({words(n), words(std::min(n, kSort4)), words(std::min(n, kSort8))});
 }
 
 int launch_sort_key_pairs(uint32_t* lo[2], uint32_t* hi[2], uint32_t* val[2], uint32_t n, int lo_bits, int hi_bits,
