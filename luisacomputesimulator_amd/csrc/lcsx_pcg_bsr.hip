@@ -518,9 +518,11 @@ struct GridBsr
     }
 };
 
-// The shape of the one-launch form. The widest row is not known here: cloth-like matrices have rows
-// of up to one and a half times the mean (a row with more blocks than the shape holds makes the kernel
-// give up before its first iteration).
+// The shape of the one-launch form. The widest row is not known here (the row pointers are on the device, and
+// waiting for a count of them would cost every solve 12 us): cloth-like matrices have rows of up to one and
+// a half times the mean. A row with more blocks than the shape holds, or columns that name more rows, make the
+// kernel give up before its first iteration, which costs such a solve 25-40 us (8 iterations of 1,089 rows:
+// 176 us, 150 as launches at once, 65 where the rows fit; of 88,209 rows: 294, 260 and 137).
 GridPlan bsr_plan(const lcsx_bsr* A, uint32_t nb, uint32_t wgs)
 {
     const double mean = (double)A->nnz / A->n_rows;
@@ -558,13 +560,13 @@ void launch_bsr_grid(const GridPlan& p, const lcsx_bsr* A, const BsrWork& w, con
 
 // The solve on scratch `base` (work_floats(n) floats, 256-byte aligned).
 lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_options& o, hipStream_t s, float* base,
-                  lcsx_pcg_result* res, bool one_launch = true)
+                  lcsx_pcg_result* res)
 {
     const BsrWork  w  = carve(base, (uint32_t)A->n_rows);
     const float    rel2 = o.rel_tol * o.rel_tol;
     GridPlan       gp;
     GridLease      lease;
-    if (one_launch && o.max_iters > 0)
+    if (o.max_iters > 0)
     {
         int dev = 0;
         if (hipGetDevice(&dev) == hipSuccess) gp = bsr_plan(A, w.nb, grid_wgs(dev));
@@ -588,9 +590,21 @@ lcsx_status solve(const lcsx_bsr* A, const float* b, float* x, const lcsx_pcg_op
         issued += chunk;
         LCSX_HIP(hipMemcpyAsync(&h, w.st, sizeof(BsrState), hipMemcpyDeviceToHost, s));
         LCSX_HIP(hipStreamSynchronize(s));
-        if (gp.U && !h.bad_index) lease.outcome(h.fail);
-        if (gp.U && h.fail && !h.bad_index) return solve(A, b, x, o, s, base, res, false);
-        if (h.converged || h.bad_index) break;
+        if (h.bad_index) break;
+        if (gp.U)
+        {
+            lease.outcome(h.fail);
+            if (h.fail)
+            {
+                // From the start, as launches. What does not fit is found before the first update, so the vectors
+                // are still the init's (unless a wait ran out: some workgroups may have ended before it).
+                if (!(h.fail & kGridUnfit)) k_bsr_init<<<w.nb, kB, 0, s>>>(w, A->diag, b, x);
+                gp     = GridPlan{};
+                issued = 0;
+                continue;
+            }
+        }
+        if (h.converged) break;
     }
     if (h.bad_index) return arg_error("a block column or row range is outside the matrix");
     if (h.nan)
