@@ -54,8 +54,9 @@ struct EventPool
         }
     }
 };
+// per thread, as solvers may run in several at once
 thread_local EventPool* g_pool = nullptr;
-hipEvent_t              g_open = nullptr;
+thread_local hipEvent_t g_open = nullptr;
 }  // namespace
 
 Solver::~Solver()
