@@ -32,7 +32,8 @@ def tube_on_ring():
     return sc
 
 
-# rows: less than one 64-row chunk, one row past it, several workgroups, many
+# rows: less than one 64-row chunk, one row past it, several workgroups, many, and above 65,536 rows (two row
+# blocks per workgroup) without and with contacts
 CASES = {
     "square_7": (lambda: scenes.square_cloth(7), 3),
     "square_33": (lambda: scenes.square_cloth(33), 3),
@@ -42,6 +43,8 @@ CASES = {
     "tube_41x48": (lambda: scenes.cylinder_tube(rings=41, per_ring=48, cyl_segments=24, cyl_rings=9), 5),
     "tube_contact": (tube_on_ring, 2),
     "boxes": (boxes, 4),
+    "square_257": (lambda: scenes.square_cloth(257), 1),
+    "sphere_257": (lambda: scenes.cloth_on_sphere(257, 0.02, -0.01, seed=4, sphere_subdiv=2, height=0.3015), 2),
 }
 
 
@@ -59,8 +62,11 @@ def test_one_launch_equals_launches(require_gpu, name, precision):
     launches.set_graphs(False)
     contacts = 0
     for f in range(frames):
-        one.physics_step_gpu(1)
+        _, form = counted(lambda: one.physics_step_gpu(1))
         launches.physics_step_gpu(1)
+        assert set(form) <= {"one_launch"}
+        # (the tubes' later frames have more contacts than it takes)
+        assert form == {"one_launch": one.stats()["newton_iters"]} or (name in ("tube_41x48", "tube_contact") and f > 0)
         a, b = one.stats(), launches.stats()
         contacts = max(contacts, a["num_contacts"])
         print(f"[gpu-grid] {name} {precision} frame {f}: Newton {a['newton_iters']}/{b['newton_iters']}, "
@@ -70,7 +76,7 @@ def test_one_launch_equals_launches(require_gpu, name, precision):
         assert np.array_equal(one.get_simulation_results(), launches.get_simulation_results())
         assert np.array_equal(one.get_velocities(), launches.get_velocities())
     assert one.kernel_times()["pcg_grid"][1] > 0 and "pcg_grid" not in launches.kernel_times()
-    if name in ("tube_contact", "sphere_24", "boxes"):
+    if name in ("tube_contact", "sphere_24", "boxes", "sphere_257"):
         assert contacts > 0
 
 
@@ -178,14 +184,15 @@ def test_a_refused_lease_takes_the_launches(require_gpu):
 def test_batch_one_launch_equals_launches(require_gpu, sizes, one_launch):
     one, launches = (NewtonSolver.from_scenes(batch(sizes)) for _ in range(2))
     launches.set_graphs(False)
-    frames = 4 if max(sizes) < 100 else 1
+    frames, contacts = 4 if max(sizes) < 100 else 1, 0
     for f in range(frames):
         one.physics_step_gpu(1)
         launches.physics_step_gpu(1)
-        print(f"[gpu-grid] batch {sizes} frame {f}: {one.stats()['pcg_iters_total']}", flush=True)
+        contacts = max(contacts, one.stats()["num_contacts"])
+        print(f"[gpu-grid] batch {sizes} frame {f}: {one.stats()['pcg_iters_total']}, {contacts} contacts", flush=True)
         assert one.stats()["pcg_iters_total"] == launches.stats()["pcg_iters_total"]
         assert np.array_equal(one.get_simulation_results(), launches.get_simulation_results())
-    assert ("pcg_grid" in one.kernel_times()) == one_launch
+    assert contacts > 0 and ("pcg_grid" in one.kernel_times()) == one_launch
 
 
 def banded(n, half, seed):
