@@ -290,10 +290,8 @@ lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on);
  * launch where the system fits (a scene of up to 131,072 rows of at most 12 blocks or 65,536 of at most 32,
  * a batch in up to two such launches, and contacts that are few beside the rows), whatever
  * lcsx_solver_set_graphs and lcsx_solver_set_spmv_shape say of the solves that do not; this takes back
- * their choice of the launches. 0: launches only. polls bounds each wait of its workgroups for each other,
- * at about 0.7 us a poll (0: 200,000); past it the solve starts over as launches. With another bound than
- * the default the solver keeps to the launches after that, until this is called again. */
-lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on, uint32_t polls);
+ * their choice of the launches. 0: launches only. */
+lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on);
 /* LBVH traversal shape of the solver's broad-phase queries (no counterpart in the reference; the
  * same pairs in every shape). Binary steps (one 64 B record, two children tested per step, the
  * reference's 32-entry stack): 0 keeps the whole stack in LDS and stages 256 pairs per wavefront

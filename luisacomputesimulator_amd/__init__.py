@@ -107,7 +107,7 @@ _SIGS = {
     "lcsx_solver_kernel_times": (C.c_int, [C.c_void_p, C.c_char_p, C.c_size_t, C.c_int]),
     "lcsx_solver_set_timing": (C.c_int, [C.c_void_p, C.c_int]),
     "lcsx_solver_set_graphs": (C.c_int, [C.c_void_p, C.c_int]),
-    "lcsx_solver_set_one_launch": (C.c_int, [C.c_void_p, C.c_int, C.c_uint32]),
+    "lcsx_solver_set_one_launch": (C.c_int, [C.c_void_p, C.c_int]),
     "lcsx_solver_set_query_shape": (C.c_int, [C.c_void_p, C.c_int]),
     "lcsx_solver_set_spmv_shape": (C.c_int, [C.c_void_p, C.c_int]),
     "lcsx_solver_save_state": (C.c_int, [C.c_void_p, C.c_char_p]),
@@ -403,10 +403,10 @@ class NewtonSolver:
         """Replay captured hipGraphs of the PCG iterations, or launch each kernel (the default)."""
         _check(self.lib.lcsx_solver_set_graphs(self.h, int(on)))
 
-    def set_one_launch(self, on: bool = True, polls: int = 0) -> None:
+    def set_one_launch(self, on: bool = True) -> None:
         """The PCG in one launch where the system fits (the default; takes back the choice of the launches by
-        set_graphs and set_spmv_shape), or launches only; polls bounds its waits (0: the default)."""
-        _check(self.lib.lcsx_solver_set_one_launch(self.h, int(on), int(polls)))
+        set_graphs and set_spmv_shape), or launches only."""
+        _check(self.lib.lcsx_solver_set_one_launch(self.h, int(on)))
 
     def set_query_shape(self, shape: int) -> None:
         """Broad-phase traversal shape (0..3 binary steps, 4..6 four-wide steps of the LBVH with

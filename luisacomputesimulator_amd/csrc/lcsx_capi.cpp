@@ -686,6 +686,7 @@ lcsx_status lcsx_solver_run_stage(lcsx_solver* s, const char* stage)
         else if (st == "newton_iteration") S.newton_iteration_until_done();
         else if (st == "post_dist_check") S.post_dist_check();
         else if (st == "shrink_lists") S.alloc_collision(1024u, 1024u, 1024u);  // exercises the growth path
+        else if (st == "withhold_workgroup") S.grid_withhold = true;  // exercises a wait that runs out
         else if (st == "frame_end") S.frame_end();
         else if (st == "step") S.step();
         else if (st == "spmv_dx") S.spmv_dx();
@@ -785,11 +786,10 @@ lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on)
     return LCSX_OK;
 }
 
-lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on, uint32_t polls)
+lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on)
 {
     if (!s || (on != 0 && on != 1)) return arg_error("invalid arguments");
-    s->s.pcg_grid   = on == 1;
-    s->s.grid_polls = polls ? polls : kGridPolls;
+    s->s.pcg_grid = on == 1;
     return LCSX_OK;
 }
 

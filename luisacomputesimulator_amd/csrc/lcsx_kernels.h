@@ -421,7 +421,6 @@ constexpr uint32_t kGridRows    = 4096;  // rows whose p a workgroup holds: its 
 constexpr uint32_t kGridOwn     = 512;   // own rows of a workgroup
 constexpr uint32_t kGridWgs     = 256;   // most workgroups of a launch: one per CU of the GPU (grid_wgs)
 constexpr uint32_t kGridThreads = 512;
-constexpr uint32_t kGridPolls   = 200000;  // polls of one wait (about 0.7 us each)
 // Why a launch gave up: a row has more blocks, or a workgroup names more rows, than the shape holds; or a
 // wait ran out.
 constexpr uint32_t kGridUnfit = 1, kGridWaited = 2;
@@ -432,7 +431,6 @@ struct GridSync
     unsigned long long* zx;    // and three per row: z as it is exchanged
     const uint2*        tab;   // per workgroup: its scene and its place in it (null: one scene)
     uint32_t            epoch; // of the launch's first iteration (from 2); later launches use later ones
-    uint32_t            polls; // of one wait before the launch gives up
 };
 struct GridPlan
 {

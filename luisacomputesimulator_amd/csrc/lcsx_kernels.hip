@@ -2316,7 +2316,7 @@ struct GridContacts
         f3 p[4];
     };
     LCSX_D P4 rows4(const PcgArgs& a, const grid::Word* zx, bool first, uint32_t zep, const float* p_old, float beta,
-                    const uint32_t (&r)[4], uint32_t polls, uint32_t& bad) const
+                    const uint32_t (&r)[4], uint32_t& bad) const
     {
         P4 o;
         if (first)
@@ -2347,7 +2347,7 @@ struct GridContacts
             for (int j = 0; j < 4; j++)
 #pragma unroll
                 for (int d = 0; d < 3; d++) ok = ok && (r[j] == kInvalid || grid::epoch_of(w[j][d]) == zep);
-            if (!ok && tries > polls) bad = 1u;
+            if (!ok && tries > grid::kPolls) bad = 1u;
             if (ok || *(volatile uint32_t*)&bad != 0u)
             {
 #pragma unroll
@@ -2362,7 +2362,7 @@ struct GridContacts
     // expression, so the same bits): a wait of all workgroups for the t_c would cost more than the
     // repetition as long as the contacts are few (the limit in Solver::pcg_run).
     LCSX_D void slots(const PcgArgs& a, const grid::Word* zx, bool first, uint32_t zep, const float* p_old, float beta,
-                      grid::Word* words, uint32_t epoch, float* sh, uint32_t polls, uint32_t& bad) const
+                      grid::Word* words, uint32_t epoch, float* sh, uint32_t& bad) const
     {
         const uint32_t gpw = blockDim.x >> 8, grp = threadIdx.x >> 8, wv = threadIdx.x >> 6;
         for (uint32_t base = part * gpw; base < nch; base += parts * gpw)
@@ -2382,7 +2382,7 @@ struct GridContacts
                     float          fa[4], fb[4];
                     gdofs4(c, k, 0u, ra, fa);
                     gdofs4(c, k, 1u, rb, fb);
-                    const P4       A = rows4(a, zx, first, zep, p_old, beta, ra, polls, bad);
+                    const P4       A = rows4(a, zx, first, zep, p_old, beta, ra, bad);
                     float          t = fa[0] * dot(nn, A.p[0]);
 #pragma unroll
                     for (int j = 0; j < 4; j++)
@@ -2392,7 +2392,7 @@ struct GridContacts
                     }
                     if (rb[0] != kInvalid || rb[1] != kInvalid || rb[2] != kInvalid || rb[3] != kInvalid)
                     {
-                        const P4 B = rows4(a, zx, first, zep, p_old, beta, rb, polls, bad);
+                        const P4 B = rows4(a, zx, first, zep, p_old, beta, rb, bad);
 #pragma unroll
                         for (int j = 0; j < 4; j++)
                         {

@@ -549,7 +549,7 @@ void launch_bsr_grid(const GridPlan& p, const lcsx_bsr* A, const BsrWork& w, con
     a.abs_tol     = o.abs_tol;
     a.check_every = (uint32_t)o.check_every;
     const GridBsr  M{A->row_ptr, A->col, A->blocks, A->diag, w.st, (uint32_t)A->nnz};
-    const GridSync g{w.words, w.words + w.nb, w.words + 5u * w.nb, nullptr, 2u, kGridPolls};
+    const GridSync g{w.words, w.words + w.nb, w.words + 5u * w.nb, nullptr, 2u};
     const unsigned wgs = (w.nb + p.row_blocks() - 1u) / p.row_blocks();
     auto go = [&](auto kern) { kern<<<wgs, kGridThreads, 0, s>>>(a, M, NoContacts{}, g, (uint32_t)o.max_iters); };
     if (p.U == 4) go(k_pcg_grid<GridBsr, 4, 3, false, NoContacts>);

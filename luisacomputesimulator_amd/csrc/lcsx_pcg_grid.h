@@ -27,7 +27,7 @@
 //
 // Waiting: the launch has at most one workgroup per CU (its LDS fills most of one) and the host starts one
 // such launch at a time per GPU in the process, so all workgroups become resident. Every wait is bounded
-// all the same: past g.polls polls a workgroup poisons its words, sets the state's `fail` and returns, and
+// all the same: past kPolls polls a workgroup poisons its words, sets the state's `fail` and returns, and
 // so does every workgroup that reads a poisoned word.
 #pragma once
 #include "lcsx_common.h"
@@ -38,8 +38,10 @@ namespace lcsx
 namespace grid
 {
 constexpr uint32_t kPoison = 0xffffffffu;  // epoch of a word whose workgroup has given up
+constexpr uint32_t kPolls  = 200000;       // polls of one wait (about 0.7 us each)
 constexpr uint32_t kHash   = 8192;         // hash table entries (columns outside the own rows)
 constexpr uint32_t kProbes = 256;
+constexpr uint32_t kUnfit  = 2;  // Lds::bad before the loop
 static_assert(kGridRows * sizeof(float4) >= kHash * 6u, "the hash table lies in the p rows' space");
 
 struct Lds
@@ -58,7 +60,7 @@ struct Lds
     float    q[3 * kGridOwn];
     float    sh[4][8];
     float    red[2][4], cs[8];
-    uint32_t nhalo, bad, bad_tc;
+    uint32_t nhalo, bad, bad_tc;  // bad: kUnfit, or 1 once a wait has failed
 };
 static_assert(sizeof(Lds) <= 160 * 1024, "LDS of one CU");
 
@@ -93,14 +95,14 @@ LCSX_D void st_z(Word* zx, uint32_t n, uint32_t i, f3 v, uint32_t epoch)
     post(zx + n + (size_t)i, v.y, epoch);
     post(zx + 2 * (size_t)n + i, v.z, epoch);
 }
-LCSX_D f3 wait_z(const Word* zx, uint32_t n, uint32_t i, uint32_t epoch, uint32_t polls, uint32_t& bad)
+LCSX_D f3 wait_z(const Word* zx, uint32_t n, uint32_t i, uint32_t epoch, uint32_t& bad)
 {
     for (uint32_t tries = 0;; tries++)
     {
         const Word x = peek(zx + i), y = peek(zx + n + (size_t)i), z = peek(zx + 2 * (size_t)n + i);
         if (epoch_of(x) == epoch && epoch_of(y) == epoch && epoch_of(z) == epoch)
             return mk(value_of(x), value_of(y), value_of(z));
-        if (tries > polls || *(volatile uint32_t*)&bad != 0u)
+        if (tries > kPolls || *(volatile uint32_t*)&bad != 0u)
         {
             bad = 1u;
             return mk(0.0f, 0.0f, 0.0f);
@@ -113,8 +115,7 @@ LCSX_D f3 wait_z(const Word* zx, uint32_t n, uint32_t i, uint32_t epoch, uint32_
 // go to red). Called by the first four wavefronts. L.bad is set when a word was poisoned or the wait ran
 // out.
 template <int kIn>  // words in flight per thread
-LCSX_D void wait_sum(const Word* s0, uint32_t n0, const Word* s1, uint32_t n1, uint32_t epoch, uint32_t polls, Lds& L,
-                     float* red)
+LCSX_D void wait_sum(const Word* s0, uint32_t n0, const Word* s1, uint32_t n1, uint32_t epoch, Lds& L, float* red)
 {
     const uint32_t n = n0 + n1;
     float          v = 0.0f;
@@ -130,7 +131,7 @@ LCSX_D void wait_sum(const Word* s0, uint32_t n0, const Word* s1, uint32_t n1, u
                 const uint32_t i = i0 + 256u * u;
                 w[u]             = i < n ? peek(i < n0 ? s0 + i : s1 + (i - n0)) : (Word)epoch << 32;
             }
-            bool ok = true, gone = ++tries > polls || *(volatile uint32_t*)&L.bad != 0u;
+            bool ok = true, gone = ++tries > kPolls || *(volatile uint32_t*)&L.bad != 0u;
 #pragma unroll
             for (int u = 0; u < kIn; u++)
             {
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
             }
         }
     }
-    if (!good) L.bad = 1u;
+    if (!good) L.bad = kUnfit;
     __syncthreads();
     for (uint32_t h = t; h < kHash; h += T)
         if (L.h.key[h] != kInvalid)
@@ -272,7 +273,6 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
     __syncthreads();
     // more named rows than there is room for: halo holds the first ones only, and none is read
     bool           ok    = L.bad == 0u && L.nhalo <= kGridRows - R;
-    const bool     fits  = ok;
     const uint32_t nhalo = ok ? L.nhalo : 0u;
     if (ok)
     {
@@ -392,10 +392,10 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
         if (t < nc) post(S_pq + 4u * (b0 - rb0) + t, sum4(&L.sh[t / gpw][4u * (t % gpw)]), ep);
         if (CT)
         {
-            ct.slots(a, g.zx, it == 0u, ep - 1u, p_cur, beta, S_ch, ep, L.cs, g.polls, L.bad_tc);
+            ct.slots(a, g.zx, it == 0u, ep - 1u, p_cur, beta, S_ch, ep, L.cs, L.bad_tc);
             __syncthreads();
         }
-        if (t < 256u) wait_sum<4 * U / 2>(S_pq, 4u * nrb, S_ch + ct.first(), ct.chunks(), ep, g.polls, L, L.red[1]);
+        if (t < 256u) wait_sum<4 * U / 2>(S_pq, 4u * nrb, S_ch + ct.first(), ct.chunks(), ep, L, L.red[1]);
         __syncthreads();
         ok = (L.bad | L.bad_tc) == 0u;
         if (!ok) break;
@@ -419,8 +419,8 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
         __syncthreads();
         if (t < nb) post(S_rz + (b0 - rb0) + t, sum4(&L.cs[4u * t]), ep);
         // ---- r.z of all row blocks, and the named rows' z, waited for by the other wavefronts meanwhile
-        if (t < 256u) wait_sum<U / 2>(S_rz, nrb, nullptr, 0u, ep, g.polls, L, L.red[0]);
-        for (uint32_t e = (t + 256u) % T; e < nhalo; e += T) st3(L.z, e, wait_z(g.zx, n, L.halo[e], ep, g.polls, L.bad));
+        if (t < 256u) wait_sum<U / 2>(S_rz, nrb, nullptr, 0u, ep, L, L.red[0]);
+        for (uint32_t e = (t + 256u) % T; e < nhalo; e += T) st3(L.z, e, wait_z(g.zx, n, L.halo[e], ep, L.bad));
         __syncthreads();
         ok = L.bad == 0u;
         if (!ok) break;
@@ -438,7 +438,9 @@ __global__ __launch_bounds__(kGridThreads) void k_pcg_grid(PcgArgs a, Mat A, Con
         if (t == 0)
         {
             ct.poison(S_ch);
-            __hip_atomic_fetch_or(&st->fail, fits ? kGridWaited : kGridUnfit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // (unfit: known before the loop, so the LDS words are still what they were there)
+            const bool unfit = L.bad == kUnfit || L.nhalo > kGridRows - R;
+            __hip_atomic_fetch_or(&st->fail, unfit ? kGridUnfit : kGridWaited, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
     }
@@ -459,7 +461,7 @@ struct NoContacts
     LCSX_D uint32_t first() const { return 0u; }
     LCSX_D uint32_t chunks() const { return 0u; }
     LCSX_D void     slots(const PcgArgs&, const grid::Word*, bool, uint32_t, const float*, float, grid::Word*, uint32_t,
-                          float*, uint32_t, uint32_t&) const
+                          float*, uint32_t&) const
     {
     }
     LCSX_D void poison(grid::Word*) const {}

@@ -740,9 +740,9 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
             for (size_t r = 0; r + 1 < grid_round.size(); r++)
             {
                 const uint32_t w0 = grid_round[r];
-                const GridSync g{grid_slots.p, grid_slots.p + S.n_rb, grid_zx.p, ns > 1 ? grid_tab.p + w0 : nullptr, grid_epoch,
-                                 grid_polls};
-                launch_pcg_grid(gp, grid_round[r + 1] - w0, b, A, cv, vc, g, (uint32_t)chunk, stream);
+                const GridSync g{grid_slots.p, grid_slots.p + S.n_rb, grid_zx.p, ns > 1 ? grid_tab.p + w0 : nullptr, grid_epoch};
+                const uint32_t wgs = grid_round[r + 1] - w0;
+                launch_pcg_grid(gp, grid_withhold && wgs > 1 ? wgs - 1 : wgs, b, A, cv, vc, g, (uint32_t)chunk, stream);
             }
             grid_epoch += (uint32_t)chunk;
             par = (par + chunk) & 1;
@@ -833,11 +833,10 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
         for (const PcgState& h : host_pcg) gave_up |= gp.U ? h.fail : 0u;
         if (gave_up)
         {
-            // the launches from the start; from now on, if the rows do not fit (the pattern stays what it is) or
-            // a wait of the caller's bound ran out (which says nothing about the device)
-            lease.outcome(gave_up, grid_polls == kGridPolls);
+            // the launches from the start; from now on, if the rows do not fit (the pattern stays what it is)
+            lease.outcome(gave_up, !grid_withhold);
+            grid_withhold = false;
             if (gave_up & kGridUnfit) grid_shape = GridPlan{};
-            else if (grid_polls != kGridPolls) pcg_grid = false;
             grid_slots.free();
             if (timing) times["pcg_grid_gave_up"].second += 1;
             return pcg_run(a, A, cv, vc, max_iters, replace_every, false);

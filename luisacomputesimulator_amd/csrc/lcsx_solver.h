@@ -192,7 +192,7 @@ struct Solver
     // PCG in one launch (lcsx_pcg_grid.h), the default where it fits; off while the caller chooses
     // the form of the launches (set_graphs, set_spmv_shape, set_one_launch) or times them
     bool                     pcg_grid = true;
-    uint32_t                 grid_polls = kGridPolls;
+    bool                     grid_withhold = false;  // exercises a wait that runs out: a workgroup is not launched
     GridPlan                 grid_shape;      // U 0: the rows or scenes do not fit
     std::vector<uint32_t>    grid_round;      // workgroups of round r: [grid_round[r], grid_round[r + 1])
     DBuf<uint2>              grid_tab;        // per workgroup: scene, place in it (several scenes)

@@ -109,20 +109,16 @@ def test_forms_of_the_launches_and_back(require_gpu):
         g.set_one_launch(2)
 
 
-@pytest.mark.parametrize("name", ["square_33", "tube_contact"])
+@pytest.mark.parametrize("name", ["square_33", "tube_contact", "square_257"])
 def test_a_wait_that_runs_out_starts_over(require_gpu, name):
-    """Waits bounded to one poll run out at once; the solve is the launches' then, bit for bit, and the solver
-    keeps to them until it is told otherwise. Other solvers are not kept from the form."""
-    a, b, c = (NewtonSolver.from_scene(CASES[name][0]()) for _ in range(3))
-    a.set_one_launch(True, 1)
+    """One workgroup of the first solve is not launched, so the others' waits for it run out and they end (about
+    0.14 s); the solve is the launches' then, bit for bit, and the next ones run in one launch again."""
+    a, b = (NewtonSolver.from_scene(CASES[name][0]()) for _ in range(2))
     b.set_graphs(False)
+    a.stage("withhold_workgroup")
     (_, forms), _ = counted(lambda: a.physics_step_gpu(1)), b.physics_step_gpu(1)
-    assert forms == {"waited": 1} and a.kernel_times()["pcg_grid_gave_up"][1] == 1
-    assert np.array_equal(a.get_simulation_results(), b.get_simulation_results())
-    assert set(counted(lambda: c.physics_step_gpu(1))[1]) == {"one_launch"}
-    a.set_one_launch()
-    assert set(counted(lambda: a.physics_step_gpu(1))[1]) == {"one_launch"}
-    b.physics_step_gpu(1)
+    assert forms == {"waited": 1, "one_launch": a.stats()["newton_iters"] - 1}
+    assert a.kernel_times()["pcg_grid_gave_up"][1] == 1
     assert np.array_equal(a.get_simulation_results(), b.get_simulation_results())
 
 
