@@ -302,8 +302,7 @@ lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on);
  * tests grandchild j, so a step's record is one contiguous load shared by the four lanes), 16 or
  * 32 stack entries in LDS, 512 pairs staged; 7 is the default. 9: two lanes per query on the 128 B
  * records (lane j tests grandchildren 2j and 2j + 1), 16 stack entries in LDS, 512 pairs staged
- * (faster where the queries fill the GPU, as in large batches). Before a tree's
- * first refit the 4-wide shapes run as the binary shape 1 or 3. That is how a standalone tree is
+ * (faster where the queries fill the GPU, as in large batches). That is how a standalone tree is
  * queried; in a solver 7, 8 and 9 all walk its own hierarchies, 16 neighbouring queries per
  * wavefront, whose walks have no stack to overflow. */
 lcsx_status lcsx_solver_set_query_shape(lcsx_solver* s, int shape);
@@ -329,7 +328,10 @@ lcsx_status lcsx_solver_autotune(lcsx_solver* s, char* report, size_t report_len
 
 /* ----------------------------------------------- standalone LBVH (device pointers)
  * LBVH over faces (arity 3) or edges (arity 2), lbvh.h:166-304. All pointers are device
- * pointers on the solver-independent stream `stream` (a hipStream_t, NULL = default). */
+ * pointers on the solver-independent stream `stream` (a hipStream_t, NULL = default). The calls return
+ * before the GPU is done: a tree's construction, refit and queries belong on one stream, or behind an
+ * event or synchronisation of the caller's. A refit before the first construction and a query before the
+ * first refit return LCSX_ERR_STATE. */
 typedef struct lcsx_lbvh lcsx_lbvh;
 lcsx_status lcsx_lbvh_create(int arity, const uint32_t* device_prims, int n_leaves, lcsx_lbvh** out);
 lcsx_status lcsx_lbvh_destroy(lcsx_lbvh* t);

@@ -50,6 +50,7 @@ struct lcsx_lbvh
     Lbvh        t;
     hipStream_t last  = nullptr;
     int         shape = kQueryDefault;
+    bool        constructed = false, refitted = false;  // (what comes before has nothing to read)
 };
 
 namespace
@@ -882,18 +883,20 @@ lcsx_status lcsx_lbvh_construct(lcsx_lbvh* t, const float* x, int n_verts, void*
     if (!t || !x || n_verts <= 0) return arg_error("invalid arguments");
     t->last = (hipStream_t)stream;
     const uint32_t nvs = (uint32_t)n_verts;
-    LCSX_GUARD(t->t.construct(x, &nvs, (hipStream_t)stream); return LCSX_OK;)
+    LCSX_GUARD(t->t.construct(x, &nvs, (hipStream_t)stream); t->constructed = true; return LCSX_OK;)
 }
 lcsx_status lcsx_lbvh_refit(lcsx_lbvh* t, const float* x0, const float* x1, const float* pad, void* stream)
 {
     if (!t || !x0 || !x1 || !pad) return arg_error("invalid arguments");
+    if (!t->constructed) { set_error("refit before construct"); return LCSX_ERR_STATE; }
     t->last = (hipStream_t)stream;
-    LCSX_GUARD(t->t.refit(x0, x1, pad, (hipStream_t)stream); return LCSX_OK;)
+    LCSX_GUARD(t->t.refit(x0, x1, pad, (hipStream_t)stream); t->refitted = true; return LCSX_OK;)
 }
 lcsx_status lcsx_lbvh_query(lcsx_lbvh* t, const float* boxes, int n_queries, int edge_filter, uint32_t* pairs,
                             uint32_t capacity, uint32_t* count, void* stream)
 {
     if (!t || !boxes || n_queries < 0 || !pairs || !count) return arg_error("invalid arguments");
+    if (!t->refitted) { set_error("query before refit"); return LCSX_ERR_STATE; }
     QueryArgs q{};
     q.mode        = QueryBoxes;
     q.n_queries   = (uint32_t)n_queries;

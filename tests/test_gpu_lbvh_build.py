@@ -7,7 +7,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from luisacomputesimulator_amd import _check, hiprt, load_library
+from luisacomputesimulator_amd import LcsxError, _check, hiprt, load_library
 from oracle import morton32
 
 pytestmark = pytest.mark.gpu
@@ -65,5 +65,28 @@ def test_construct_sizes(require_gpu, n):
         _check(lib.lcsx_lbvh_query(h, db.ptr, m, 0, dp.ptr, len(want) + 64, dc.ptr, None))
         got = dp.numpy()[:2 * int(dc.numpy()[0])].reshape(-1, 2)
         assert np.array_equal(got[np.lexsort((got[:, 1], got[:, 0]))], want)
+    finally:
+        lib.lcsx_lbvh_destroy(h)
+
+
+def test_order_of_calls(require_gpu):
+    """A refit before the construction and a query before the refit are refused: they would walk arrays that
+    nothing has written."""
+    lib = load_library()
+    x = hiprt.DeviceArray(np.arange(12, dtype=np.float32))
+    e = hiprt.DeviceArray(np.array([0, 1, 1, 2, 2, 3], dtype=np.uint32))
+    pad, box = hiprt.DeviceArray(np.full(4, 1e-3, np.float32)), hiprt.DeviceArray(np.array([0, 0, 0, 9, 9, 9], np.float32))
+    pairs, count = hiprt.DeviceArray(np.zeros(16, np.uint32)), hiprt.DeviceArray(np.zeros(1, np.uint32))
+    h = C.c_void_p()
+    _check(lib.lcsx_lbvh_create(2, e.ptr, 3, C.byref(h)))
+    try:
+        with pytest.raises(LcsxError, match="refit before construct"):
+            _check(lib.lcsx_lbvh_refit(h, x.ptr, x.ptr, pad.ptr, None))
+        _check(lib.lcsx_lbvh_construct(h, x.ptr, 4, None))
+        with pytest.raises(LcsxError, match="query before refit"):
+            _check(lib.lcsx_lbvh_query(h, box.ptr, 1, 0, pairs.ptr, 8, count.ptr, None))
+        _check(lib.lcsx_lbvh_refit(h, x.ptr, x.ptr, pad.ptr, None))
+        _check(lib.lcsx_lbvh_query(h, box.ptr, 1, 0, pairs.ptr, 8, count.ptr, None))
+        assert int(count.numpy()[0]) == 3
     finally:
         lib.lcsx_lbvh_destroy(h)
