@@ -320,8 +320,8 @@ lcsx_status lcsx_solver_set_spmv_shape(lcsx_solver* s, int shape);
  * per contact or per 256-slot chunk), the PCG SpMV mapping (lcsx_solver_set_spmv_shape) and the
  * broad-phase traversal shape (lcsx_solver_set_query_shape; 7 to 9 are one in a solver); a setting
  * changes only for a candidate more than 3% faster than the current one. The PCG's settings are timed and
- * kept for the solves that run as launches; those that fit one launch still do. No choice changes a result. The state (positions,
- * velocities, statistics, timings) is restored. report (may be NULL) receives
+ * kept for the solves that run as launches; those that fit one launch still do. No choice changes a result.
+ * The state (positions, velocities, statistics, timings) is restored. report (may be NULL) receives
  * "name[setting]=ms;...;chosen:..." (truncated to report_len). Best called after a few frames,
  * on a state with contacts. */
 lcsx_status lcsx_solver_autotune(lcsx_solver* s, char* report, size_t report_len);

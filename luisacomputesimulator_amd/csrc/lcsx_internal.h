@@ -131,7 +131,7 @@ struct Lbvh
     uint32_t n_nodes() const { return n + ni; }
 };
 
-// Exclusive scan of n counts into out[0..n] (out[n] = total; out may be in), three launches.
+// Exclusive scan of n counts into out[0..n] (out[n] = total; out may be in), one launch or three.
 // tmp holds scan_tmp_words(n) words.
 uint32_t scan_tmp_words(uint32_t n);
 void     launch_scan_excl_u32(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp, hipStream_t s);

@@ -519,7 +519,7 @@ struct GridBsr
 };
 
 // The shape of the one-launch form. The widest row is not known here (the row pointers are on the device, and
-// waiting for a count of them would cost every solve 12 us): cloth-like matrices have rows of up to one and
+// a count of them would cost every solve a wait): cloth-like matrices have rows of up to one and
 // a half times the mean. A row with more blocks than the shape holds, or columns that name more rows, make the
 // kernel give up before its first iteration, which costs such a solve 25-40 us (8 iterations of 1,089 rows:
 // 176 us, 150 as launches at once, 65 where the rows fit; of 88,209 rows: 294, 260 and 137).

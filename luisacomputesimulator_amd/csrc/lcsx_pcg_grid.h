@@ -7,8 +7,8 @@
 // vectors and preconditioner once, finds the rows outside its own that its blocks' columns name (a
 // hash table in LDS), and holds p of all of them in LDS, so the product reads registers and LDS only.
 // A scene of a batch is solved by its own workgroups, which wait only for each other; a batch that needs
-// more workgroups than CUs takes several launches. An iteration waits twice: for every 64-row chunk's p.q partial, and for every row block's r.z partial
-// together with the z of the named rows. A partial is posted as one 8-byte word (value, epoch), and so
+// more workgroups than CUs takes several launches. An iteration waits twice: for every 64-row chunk's p.q
+// partial, and for every row block's r.z partial together with the z of the named rows. A partial is posted as one 8-byte word (value, epoch), and so
 // is every entry of z: the word that carries a value also says that it is there, so nothing has to be
 // ordered between the stores. Every workgroup adds the partials up itself.
 //
