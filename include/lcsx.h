@@ -304,7 +304,8 @@ lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on);
  * records (lane j tests grandchildren 2j and 2j + 1), 16 stack entries in LDS, 512 pairs staged
  * (faster where the queries fill the GPU, as in large batches). That is how a standalone tree is
  * queried; in a solver 7, 8 and 9 all walk its own hierarchies, 16 neighbouring queries per
- * wavefront, whose walks have no stack to overflow. */
+ * wavefront, whose walks have no stack to overflow, or as shape 4 where those would be slow: scenes of
+ * thousands of separate pieces, and batches of tiny scenes (lcsx_solver_read "cluster_use": faces, edges). */
 lcsx_status lcsx_solver_set_query_shape(lcsx_solver* s, int shape);
 /* Mapping of the PCG block SpMV (no counterpart in the reference; every shape gives the same
  * bits, the blocks of a row being added in the same order). 0: three blocks per lane and pass with

@@ -215,7 +215,7 @@ _NP = {"f": np.float32, "u": np.uint32, "q": np.uint64, "b": np.uint8, "d": np.f
 # dtype of each readable buffer (see lcsx_solver_read)
 _DTYPES: Dict[str, str] = {n: "u" for n in ("faces", "edges", "hinges", "csr", "stretch_faces", "bending_hinges",
                                             "stretch_springs",
-                                             "fixed_verts", "pairs_vf", "pairs_ee", "contact_idx", "contact_type",
+                                             "fixed_verts", "cluster_use", "pairs_vf", "pairs_ee", "contact_idx", "contact_type",
                                              "ccd_rest_vf", "ccd_rest_ee", "contact_triplets")}
 _DTYPES["is_fixed"] = "b"
 _DTYPES["energy"] = "d"
@@ -411,7 +411,8 @@ class NewtonSolver:
     def set_query_shape(self, shape: int) -> None:
         """Broad-phase traversal shape (0..3 binary steps, 4..6 four-wide steps of the LBVH with
         different LDS stack entries and per-wavefront pair staging; 7..9 the solver's own
-        hierarchies, 16 queries per wavefront; every shape finds the same pairs)."""
+        hierarchies, 16 queries per wavefront, or as 4 in scenes of thousands of pieces and batches of
+        tiny scenes; every shape finds the same pairs)."""
         _check(self.lib.lcsx_solver_set_query_shape(self.h, int(shape)))
 
     def set_spmv_shape(self, shape: int) -> None:

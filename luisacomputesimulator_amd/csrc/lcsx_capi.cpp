@@ -145,7 +145,7 @@ bool is_static_buffer(const std::string& n)
     static const char* k[] = {"rest_x", "faces", "edges", "hinges", "csr", "stretch_faces", "bending_hinges",
                               "fixed_verts", "is_fixed", "face_area", "edge_area", "vert_area", "vert_mass", "offset",
                               "dhat", "sf_Dm", "sf_area", "sf_mu", "sf_lambda", "bh_angle", "bh_hbar", "bh_k",
-                              "stretch_springs", "sp_rest", "sp_k"};
+                              "stretch_springs", "sp_rest", "sp_k", "cluster_use"};
     for (const char* c : k)
         if (n == c) return true;
     return false;
@@ -180,6 +180,11 @@ bool read_named(Solver& S, const std::string& name, Blob& out)
     }
     if (name == "faces") { out.set(S.S.faces); return true; }
     if (name == "edges") { out.set(S.S.edges); return true; }
+    if (name == "cluster_use")
+    {
+        out.set(std::vector<uint32_t>{S.S.cluster_f_use, S.S.cluster_e_use});
+        return true;
+    }
     if (name == "hinges") { out.set(S.S.hinges); return true; }
     if (name == "csr") { out.set(S.S.csr); return true; }
     if (name == "stretch_faces") { out.set(S.S.sf); return true; }

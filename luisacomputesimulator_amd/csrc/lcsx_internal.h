@@ -180,6 +180,7 @@ struct QueryArgs
 };
 constexpr int kQueryVariants = 10;
 constexpr int kQueryDefault  = 7;
+constexpr int kQueryElements = 4;  // of vertices and edges against an LBVH, where a shape of boxes only is asked for
 void lbvh_query(const Lbvh& t, const QueryArgs& a, hipStream_t s);
 
 // The hierarchy that the solver's broad phases walk in the shapes that share a query among lanes: over
@@ -210,6 +211,6 @@ struct ClusterTree
     void refit(const float* x0, const float* x1, const float* pad, const uint32_t* leaf_of, hipStream_t s);
     void query(const ClusterQuery& a, const uint32_t* leaf_of, hipStream_t s) const;
 };
-bool query_by_clusters(int variant);  // whether a traversal shape is one of those
+bool query_by_clusters(int variant);  // whether a traversal shape is one of those (Setup::cluster_*_use permitting)
 
 }  // namespace lcsx

@@ -2003,6 +2003,9 @@ void lbvh_query(const Lbvh& t, const QueryArgs& a, hipStream_t s)
 {
     if (t.n == 0 || a.n_queries == 0) return;
     int v = a.variant >= 0 && a.variant < kQueryVariants ? a.variant : kQueryDefault;
+    // the shapes that share a query among lanes read their boxes; vertices and edges take one lane each, with as
+    // many stack entries
+    if (kQueryShapes[v].lanes >= 2 && a.mode != QueryBoxes) v = kQueryElements;
     // 4-wide records exist after a level-ordered refit; otherwise the binary shape with the same
     // LDS stack and staging
     if (kQueryShapes[v].wide >= 4 && !t.wide_ready) v = kQueryShapes[v].lds_stack >= 16 ? 1 : 3;

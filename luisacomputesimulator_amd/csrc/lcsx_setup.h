@@ -85,6 +85,7 @@ struct Setup
     // is padded with kInvalid, to whole wavefronts of 64 points and whole blocks of kClusterLeaves elements;
     // _block: the first block of each scene, and the end.
     std::vector<uint32_t> cluster_v, cluster_f, cluster_e, cluster_f_block, cluster_e_block;
+    bool cluster_f_use = true, cluster_e_use = true;  // whether the queries walk the blocks (cluster)
 
     void build(const std::vector<MeshDesc>& meshes);
 

@@ -334,8 +334,8 @@ void Solver::upload_state_constants()
     row_kind_d.upload(S.row_kind, s);
     cluster_vert.upload(S.cluster_v, s);
     n_cluster_vert = (uint32_t)S.cluster_v.size();
-    cluster_face.init(3, faces.p, S.cluster_f, S.cluster_f_block, s);
-    cluster_edge.init(2, edges.p, S.cluster_e, S.cluster_e_block, s);
+    if (S.cluster_f_use) cluster_face.init(3, faces.p, S.cluster_f, S.cluster_f_block, s);
+    if (S.cluster_e_use) cluster_edge.init(2, edges.p, S.cluster_e, S.cluster_e_block, s);
     vert_body_d.upload(S.vert_body, s);
     body_X_d.upload(S.body_X, s);
     static_assert(sizeof(BodyDev) == sizeof(Setup::Body), "body record layout");
@@ -547,8 +547,9 @@ void Solver::query_faces(bool ccd)
     if (S.nf == 0) return;
     const float* x0 = ccd ? x_iter.p : x.p;
     Status*      st = status.p;
-    tree_face.refit(x0, x.p, offset.p, stream, !query_by_clusters(query_variant));
-    if (query_by_clusters(query_variant))
+    const bool clusters = S.cluster_f_use && query_by_clusters(query_variant);
+    tree_face.refit(x0, x.p, offset.p, stream, !clusters);
+    if (clusters)
     {
         ClusterQuery c = cluster_query(x0);
         c.order        = cluster_vert.p;
@@ -583,8 +584,9 @@ void Solver::query_edges(bool ccd)
     if (S.ne == 0) return;
     const float* x0 = ccd ? x_iter.p : x.p;
     Status*      st = status.p;
-    tree_edge.refit(x0, x.p, offset.p, stream, !query_by_clusters(query_variant));
-    if (query_by_clusters(query_variant))
+    const bool clusters = S.cluster_e_use && query_by_clusters(query_variant);
+    tree_edge.refit(x0, x.p, offset.p, stream, !clusters);
+    if (clusters)
     {
         ClusterQuery    c       = cluster_query(x0);
         const uint32_t* leaf_of = sorted_ee ? tree_edge.leaf_of.p : nullptr;

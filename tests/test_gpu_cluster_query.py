@@ -23,6 +23,19 @@ def boxes():
     return sc
 
 
+def patches(count, n=3):
+    """One mesh of `count` separate n x n patches, scattered, in an order that has nothing to do with where they are."""
+    sc = scenes.square_cloth(n, height=0.0)
+    v, t = sc.meshes[0].verts * np.float32(0.02), sc.meshes[0].tris
+    k = int(np.ceil(count ** (1 / 3)))
+    at = np.stack(np.meshgrid(*[np.arange(k)] * 3, indexing="ij"), -1).reshape(-1, 3)[:count] * 0.0215 + [0.0, 0.3, 0.0]
+    np.random.default_rng(11).shuffle(at)
+    sc.meshes[0].verts = (v[None] + at[:, None]).reshape(-1, 3).astype(np.float32)
+    sc.meshes[0].tris = (t[None] + (np.arange(count) * n * n)[:, None, None]).reshape(-1, 3).astype(np.int32)
+    sc.meshes[0].fixed = [scenes.FixedPoints("LeftBack", 0.001)]
+    return sc
+
+
 # edges per scene: 5 (one record and a part), 1008 and 1121 (around a block of 1024 positions), 70,000 (more
 # than 64 blocks: the list of blocks takes two steps), long edges beside short ones, several scenes
 CASES = {
@@ -36,7 +49,12 @@ CASES = {
     "boxes": lambda: [boxes()],
     "batch": lambda: [scenes.square_cloth(2), scenes.square_cloth(33),
                       scenes.cloth_on_sphere(17, 0.05, -0.03, seed=1, sphere_subdiv=2, height=0.3015)],
+    # where the hierarchies would be slow the LBVH is walked: for the edges of 4,200 pieces (66 blocks of more than
+    # one; the faces' 33 are walked), and for a batch of 80 tiny scenes
+    "pieces": lambda: [patches(4200)],
+    "tiny_batch": lambda: [scenes.square_cloth(3, seed=k) for k in range(80)],
 }
+USE = {"pieces": [1, 0], "tiny_batch": [0, 0]}
 
 
 def pairs(s, key):
@@ -48,6 +66,7 @@ def pairs(s, key):
 def test_clusters_find_the_pairs_of_the_lbvh(require_gpu, name):
     scs = CASES[name]()
     s = NewtonSolver.from_scenes(scs) if len(scs) > 1 else NewtonSolver.from_scene(scs[0])
+    assert s.read("cluster_use").tolist() == USE.get(name, [1, 1])
     for frame in range(2):
         for stage in ("frame_begin", "predict", "iter_begin"):
             s.stage(stage)
