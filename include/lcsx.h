@@ -288,7 +288,8 @@ lcsx_status lcsx_solver_set_timing(lcsx_solver* s, int level);
 lcsx_status lcsx_solver_set_graphs(lcsx_solver* s, int on);
 /* The PCG in one launch (no counterpart in the reference). on 1, the default: a solve runs as a single
  * launch where the system fits (a scene of up to 131,072 rows of at most 12 blocks or 65,536 of at most 32,
- * a batch in up to two such launches, and contacts that are few beside the rows), whatever
+ * a batch in up to two such launches, and contacts that are few beside the rows; rows of more than 16
+ * blocks with contacts only in small scenes), whatever
  * lcsx_solver_set_graphs and lcsx_solver_set_spmv_shape say of the solves that do not; this takes back
  * their choice of the launches. 0: launches only. */
 lcsx_status lcsx_solver_set_one_launch(lcsx_solver* s, int on);

@@ -263,6 +263,7 @@ void Solver::plan_grid()
     uint32_t width = 0, most = 0;
     for (size_t k = 0; k + 1 < S.sl_off.size(); k++) width = std::max(width, S.sl_off[k + 1] - S.sl_off[k]);
     for (uint32_t sc = 0; sc < S.nscenes; sc++) most = std::max(most, S.sc_rb0[sc + 1] - S.sc_rb0[sc]);
+    grid_most = most;
     const uint32_t limit = grid_wgs(device);
     grid_shape = grid_plan(most, S.n_rb, width, limit);
     grid_round.clear();
@@ -704,13 +705,19 @@ int Solver::pcg_run(PcgArgs& a, const SellView& A, const ContactView& cv, const 
     // row blocks per workgroup spill with contacts (94,000 rows, 100 iterations: 1.09 against 1.94 ms
     // without contacts, 1.95 against 2.05 with 215, 2.19 against 2.09 with 1,172, 2.87 against 2.22 with
     // 18,000): a chunk per scene and one for 16 workgroups, or 8 in a batch, whose scenes wait for their own
-    // chunks only (202,000 rows with a chunk for 11 workgroups: 2.48 against 2.99).
+    // chunks only (202,000 rows with a chunk for 11 workgroups: 2.48 against 2.99). Rows of 17 to 32 blocks
+    // (irregular triangulations) spill most with contacts, and what is spilled is read back every iteration:
+    // only up to 20 row blocks in the largest scene, or 64 of 16-bit blocks (one launch against the launches,
+    // us a solve of about 100 iterations in first contact: FP32 4,867 rows 239 and 224 to 267 from run to run,
+    // 10,051 292 and 283, 63,142 595 and 385; FP16 13,186 rows 319 and 336, 40,642 384 and 356; FP32 8 scenes
+    // of 4,867 322 and 349).
     GridPlan  gp;
     GridLease lease;
     const uint32_t gw = grid_round.empty() ? 0u : grid_round.back();
     const uint32_t grid_chunks = 2u * gw * (kGridThreads / 256u);  // that the words are for
     const uint32_t most_chunks = grid_shape.U == 2 ? grid_chunks : std::min(grid_chunks, ns + gw / (ns == 1u ? 16u : 8u));
-    if (one_launch && pcg_grid && grid_shape.U && spmv_sample == 0 && mc <= most_chunks &&
+    const bool     wide = grid_shape.K == 8 && mc && grid_most > (A.val_p ? 64u : 20u);
+    if (one_launch && pcg_grid && grid_shape.U && spmv_sample == 0 && mc <= most_chunks && !wide &&
         lease.take(device))
         gp = grid_shape;
     const size_t grid_words = 5 * (size_t)S.n_rb + grid_chunks;

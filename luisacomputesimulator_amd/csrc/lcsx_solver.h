@@ -194,6 +194,7 @@ struct Solver
     bool                     pcg_grid = true;
     bool                     grid_withhold = false;  // exercises a wait that runs out: a workgroup is not launched
     GridPlan                 grid_shape;      // U 0: the rows or scenes do not fit
+    uint32_t                 grid_most = 0;   // row blocks of the largest scene
     std::vector<uint32_t>    grid_round;      // workgroups of round r: [grid_round[r], grid_round[r + 1])
     DBuf<uint2>              grid_tab;        // per workgroup: scene, place in it (several scenes)
     DBuf<unsigned long long> grid_slots, grid_zx;

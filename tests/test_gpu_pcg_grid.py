@@ -32,6 +32,23 @@ def tube_on_ring():
     return sc
 
 
+def irregular(n):
+    """A cloth of randomly moved grid points and their Delaunay triangles on a sphere: rows of up to 20 blocks."""
+    from scipy.spatial import Delaunay
+
+    sc = scenes.cloth_on_sphere(n, 0.02, -0.01, seed=4, sphere_subdiv=3, height=0.3015)
+    m, rng = sc.meshes[0], np.random.default_rng(0)
+    g = np.stack(np.meshgrid(np.arange(n), np.arange(n), indexing="ij"), -1).reshape(-1, 2).astype(float)
+    inner = ((g > 0) & (g < n - 1)).all(1)
+    g[inner] += rng.uniform(-0.48, 0.48, size=(int(inner.sum()), 2))
+    v, t = m.verts.copy(), Delaunay(g).simplices.astype(np.int32)
+    v[:, 0], v[:, 2] = g[:, 1] / (n - 1) - 0.5, g[:, 0] / (n - 1) - 0.5
+    a, b = g[t[:, 1]] - g[t[:, 0]], g[t[:, 2]] - g[t[:, 0]]
+    area = np.abs(a[:, 0] * b[:, 1] - a[:, 1] * b[:, 0])
+    m.verts, m.tris = v.astype(np.float32), t[area > 1e-6]
+    return sc
+
+
 # rows: less than one 64-row chunk, one row past it, several workgroups, many, and above 65,536 rows (two row
 # blocks per workgroup) without and with contacts
 CASES = {
@@ -83,6 +100,33 @@ def test_one_launch_equals_launches(require_gpu, name, precision):
 def batch(sizes):
     return [scenes.square_cloth(n, seed=k) if k % 2 else
             scenes.cloth_on_sphere(n, 0.02, -0.01, seed=k, sphere_subdiv=2, height=0.3015) for k, n in enumerate(sizes)]
+
+
+# rows of 17 to 32 blocks: in contact up to 20 row blocks, or 64 of 16-bit blocks
+@pytest.mark.parametrize("n,precision,one", [(33, "fp32", True), (33, "mixed", True), (112, "fp32", False),
+                                             (112, "mixed_bf16", True)])
+def test_rows_of_an_irregular_mesh(require_gpu, n, precision, one):
+    def solver(collide=True):
+        sc = irregular(n)
+        sc.params.precision, sc.params.use_self_collision = precision, collide
+        return NewtonSolver.from_scene(sc)
+
+    a, b, c = solver(), solver(), solver(False)
+    csr = a.read("csr").astype(np.int64)
+    width = int(np.diff(csr[:a.num_verts + 1]).max())
+    assert 16 < width <= 32
+    b.set_graphs(False)
+    forms = {}
+    for f in range(2):
+        _, form = counted(lambda: a.physics_step_gpu(1))
+        b.physics_step_gpu(1)
+        forms = {k: forms.get(k, 0) + v for k, v in form.items()}
+        assert a.stats()["pcg_iters_total"] == b.stats()["pcg_iters_total"]
+        assert np.array_equal(a.get_simulation_results(), b.get_simulation_results())
+    print(f"[gpu-grid] irregular {n} {precision}: rows of {width}, {a.stats()['num_contacts']} contacts, {forms}", flush=True)
+    assert a.stats()["num_contacts"] > 0
+    assert set(forms) == ({"one_launch"} if one else set())
+    assert set(counted(lambda: c.physics_step_gpu(1))[1]) == {"one_launch"}  # without contacts, whatever the size
 
 
 def test_forms_of_the_launches_and_back(require_gpu):
