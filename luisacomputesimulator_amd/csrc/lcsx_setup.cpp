@@ -208,19 +208,6 @@ void Setup::cluster()
     };
     // the elements of all meshes, each mesh's along its curve, every scene padded to whole units (the meshes
     // are numbered scene by scene); arity 0: points
-    // Pieces: what edges hold together. A block of a piece's elements stays small in space however the pieces
-    // move; one over many pieces may reach over the whole scene, and so may all such blocks.
-    std::vector<uint32_t> piece(nv);
-    for (uint32_t i = 0; i < nv; i++) piece[i] = i;
-    auto root = [&](uint32_t i) {
-        while (piece[i] != i) i = piece[i] = piece[piece[i]];
-        return i;
-    };
-    for (uint32_t e = 0; e < ne; e++)
-    {
-        const uint32_t a = root(edges[2 * e]), b = root(edges[2 * e + 1]);
-        piece[std::max(a, b)] = std::min(a, b);
-    }
     std::vector<uint32_t> code, id, first, tmp;
     auto ordered = [&](uint32_t n, uint32_t arity, const std::vector<uint32_t>& prims, uint32_t unit,
                        std::vector<uint32_t>& out, std::vector<uint32_t>* block) {
@@ -259,6 +246,23 @@ void Setup::cluster()
     ordered(nv, 0, faces, 64, cluster_v, nullptr);
     ordered(nf, 3, faces, kClusterLeaves, cluster_f, &cluster_f_block);
     ordered(ne, 2, edges, kClusterLeaves, cluster_e, &cluster_e_block);
+    // Pieces: what edges hold together (made when first asked for). A block of a piece's elements stays small in
+    // space however the pieces move; one over many pieces may reach over the whole scene, and so may all such
+    // blocks.
+    std::vector<uint32_t> piece;
+    auto root = [&](uint32_t i) {
+        while (piece[i] != i) i = piece[i] = piece[piece[i]];
+        return i;
+    };
+    auto join = [&]() {
+        piece.resize(nv);
+        for (uint32_t i = 0; i < nv; i++) piece[i] = i;
+        for (uint32_t e = 0; e < ne; e++)
+        {
+            const uint32_t a = root(edges[2 * e]), b = root(edges[2 * e + 1]);
+            piece[std::max(a, b)] = std::min(a, b);
+        }
+    };
     // The blocks are walked unless a scene has more than kMost of them over several pieces (every query meets
     // nearly all of those: the line is one step of the walk over the blocks), or there are more than kMost in all
     // and less than a quarter of their positions are taken (batches of tiny scenes; a block costs the same
@@ -272,6 +276,8 @@ void Setup::cluster()
         uint32_t           most  = 0;
         for (uint32_t sc = 0; sc < nscenes; sc++)
         {
+            if (block[sc + 1] - block[sc] <= kMost) continue;
+            if (piece.empty()) join();
             uint32_t mixed = 0;
             for (uint32_t b = block[sc]; b < block[sc + 1]; b++)
             {
